@@ -82,6 +82,110 @@ hipError_t scratch_address(int device, void **ptr) {
 }
 }  // namespace
 
+// ---- work vectors kept between calls ------------------------------------------
+// A solve, an inner solve or a residual check takes its work vectors (one
+// allocation a vector: 54 for an order-8 inner solve of 6 columns) from this
+// per-device list and returns them to it with its stream idle.  Allocating and
+// freeing them on each call cost far more than the work, since the driver clears
+// what it hands out: with the list an order-8 inner solve of 6 columns at NN = 13
+// (4 GB of vectors) takes 20.7 ms instead of 120, one of order 4 on 4 columns at
+// NN = 21 (27 GB) 108 ms instead of 316 to 1350, two eigensolver iterations of
+// 10 columns at NN = 11 149 ms instead of 206.
+// Any thread and context may take a listed block: nothing is queued on it.  At
+// most an eighth of the device's memory stays listed (the blocks idle longest go
+// first), all of it is freed when the last context on the device is destroyed,
+// and when an allocation of this library fails the list is freed and the
+// allocation tried again.
+namespace {
+struct IdleBlocks {
+  std::mutex mu;
+  std::vector<std::pair<void *, size_t>> idle;  // oldest first
+  size_t bytes = 0, cap = 0;
+  int contexts = 0;
+};
+IdleBlocks g_idle[kMaxDevices];
+
+void free_blocks(const std::vector<std::pair<void *, size_t>> &blocks) {
+  for (const auto &b : blocks) (void)hipFree(b.first);
+}
+
+void drop_idle(int device) {
+  std::vector<std::pair<void *, size_t>> out;
+  {
+    IdleBlocks &l = g_idle[device];
+    std::lock_guard<std::mutex> lk(l.mu);
+    out.swap(l.idle);
+    l.bytes = 0;
+  }
+  free_blocks(out);
+}
+
+// hipMalloc on the current device `device`, once more without the idle blocks
+// where it fails.
+hipError_t device_malloc(int device, void **ptr, size_t bytes) {
+  hipError_t e = hipMalloc(ptr, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  drop_idle(device);
+  return hipMalloc(ptr, bytes);
+}
+
+// A block of exactly `bytes` (contents undefined): listed, else allocated.
+hipError_t block_take(int device, void **ptr, size_t bytes) {
+  {
+    IdleBlocks &l = g_idle[device];
+    std::lock_guard<std::mutex> lk(l.mu);
+    for (size_t i = l.idle.size(); i-- > 0;)
+      if (l.idle[i].second == bytes) {
+        *ptr = l.idle[i].first;
+        l.idle.erase(l.idle.begin() + std::ptrdiff_t(i));
+        l.bytes -= bytes;
+        return hipSuccess;
+      }
+  }
+  return device_malloc(device, ptr, bytes);
+}
+
+// Returns a block of block_take; no queued work may use it any more.
+void block_give(int device, void *ptr, size_t bytes) {
+  std::vector<std::pair<void *, size_t>> out;
+  {
+    IdleBlocks &l = g_idle[device];
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.idle.emplace_back(ptr, bytes);
+    l.bytes += bytes;
+    size_t n = 0;
+    while (l.bytes > l.cap) l.bytes -= l.idle[n++].second;
+    out.assign(l.idle.begin(), l.idle.begin() + std::ptrdiff_t(n));
+    l.idle.erase(l.idle.begin(), l.idle.begin() + std::ptrdiff_t(n));
+  }
+  free_blocks(out);
+}
+
+// The blocks one call holds: returned when it ends, after its stream has drained.
+struct Blocks {
+  int device;
+  hipStream_t stream;
+  std::vector<std::pair<void *, size_t>> held;
+  Blocks(int device_, hipStream_t stream_) : device(device_), stream(stream_) {}
+  Blocks(const Blocks &) = delete;
+  Blocks &operator=(const Blocks &) = delete;
+  hipError_t take(void **ptr, size_t bytes) {
+    const hipError_t e = block_take(device, ptr, bytes);
+    if (e == hipSuccess) held.emplace_back(*ptr, bytes);
+    return e;
+  }
+  ~Blocks() {
+    if (held.empty()) return;
+    if (hipStreamSynchronize(stream) != hipSuccess) {
+      free_blocks(held);
+      return;
+    }
+    for (const auto &b : held) block_give(device, b.first, b.second);
+  }
+};
+}  // namespace
+
 struct dex_ctx {
   dex_params p{};
   int nn = 0;
@@ -218,7 +322,7 @@ hipError_t stage_upload(dex_ctx *c, void *dev, const void *src, size_t bytes) {
 
 int ensure_u(dex_ctx *c) {
   if (c->d_u) return 0;
-  DEX_HIP(hipMalloc(&c->d_u, size_t(c->d) * sizeof(Dbl2)));
+  DEX_HIP(device_malloc(c->p.device, &c->d_u, size_t(c->d) * sizeof(Dbl2)));
   return 0;
 }
 
@@ -232,7 +336,7 @@ int64_t batch_cols(const dex_ctx *c) {
 
 int ensure_ub(dex_ctx *c) {
   if (c->d_ub || batch_cols(c) < 2) return 0;
-  DEX_HIP(hipMalloc(&c->d_ub, size_t(batch_cols(c)) * size_t(c->d) * sizeof(Dbl2)));
+  DEX_HIP(device_malloc(c->p.device, &c->d_ub, size_t(batch_cols(c)) * size_t(c->d) * sizeof(Dbl2)));
   return 0;
 }
 
@@ -675,22 +779,38 @@ int dex_ctx_create(const dex_params *p, dex_ctx **out) {
   // two-pass kernels exist (used to cross-check the two implementations).
   if (const char *mv = std::getenv("DEX_MATVEC"))
     if (std::strcmp(mv, "generic") == 0) c->fast64 = false;
+  // (the device ordinal was accepted by hipSetDevice; the scratch address below bounds it)
+  if (p->device < 0 || p->device >= kMaxDevices) {
+    delete c;
+    return hip_fail(hipErrorInvalidDevice, "dex_ctx_create");
+  }
+  {
+    size_t free_now = 0, total = 0;
+    if (hipMemGetInfo(&free_now, &total) != hipSuccess) total = 0;
+    IdleBlocks &l = g_idle[p->device];
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.cap = total / 8;
+    ++l.contexts;
+  }
   // A blocking stream: work on it is ordered after work already queued on the
   // default stream (where callers such as torch place their kernels) and vice versa.
+  auto dmalloc = [c](auto **ptr, size_t bytes) {
+    return device_malloc(c->p.device, reinterpret_cast<void **>(ptr), bytes);
+  };
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamDefault);
-  if (e == hipSuccess) e = hipMalloc(&c->d_tinv, c->tinv_host.size() * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&c->d_vn, c->vn_host.size() * sizeof(double));
+  if (e == hipSuccess) e = dmalloc(&c->d_tinv, c->tinv_host.size() * sizeof(double));
+  if (e == hipSuccess) e = dmalloc(&c->d_vn, c->vn_host.size() * sizeof(double));
   if (e == hipSuccess)
     e = hipMemcpy(c->d_tinv, c->tinv_host.data(), c->tinv_host.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(c->d_vn, c->vn_host.data(), c->vn_host.size() * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&c->d_desc, kMaxDesc * sizeof(ColDesc));
-  if (e == hipSuccess) e = hipMalloc(&c->d_args, kMaxDesc * sizeof(ColDesc) + 2 * kMaxSmall * sizeof(Dbl2) + 512);
-  if (e == hipSuccess) e = hipMalloc(&c->d_gram_out, 192 * 192 * sizeof(Dbl2));
+  if (e == hipSuccess) e = dmalloc(&c->d_desc, kMaxDesc * sizeof(ColDesc));
+  if (e == hipSuccess) e = dmalloc(&c->d_args, kMaxDesc * sizeof(ColDesc) + 2 * kMaxSmall * sizeof(Dbl2) + 512);
+  if (e == hipSuccess) e = dmalloc(&c->d_gram_out, 192 * 192 * sizeof(Dbl2));
   c->partial_bytes = std::max(dex::gram_partial_elems(64, 128) * sizeof(Dbl2),
                               dex::coldots_partial_elems(64) * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&c->d_partial, c->partial_bytes);
-  if (e == hipSuccess) e = hipMalloc(&c->d_dots, 64 * 4 * sizeof(double));
+  if (e == hipSuccess) e = dmalloc(&c->d_partial, c->partial_bytes);
+  if (e == hipSuccess) e = dmalloc(&c->d_dots, 64 * 4 * sizeof(double));
   for (int i = 0; i < 3 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
   if (e == hipSuccess) {
     c->stage_cap = size_t(4) << 20;
@@ -723,6 +843,13 @@ int dex_ctx_destroy(dex_ctx *c) {
   for (hipEvent_t ev : c->free_events) (void)hipEventDestroy(ev);
   if (c->h_stage) (void)hipHostFree(c->h_stage);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  bool last = false;
+  {
+    IdleBlocks &l = g_idle[c->p.device];
+    std::lock_guard<std::mutex> lk(l.mu);
+    last = --l.contexts == 0;
+  }
+  if (last) drop_idle(c->p.device);
   delete c;
   return DEX_OK;
 }
@@ -973,14 +1100,12 @@ int dex_matvec(dex_ctx *c, const double *in, double *out, int32_t howmany, int64
   if (!c || !in || !out) return fail(DEX_EINVAL, "null argument");
   if (checksize != c->d) return fail(DEX_ESIZE, "SIZE ERROR: checksize != M*MBLK");
   DEX_HIP(hipSetDevice(c->p.device));
-  Dbl2 *dx = nullptr, *dy = nullptr;
+  void *dx = nullptr, *dy = nullptr;
   const size_t bytes = size_t(c->d) * sizeof(Dbl2);
-  DEX_HIP(hipMalloc(&dx, bytes));
-  hipError_t e = hipMalloc(&dy, bytes);
-  if (e != hipSuccess) {
-    (void)hipFree(dx);
-    return hip_fail(e, "hipMalloc");
-  }
+  Blocks blocks(c->p.device, c->stream);
+  DEX_HIP(blocks.take(&dx, bytes));
+  DEX_HIP(blocks.take(&dy, bytes));
+  hipError_t e = hipSuccess;
   int st = DEX_OK;
   for (int j = 0; j < howmany && st == DEX_OK; ++j) {
     e = hipMemcpyAsync(dx, in + size_t(j) * c->d * 2, bytes, hipMemcpyHostToDevice, c->stream);
@@ -994,8 +1119,6 @@ int dex_matvec(dex_ctx *c, const double *in, double *out, int32_t howmany, int64
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) st = hip_fail(e, "copy out");
   }
-  (void)hipFree(dx);
-  (void)hipFree(dy);
   return st;
 }
 
@@ -1020,21 +1143,16 @@ int dex_dots(dex_ctx *c, const double *bras, const double *kets, int64_t size, i
   if (size != c->d) return fail(DEX_ESIZE, "SIZE ERROR: size != M*MBLK");
   DEX_HIP(hipSetDevice(c->p.device));
   void *db = nullptr, *dk = nullptr;
-  DEX_HIP(hipMalloc(&db, size_t(nn) * size * 16));
-  hipError_t e = hipMalloc(&dk, size_t(mm) * size * 16);
-  if (e != hipSuccess) {
-    (void)hipFree(db);
-    return hip_fail(e, "hipMalloc");
-  }
+  Blocks blocks(c->p.device, c->stream);
+  DEX_HIP(blocks.take(&db, size_t(nn) * size * 16));
+  DEX_HIP(blocks.take(&dk, size_t(mm) * size * 16));
   int st = DEX_OK;
-  e = hipMemcpy(db, bras, size_t(nn) * size * 16, hipMemcpyHostToDevice);
+  hipError_t e = hipMemcpy(db, bras, size_t(nn) * size * 16, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dk, kets, size_t(mm) * size * 16, hipMemcpyHostToDevice);
   if (e != hipSuccess)
     st = hip_fail(e, "copy in");
   else
     st = dex_dots_device(c, db, dk, size, nn, mm, out);
-  (void)hipFree(db);
-  (void)hipFree(dk);
   return st;
 }
 
@@ -1563,7 +1681,8 @@ struct Solver {
     return 0;
   }
 
-  std::vector<Dbl2 *> *store = nullptr;  // every buffer ever handed out (freed by the caller)
+  Blocks *blocks = nullptr;              // where new work vectors come from (the caller's)
+  std::vector<Dbl2 *> *store = nullptr;  // every vector taken from it
 
   // A free work vector of format fmt (0 complex128, 1 complex64, tagged): from
   // its pool, else a fresh allocation.  nullptr on OOM.
@@ -1574,8 +1693,9 @@ struct Solver {
       pl.pop_back();
       return p;
     }
-    Dbl2 *p = nullptr;
-    if (hipMalloc(&p, size_t(c->d) * (fmt ? 8 : 16)) != hipSuccess) return nullptr;
+    void *v = nullptr;
+    if (blocks->take(&v, size_t(c->d) * (fmt ? 8 : 16)) != hipSuccess) return nullptr;
+    Dbl2 *p = static_cast<Dbl2 *>(v);
     if (fmt) p = tag32(p);
     store->push_back(p);
     return p;
@@ -1603,7 +1723,7 @@ struct Solver {
 // combination); X and AX stay complex128 and AX = H X is applied in FP64.
 int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out, cd sigma, int ns,
               int maxit, double tol, int inner, int outmodulus, const dex_solve_opts &o, dex_result *res,
-              bool lowp, std::vector<Dbl2 *> &store) {
+              bool lowp, Blocks &blocks, std::vector<Dbl2 *> &store) {
   const int nev = int(xcols.size());
   Solver S{c, nev, ns, o.strict_cholesky != 0, o.symmetry};
   S.inner32 = o.inner_fp32 != 0 || lowp;
@@ -1613,6 +1733,7 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
   W.fmt = AW.fmt = P.fmt = AP.fmt = lf;
   X.cols = xcols;
   for (Dbl2 *p : store) S.give(p);
+  S.blocks = &blocks;
   S.store = &store;
   if (int st = S.grow(AX, nev)) return st;
   if (int st = S.grow(W, nev)) return st;
@@ -2034,18 +2155,13 @@ extern "C" int dex_gplmr_eig_device(dex_ctx *c, void *x_dev, double *e, int32_t 
   // (5 + 2 NS) (NEV + guard) search-block vectors, complex64 in the mixed form
   const int nwork = (5 + 2 * ns) * nblk + nblk;
   std::vector<Dbl2 *> store, guards;
-  auto free_all = [&]() {
-    for (Dbl2 *q : store) (void)hipFree(untag(q));
-    for (Dbl2 *q : guards) (void)hipFree(q);
-  };
+  Blocks blocks(c->p.device, c->stream);
   for (int j = 0; j < nwork + guard; ++j) {
     const bool lo = mixed && j >= nblk && j < nwork;
-    Dbl2 *p = nullptr;
-    hipError_t err = hipMalloc(&p, size_t(c->d) * (lo ? 8 : 16));
-    if (err != hipSuccess) {
-      free_all();
+    void *v = nullptr;
+    if (blocks.take(&v, size_t(c->d) * (lo ? 8 : 16)) != hipSuccess)
       return fail(DEX_EOOM, "device allocation for GPLMR work vectors failed");
-    }
+    Dbl2 *p = static_cast<Dbl2 *>(v);
     if (j < nwork)
       store.push_back(lo ? tag32(p) : p);
     else
@@ -2067,12 +2183,13 @@ extern "C" int dex_gplmr_eig_device(dex_ctx *c, void *x_dev, double *e, int32_t 
   // around the complex128 X and AX, whose FP64 refreshes gplmr_run does; a run
   // that ends at MAXIT unconverged may be followed by up to fp64_restarts
   // restarts from its X (each with a fresh FP64 AX and no P block).
-  st = gplmr_run(c, xcols, nev, ev.data(), sigma, ns, maxit, tol, inner_iter, outmodulus, o, res, mixed, store);
+  st = gplmr_run(c, xcols, nev, ev.data(), sigma, ns, maxit, tol, inner_iter, outmodulus, o, res, mixed, blocks,
+                 store);
   if (mixed && st == DEX_ENOTCONVERGED) {
     for (int r = 0; r < o.fp64_restarts && c->stop.load(std::memory_order_relaxed) == 0; ++r) {
       dex_result sub{};
       st = gplmr_run(c, xcols, nev, ev.data(), sigma, ns, maxit, tol, inner_iter, outmodulus, o,
-                     res ? &sub : nullptr, true, store);
+                     res ? &sub : nullptr, true, blocks, store);
       if (res) {
         res->matvecs += sub.matvecs;
         res->iterations += sub.iterations;
@@ -2090,7 +2207,6 @@ extern "C" int dex_gplmr_eig_device(dex_ctx *c, void *x_dev, double *e, int32_t 
       if (st != DEX_ENOTCONVERGED) break;
     }
   }
-  free_all();
   for (int j = 0; j < nev; ++j) {
     e[2 * j] = ev[j].real();
     e[2 * j + 1] = ev[j].imag();
@@ -2110,7 +2226,9 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
   if (x_dev == px_dev) return fail(DEX_EINVAL, "X and PX must not alias");
   DEX_HIP(hipSetDevice(c->p.device));
   Solver S{c, nev, 1, false, false, symmetry};
+  Blocks blocks(c->p.device, c->stream);
   std::vector<Dbl2 *> store;
+  S.blocks = &blocks;
   S.store = &store;
   Block in, out;
   for (int j = 0; j < nev; ++j) {
@@ -2128,7 +2246,6 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
     if (!st) st = S.inner_solve(out, inner_iter, cd(sigma_re, sigma_im));
   }
   if (hipStreamSynchronize(c->stream) != hipSuccess && !st) st = fail(DEX_EHIP, "stream synchronise failed");
-  for (Dbl2 *p : store) (void)hipFree(p);
   return st;
 }
 
@@ -2173,15 +2290,11 @@ extern "C" int dex_diagsubspace_device(dex_ctx *c, const double *orbitals, int32
   }
   // device buffers: X, conj-or-plain X for the Y X products, T, W, one vector
   Dbl2 *dx = nullptr, *dt = nullptr, *dw = nullptr, *dpsi = nullptr, *dy = nullptr;
-  auto cleanup = [&]() {
-    for (void *ptr : {(void *)dx, (void *)dt, (void *)dw, (void *)dpsi, (void *)dy})
-      if (ptr) (void)hipFree(ptr);
-  };
+  Blocks blocks(c->p.device, c->stream);
+  auto take = [&](Dbl2 **ptr, size_t bytes) { return blocks.take(reinterpret_cast<void **>(ptr), bytes); };
   const size_t mk = size_t(m) * k * sizeof(Dbl2);
-  if (hipMalloc(&dx, mk) != hipSuccess || hipMalloc(&dt, mk) != hipSuccess || hipMalloc(&dw, mk) != hipSuccess ||
-      hipMalloc(&dpsi, size_t(c->d) * sizeof(Dbl2)) != hipSuccess ||
-      hipMalloc(&dy, size_t(c->d) * sizeof(Dbl2)) != hipSuccess) {
-    cleanup();
+  if (take(&dx, mk) != hipSuccess || take(&dt, mk) != hipSuccess || take(&dw, mk) != hipSuccess ||
+      take(&dpsi, size_t(c->d) * sizeof(Dbl2)) != hipSuccess || take(&dy, size_t(c->d) * sizeof(Dbl2)) != hipSuccess) {
     return fail(DEX_EOOM, "device allocation for the orbital subspace failed");
   }
   int st = DEX_OK;
@@ -2295,7 +2408,6 @@ extern "C" int dex_diagsubspace_device(dex_ctx *c, const double *orbitals, int32
     }
   }
   if (hipStreamSynchronize(c->stream) != hipSuccess && st == DEX_OK) st = fail(DEX_EHIP, "sync");
-  cleanup();
   return st;
 }
 
@@ -2309,16 +2421,13 @@ extern "C" int dex_gplmr_eig(dex_ctx *c, double *x, double *e, int32_t m, int32_
   DEX_HIP(hipSetDevice(c->p.device));
   const size_t bytes = size_t(c->d) * nev * sizeof(Dbl2);
   void *dx = nullptr;
-  DEX_HIP(hipMalloc(&dx, bytes));
+  Blocks blocks(c->p.device, c->stream);
+  DEX_HIP(blocks.take(&dx, bytes));
   hipError_t err = hipMemcpy(dx, x, bytes, hipMemcpyHostToDevice);
-  if (err != hipSuccess) {
-    (void)hipFree(dx);
-    return hip_fail(err, "copy in");
-  }
+  if (err != hipSuccess) return hip_fail(err, "copy in");
   int st = dex_gplmr_eig_device(c, dx, e, m, mb, sigma_re, sigma_im, nev, ns, maxit, tol, inner_iter,
                                 outmodulus, opts, res);
   err = hipMemcpy(x, dx, bytes, hipMemcpyDeviceToHost);
-  (void)hipFree(dx);
   if (err != hipSuccess && st == DEX_OK) return hip_fail(err, "copy out");
   return st;
 }
@@ -2331,8 +2440,16 @@ extern "C" int dex_heplus_lanczos_device(dex_ctx *c, int32_t blocksize, int32_t 
   std::vector<cd> eig, vecs;
   std::vector<double> resid;
   int iters = 0;
-  const int st = dex::heplus_lanczos(c->stream, c->nn, c->d_vn, c->coef, blocksize, kdim, check, tol, numeigs,
-                                     seed, eig, vecs, resid, iters);
+  auto run = [&]() {
+    return dex::heplus_lanczos(c->stream, c->nn, c->d_vn, c->coef, blocksize, kdim, check, tol, numeigs, seed, eig,
+                               vecs, resid, iters);
+  };
+  int st = run();
+  if (st == DEX_EOOM) {  // nothing has run: once more without the idle blocks
+    (void)hipGetLastError();
+    drop_idle(c->p.device);
+    st = run();
+  }
   if (st != DEX_OK && st != DEX_ENOTCONVERGED) return st;
   for (int k = 0; k < numeigs && k < int(eig.size()); ++k) {
     eigenvalues[2 * k] = eig[k].real();
@@ -2348,8 +2465,10 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
                                     double *res_out) {
   if (!c || !x_dev || !e || !res_out) return fail(DEX_EINVAL, "null argument");
   DEX_HIP(hipSetDevice(c->p.device));
-  Dbl2 *ax = nullptr;
-  DEX_HIP(hipMalloc(&ax, size_t(c->d) * sizeof(Dbl2)));
+  void *v = nullptr;
+  Blocks blocks(c->p.device, c->stream);
+  DEX_HIP(blocks.take(&v, size_t(c->d) * sizeof(Dbl2)));
+  Dbl2 *ax = static_cast<Dbl2 *>(v);
   int st = DEX_OK;
   for (int j = 0; j < nev && st == DEX_OK; ++j) {
     const Dbl2 *xj = static_cast<const Dbl2 *>(x_dev) + size_t(j) * c->d;
@@ -2364,7 +2483,6 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
     if (st) break;
     res_out[j] = std::sqrt(aa[0]) / std::sqrt(bb[0]);
   }
-  (void)hipFree(ax);
   return st;
 }
 
