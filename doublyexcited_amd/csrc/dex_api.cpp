@@ -2225,7 +2225,7 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
   if (symmetry != 0 && !c->fast64) return fail(DEX_EUNSUPPORTED, "exchange-symmetric matvec needs the LDS kernels for this grid");
   if (x_dev == px_dev) return fail(DEX_EINVAL, "X and PX must not alias");
   DEX_HIP(hipSetDevice(c->p.device));
-  Solver S{c, nev, 1, false, false, symmetry};
+  Solver S{c, nev, 1, false, symmetry};
   Blocks blocks(c->p.device, c->stream);
   std::vector<Dbl2 *> store;
   S.blocks = &blocks;

@@ -71,3 +71,20 @@ def test_the_last_context_gives_the_memory_back(dex):
         held = before - torch.cuda.mem_get_info()[0]
         assert held >= 28 * 16 * g.d
     assert before - torch.cuda.mem_get_info()[0] <= 32 << 20  # allocator granularity
+
+
+def test_inner_solve_uses_its_exchange_symmetry(dex):
+    """The inner solve of a symmetric block applies H by the exchange-symmetric
+    passes, and agrees with the general ones to rounding."""
+    print("case: inner solve symmetry", flush=True)
+    with dex.HeliumGrid(3, 0.5, 0.3) as g:
+        x = _block(g, 3, 7)
+        got = {}
+        for sym in (0, 1):
+            g.reset_kernel_stats()
+            y = torch.empty_like(x)
+            g.precblock_device(x, y, 3, -0.7 - 0.002j, 3, symmetry=sym)
+            totals = g.kernel_totals()
+            assert (totals["symadd"][0] > 0) == (sym != 0) and (totals["pass2"][0] > 0) == (sym == 0)
+            got[sym] = y
+        assert (got[0] - got[1]).abs().max().item() <= 1e-9 * got[0].abs().max().item()
