@@ -195,8 +195,7 @@ struct dex_ctx {
   dex::MatvecCoef coef{};
   hipStream_t stream = nullptr;
   bool fast64 = false, fast32 = false;
-  void *d_u = nullptr;  // matvec intermediate, D complex128 (also used as D complex64)
-  void *d_ub = nullptr;  // intermediates of a batched matvec launch: batch_cols(c) x D complex128
+  void *d_u = nullptr;  // the general matvec's intermediate, D complex128 (also used as D complex64)
   void *d_scratch = nullptr;  // this device's copy of `scratch` (dex_matvec_noalloc)
   ColDesc *d_desc = nullptr;
   unsigned char *d_args = nullptr;  // a combine's descriptors, C and beta, packed (one upload)
@@ -326,91 +325,78 @@ int ensure_u(dex_ctx *c) {
   return 0;
 }
 
-// Columns per batched matvec launch: as many intermediates as fit in 512 MiB,
-// at most kBatchMax (16 at NN = 11, 6 at NN = 13, 2 at NN = 15, none from
-// NN = 17 on, where one column's passes already fill the device).
-int64_t batch_cols(const dex_ctx *c) {
-  const int64_t b = (int64_t(512) << 20) / (c->d * 16);
-  return b >= 2 ? std::min<int64_t>(b, dex::kBatchMax) : 1;
+// Exchange-symmetric columns of the next pair of matvec launches, `left` being
+// left: small grids need many to fill the device (16 columns at NN = 9: 224 us
+// singly, 104 together; 10 at NN = 11: 286 and, by fives, 222), large ones a few
+// so that one column's last workgroups do not leave it idle (4 at NN = 17: 1628
+// and 1551 us).  Beyond 256 MB a batch's vectors outgrow the last-level cache in
+// which the second launch finds the first one's output, so larger grids stop at
+// 4.  Batches of a call are even: a last launch of one column would cost as much
+// as many.
+constexpr size_t kBatchBytes = size_t(256) << 20;
+constexpr size_t kBatchMin = 4;
+int batch_cols(const dex_ctx *c, int io, int left) {
+  const size_t b = kBatchBytes / (size_t(c->d) * (io == dex::kIoF32 ? 8 : 16));
+  const int most = int(std::min<size_t>(std::max(b, kBatchMin), size_t(dex::kBatchMax)));
+  const int launches = (left + most - 1) / most;
+  return launches > 1 ? (left + launches - 1) / launches : left;
 }
 
-int ensure_ub(dex_ctx *c) {
-  if (c->d_ub || batch_cols(c) < 2) return 0;
-  DEX_HIP(device_malloc(c->p.device, &c->d_ub, size_t(batch_cols(c)) * size_t(c->d) * sizeof(Dbl2)));
-  return 0;
-}
-
-// H on ncols columns with X = sym X^T (sym = +-1) in two launches (batched
-// electron-1 pass, batched transpose-add pass).  io: dex::kIoF64 (complex128,
-// FP64), kIoMixed (complex128, FP32 arithmetic) or kIoF32 (complex64 columns).
-int apply_h_batch(dex_ctx *c, const Dbl2 *const *x, Dbl2 *const *y, int ncols, int io, int sym) {
-  const bool single = io != dex::kIoF64;
-  if (ncols < 1 || ncols > batch_cols(c) || sym == 0 || !(single ? c->fast32 : c->fast64))
-    return fail(DEX_EINVAL, "batched matvec: bad column count or form");
-  if (int st = ensure_ub(c)) return st;
+// H on one column, or with sym = +-1 (X = sym X^T) on up to dex::kBatchMax
+// columns, by the LDS kernels.  io: kIoF64 (complex128, FP64), kIoMixed
+// (complex128, FP32 arithmetic) or kIoF32 (complex64 columns, FP32).  u: the
+// general form's intermediate.  pass_events: also record c->ev[0..2] around the
+// passes (the matvec entry point's per-pass timing).
+int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int ncols, int sym, void *u,
+                bool pass_events = false) {
   const double dd = double(c->d) * ncols, nn = double(c->nn);
-  const double ub = single ? 8.0 : 16.0;     // intermediate U entry bytes
-  const double xb = io == dex::kIoF32 ? 8.0 : 16.0;  // X and Y entry bytes
-  const void *xs[dex::kBatchMax];
-  void *us[dex::kBatchMax];
-  void *ys[dex::kBatchMax];
-  for (int j = 0; j < ncols; ++j) {
-    xs[j] = x[j];
-    us[j] = static_cast<char *>(c->d_ub) + size_t(j) * size_t(c->d) * sizeof(Dbl2);
-    ys[j] = y[j];
-  }
+  const double xb = io == dex::kIoF32 ? 8.0 : 16.0;               // X and Y entry bytes
+  const double zb = sym != 0 ? xb : (io == dex::kIoF64 ? 16.0 : 8.0);  // Z entry bytes
+  const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  if (pass_events) DEX_HIP(hipEventRecord(c->ev[0], c->stream));
   {
-    KTimer kt(c, DEX_K_PASS1, (xb + ub) * dd, 12.0 * nn * dd);
-    DEX_HIP(dex::launch_pass1_batch(c->nn, io, xs, us, ncols, c->stream));
+    // reads X, writes Z; three axes of NN real-by-complex MACs an entry and the potential
+    KTimer kt(c, DEX_K_PASS1, (xb + zb) * dd, (12.0 * nn + 16.0) * dd);
+    DEX_HIP(dex::launch_pass1(c->nn, io, sym != 0, x, sym != 0 ? y : &u, ncols, pot, c->stream));
   }
-  {
-    KTimer kt(c, DEX_K_SYMADD, (2.0 * xb + ub) * dd, 24.0 * dd);
-    DEX_HIP(dex::launch_symadd_batch(c->nn, io, xs, us, ys, ncols, c->d_vn, c->d_tinv, c->coef, sym,
-                                     c->stream));
+  if (pass_events) DEX_HIP(hipEventRecord(c->ev[1], c->stream));
+  if (sym != 0) {
+    KTimer kt(c, DEX_K_SYMADD, 2.0 * xb * dd, 2.0 * dd);
+    DEX_HIP(dex::launch_symfold(c->nn, io, y, ncols, sym, c->stream));
+  } else {
+    KTimer kt(c, DEX_K_PASS2, (2.0 * xb + zb) * dd, (12.0 * nn + 8.0) * dd);
+    DEX_HIP(dex::launch_pass2(c->nn, io, x[0], u, y[0], c->coef, c->stream));
   }
+  if (pass_events) DEX_HIP(hipEventRecord(c->ev[2], c->stream));
   return 0;
 }
 
-// Second pass: the general electron-2 cube pass, or for X = sym X^T (sym = +-1)
-// the transpose-add pass.
-hipError_t second_pass(dex_ctx *c, int io, const void *x, void *y, int sym) {
-  if (sym != 0)
-    return dex::launch_symadd(c->nn, io, x, c->d_u, y, c->d_vn, c->d_tinv, c->coef, sym, c->stream);
-  return dex::launch_pass2(c->nn, io, x, c->d_u, y, c->d_vn, c->d_tinv, c->coef, c->stream);
+// H on exchange-(anti)symmetric columns, a batch per pair of launches.
+int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, int io, int sym) {
+  if (ncols < 0 || sym == 0 || !(io != dex::kIoF64 ? c->fast32 : c->fast64))
+    return fail(DEX_EINVAL, "batched matvec: bad column count or form");
+  for (int j = 0, k = 0; j < ncols; j += k) {
+    k = batch_cols(c, io, ncols - j);
+    if (int st = fast_passes(c, io, x + j, y + j, k, sym, nullptr)) return st;
+  }
+  return 0;
 }
 
 // One application of H on complex128 device vectors; `single` selects FP32
-// arithmetic (complex64 intermediate, complex128 in and out).
-// pass_events: also record c->ev[0..2] around the two passes (the matvec
-// entry point's per-pass timing).
+// arithmetic (complex128 in and out).
 int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool pass_events = false) {
-  if (int st = ensure_u(c)) return st;
-  hipStream_t s = c->stream;
   const bool fast = single ? c->fast32 : c->fast64;
   if (single && !fast) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
   if (fast) {
-    const int io = single ? dex::kIoMixed : dex::kIoF64;
-    if (c->timing && pass_events) DEX_HIP(hipEventRecord(c->ev[0], s));
-    const double dd = double(c->d), nn = double(c->nn);
-    const double ub = single ? 8.0 : 16.0;  // intermediate U entry bytes
-    {
-      // reads X, writes U; three axes of NN real-by-complex MACs per entry
-      KTimer kt(c, DEX_K_PASS1, (16.0 + ub) * dd, 12.0 * nn * dd);
-      DEX_HIP(dex::launch_pass1(c->nn, io, x, c->d_u, s));
-    }
-    if (c->timing && pass_events) DEX_HIP(hipEventRecord(c->ev[1], s));
-    {
-      // reads U and X, writes Y; the general pass also applies the three
-      // electron-2 axes, the transpose-add pass the exchange image
-      const double fl = sym != 0 ? 24.0 * dd : (12.0 * nn + 14.0) * dd;
-      KTimer kt(c, sym != 0 ? DEX_K_SYMADD : DEX_K_PASS2, (32.0 + ub) * dd, fl);
-      DEX_HIP(second_pass(c, io, x, y, sym));
-    }
-    if (c->timing && pass_events) DEX_HIP(hipEventRecord(c->ev[2], s));
-    return 0;
+    if (sym == 0)
+      if (int st = ensure_u(c)) return st;
+    const void *xp = x;
+    void *yp = y;
+    return fast_passes(c, single ? dex::kIoMixed : dex::kIoF64, &xp, &yp, 1, sym, c->d_u,
+                       pass_events && c->timing);
   }
   KTimer kt(c, DEX_K_GENERIC, 32.0 * double(c->d), (24.0 * c->nn + 14.0) * double(c->d));
-  DEX_HIP(dex::launch_matvec_generic(c->nn, x, y, c->d_vn, c->d_tinv, c->coef, s));
+  DEX_HIP(dex::launch_matvec_generic(c->nn, x, y, c->d_vn, c->d_tinv, c->coef, c->stream));
   // The general operator carries the rounding-level exchange-odd (even) part of
   // an exchange-even (odd) x into y, where the transpose-add kernels, which the
   // mixed form applies to its complex64 blocks, drop it: in a solve that mixes
@@ -418,25 +404,18 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
   // part, and the iteration drifts away from the wanted levels after tens of
   // iterations (seen at NN=25, where FP64 has only these kernels).  Projecting y
   // keeps both paths on the exchange-symmetric subspace.
-  if (sym != 0) DEX_HIP(dex::launch_sym_project(y, c->m, sym > 0 ? 1 : -1, s));
+  if (sym != 0) DEX_HIP(dex::launch_sym_project(y, c->m, sym > 0 ? 1 : -1, c->stream));
   return 0;
 }
 
 // H on complex64 device vectors in FP32 arithmetic (x, y hold D complex64).
-int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym) {
-  if (int st = ensure_u(c)) return st;
+int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym, bool pass_events = false) {
   if (!c->fast32) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
-  const double dd = double(c->d), nn = double(c->nn);
-  {
-    KTimer kt(c, DEX_K_PASS1, 16.0 * dd, 12.0 * nn * dd);
-    DEX_HIP(dex::launch_pass1(c->nn, dex::kIoF32, x, c->d_u, c->stream));
-  }
-  {
-    const double fl = sym != 0 ? 24.0 * dd : (12.0 * nn + 14.0) * dd;
-    KTimer kt(c, sym != 0 ? DEX_K_SYMADD : DEX_K_PASS2, 24.0 * dd, fl);
-    DEX_HIP(second_pass(c, dex::kIoF32, x, y, sym));
-  }
-  return 0;
+  if (sym == 0)
+    if (int st = ensure_u(c)) return st;
+  const void *xp = x;
+  void *yp = y;
+  return fast_passes(c, dex::kIoF32, &xp, &yp, 1, sym, c->d_u, pass_events && c->timing);
 }
 
 // ---- block helpers on one context ------------------------------------------
@@ -830,7 +809,7 @@ int dex_ctx_destroy(dex_ctx *c) {
   if (!c) return DEX_OK;
   (void)hipSetDevice(c->p.device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  for (void *ptr : {(void *)c->d_tinv, (void *)c->d_vn, c->d_u, c->d_ub, (void *)c->d_desc,
+  for (void *ptr : {(void *)c->d_tinv, (void *)c->d_vn, c->d_u, (void *)c->d_desc,
                     (void *)c->d_args, (void *)c->d_gram_out, c->d_partial,
                     (void *)c->d_dots})
     if (ptr) (void)hipFree(ptr);
@@ -953,39 +932,23 @@ int dex_matvec_sym_device(dex_ctx *c, const void *in, void *out, int32_t howmany
   const bool sp = single != 0;
   if (sp && c->p.precision != DEX_FP32) return fail(DEX_EINVAL, "complex64 I/O needs an FP32 context");
   if (sp && !c->fast32) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
-  if (int st = ensure_u(c)) return st;
-  const int nb = int(batch_cols(c));
-  if (!sp && symmetry != 0 && !c->timing && howmany >= 2 && nb >= 2 &&
-      (c->p.precision == DEX_FP32 ? c->fast32 : c->fast64)) {
-    // exchange-symmetric complex128 columns: nb per pair of launches
-    std::vector<const Dbl2 *> xs(howmany);
-    std::vector<Dbl2 *> ys(howmany);
+  const bool f32 = c->p.precision == DEX_FP32;
+  const size_t xb = sp ? 8 : 16;
+  if (symmetry != 0 && !c->timing && howmany >= 2) {
+    // exchange-symmetric columns, a batch per pair of launches
+    std::vector<const void *> xs(howmany);
+    std::vector<void *> ys(howmany);
     for (int j = 0; j < howmany; ++j) {
-      xs[j] = static_cast<const Dbl2 *>(in) + size_t(j) * c->d;
-      ys[j] = static_cast<Dbl2 *>(out) + size_t(j) * c->d;
+      xs[j] = static_cast<const char *>(in) + size_t(j) * size_t(c->d) * xb;
+      ys[j] = static_cast<char *>(out) + size_t(j) * size_t(c->d) * xb;
     }
-    for (int j0 = 0; j0 < howmany; j0 += nb) {
-      const int k = std::min(nb, howmany - j0);
-      if (int st = apply_h_batch(c, xs.data() + j0, ys.data() + j0, k,
-                                 c->p.precision == DEX_FP32 ? dex::kIoMixed : dex::kIoF64, symmetry))
-        return st;
-    }
-    return DEX_OK;
+    return apply_h_batch(c, xs.data(), ys.data(), howmany, sp ? dex::kIoF32 : (f32 ? dex::kIoMixed : dex::kIoF64),
+                         symmetry);
   }
   for (int j = 0; j < howmany; ++j) {
-    if (sp) {
-      const char *xi = static_cast<const char *>(in) + size_t(j) * c->d * 8;
-      char *yo = static_cast<char *>(out) + size_t(j) * c->d * 8;
-      if (c->timing) DEX_HIP(hipEventRecord(c->ev[0], c->stream));
-      DEX_HIP(dex::launch_pass1(c->nn, dex::kIoF32, xi, c->d_u, c->stream));
-      if (c->timing) DEX_HIP(hipEventRecord(c->ev[1], c->stream));
-      DEX_HIP(second_pass(c, dex::kIoF32, xi, yo, symmetry));
-      if (c->timing) DEX_HIP(hipEventRecord(c->ev[2], c->stream));
-    } else {
-      const Dbl2 *xi = static_cast<const Dbl2 *>(in) + size_t(j) * c->d;
-      Dbl2 *yo = static_cast<Dbl2 *>(out) + size_t(j) * c->d;
-      if (int st = apply_h(c, xi, yo, c->p.precision == DEX_FP32, symmetry, true)) return st;
-    }
+    const auto *xi = reinterpret_cast<const Dbl2 *>(static_cast<const char *>(in) + size_t(j) * size_t(c->d) * xb);
+    auto *yo = reinterpret_cast<Dbl2 *>(static_cast<char *>(out) + size_t(j) * size_t(c->d) * xb);
+    if (int st = sp ? apply_h32(c, xi, yo, symmetry, true) : apply_h(c, xi, yo, f32, symmetry, true)) return st;
   }
   const bool timed_fast = c->p.precision == DEX_FP32 ? c->fast32 : c->fast64;
   if (c->timing && howmany > 0 && timed_fast) {
@@ -1018,20 +981,26 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
   DEX_HIP(hipSetDevice(c->p.device));
   const int io = sp ? dex::kIoF32 : (f32 ? dex::kIoMixed : dex::kIoF64);
   const size_t xb = sp ? 8 : 16;  // bytes per entry of X and Y
-  for (int j = 0; j < howmany; ++j) {
-    const char *x = static_cast<const char *>(in) + size_t(j) * size_t(c->d) * xb;
-    char *y = static_cast<char *>(out) + size_t(j) * size_t(c->d) * xb;
-    if (!fast) {
-      DEX_HIP(dex::launch_matvec_generic(c->nn, reinterpret_cast<const Dbl2 *>(x), reinterpret_cast<Dbl2 *>(y),
-                                         c->d_vn, c->d_tinv, c->coef, c->stream));
-      continue;
+  const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  for (int j = 0, k = 0; j < howmany; j += k) {
+    k = fast && symmetry != 0 ? batch_cols(c, io, howmany - j) : 1;
+    const void *x[dex::kBatchMax];
+    void *y[dex::kBatchMax];
+    for (int i = 0; i < k; ++i) {
+      x[i] = static_cast<const char *>(in) + size_t(j + i) * size_t(c->d) * xb;
+      y[i] = static_cast<char *>(out) + size_t(j + i) * size_t(c->d) * xb;
     }
-    // U (fully written by the electron-1 pass before the second pass reads it)
-    DEX_HIP(dex::launch_pass1(c->nn, io, x, c->d_scratch, c->stream));
-    if (symmetry != 0)
-      DEX_HIP(dex::launch_symadd(c->nn, io, x, c->d_scratch, y, c->d_vn, c->d_tinv, c->coef, symmetry, c->stream));
-    else
-      DEX_HIP(dex::launch_pass2(c->nn, io, x, c->d_scratch, y, c->d_vn, c->d_tinv, c->coef, c->stream));
+    if (!fast) {
+      DEX_HIP(dex::launch_matvec_generic(c->nn, static_cast<const Dbl2 *>(x[0]), static_cast<Dbl2 *>(y[0]), c->d_vn,
+                                         c->d_tinv, c->coef, c->stream));
+    } else if (symmetry != 0) {
+      DEX_HIP(dex::launch_pass1(c->nn, io, true, x, y, k, pot, c->stream));
+      DEX_HIP(dex::launch_symfold(c->nn, io, y, k, symmetry, c->stream));
+    } else {
+      // Z (fully written by the electron-1 pass before the second pass reads it)
+      DEX_HIP(dex::launch_pass1(c->nn, io, false, x, &c->d_scratch, 1, pot, c->stream));
+      DEX_HIP(dex::launch_pass2(c->nn, io, x[0], c->d_scratch, y[0], c->coef, c->stream));
+    }
   }
   return DEX_OK;
 }
@@ -1179,24 +1148,20 @@ struct Solver {
   int matblock(const Block &in, const Block &out) {
     const double t0 = now_s();
     if (out.size() < in.size()) return fail(DEX_EINVAL, "matblock: output block too small");
-    const int nb = int(batch_cols(c));
     bool same = true;
     for (int j = 0; j < in.size(); ++j)
       if (is32(in.cols[j]) != is32(in.cols[0]) || is32(out.cols[j]) != is32(in.cols[j])) same = false;
     const bool lo = in.size() > 0 && is32(in.cols[0]);
-    if (same && sym != 0 && nb >= 2 && in.size() >= 2 && (lo ? c->fast32 : c->fast64)) {
-      // exchange-symmetric columns: nb columns per pair of launches
-      std::vector<Dbl2 *> xi, yo;
+    if (same && sym != 0 && in.size() >= 2 && (lo ? c->fast32 : c->fast64)) {
+      // exchange-symmetric columns: a batch per pair of launches
+      std::vector<const void *> xi;
+      std::vector<void *> yo;
       for (int j = 0; j < in.size(); ++j) {
         xi.push_back(untag(in.cols[j]));
         yo.push_back(untag(out.cols[j]));
       }
-      for (int j0 = 0; j0 < in.size(); j0 += nb) {
-        const int k = std::min(nb, in.size() - j0);
-        if (int st = apply_h_batch(c, xi.data() + j0, yo.data() + j0, k, lo ? dex::kIoF32 : dex::kIoF64, sym))
-          return st;
-        matvecs += k;
-      }
+      if (int st = apply_h_batch(c, xi.data(), yo.data(), in.size(), lo ? dex::kIoF32 : dex::kIoF64, sym)) return st;
+      matvecs += in.size();
       t_matvec += now_s() - t0;
       return 0;
     }
@@ -2073,25 +2038,27 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
 
 }  // namespace
 
-// Columns per batched matvec launch for vectors of d entries (batch_cols).
-int64_t batch_cols_d(int64_t d) {
+// Small grids: a margin of up to 16 vectors in the count below (512 MiB at
+// most), for work vectors of other sizes that stay listed while contexts live.
+// Admission decisions depend on it.
+int64_t margin_vectors(int64_t d) {
   const int64_t b = (int64_t(512) << 20) / (d * 16);
-  return b >= 2 ? std::min<int64_t>(b, dex::kBatchMax) : 1;
+  return b >= 2 ? std::min<int64_t>(b, dex::kBatchMax) : 0;
 }
 
 // Device bytes a context of grid nn holds apart from any solve: the tables,
 // the block kernels' descriptor, coefficient and partial-sum buffers (as
-// dex_ctx_create allocates them), and the matvec intermediates (U, and on small
-// grids those of the batched launches), which a solve's first matvec allocates.
+// dex_ctx_create allocates them), and the general matvec's intermediate, which
+// its first call allocates; and the margin above.
 int64_t ctx_fixed_bytes(int nn) {
   const int64_t m = int64_t(nn) * nn * nn, d = m * m, vec = d * 16;
   const int64_t L = 2 * nn + 1;
   const int64_t partial = int64_t(std::max(dex::gram_partial_elems(64, 128) * sizeof(Dbl2),
                                            dex::coldots_partial_elems(64) * sizeof(double)));
-  const int64_t bc = batch_cols_d(d);
   return (L * L * L + m) * 8 + int64_t(kMaxDesc) * int64_t(sizeof(ColDesc)) +
          (int64_t(kMaxDesc) * int64_t(sizeof(ColDesc)) + 2 * kMaxSmall * 16 + 512) + 192 * 192 * 16 + partial +
-         64 * 4 * 8 + vec + (bc >= 2 ? bc * vec : 0);
+         64 * 4 * 8 + vec +
+         margin_vectors(d) * vec;
 }
 
 // Bytes of a solve (nev, ns, inner_iter, opts) on a context of grid nn and the

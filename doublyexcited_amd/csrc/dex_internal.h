@@ -79,13 +79,22 @@ struct ColPtrsW {
   void *p[kBatchMax];
 };
 
-// Fast path: U = K1 X (electron 1), then Y = s2 (U + K2 X) + c1 Vr X.
-hipError_t launch_pass1(int nn, int io, const void *x, void *u, hipStream_t s);
-// pass 1 on ncols (1..kBatchMax) columns in one launch: U_j = K1 X_j
-hipError_t launch_pass1_batch(int nn, int io, const void *const *x, void *const *u, int ncols, hipStream_t s);
-hipError_t launch_pass2(int nn, int io, const void *x, const void *u, void *y,
-                        const double *vn, const double *tinv, const MatvecCoef &coef,
+// What the passes read beside the vectors.
+struct PotArgs {
+  const double *vn, *tinv;
+  MatvecCoef cf;
+};
+
+// Pass 1 on ncols (1..kBatchMax) columns: Z = s2 K1 X + w c1 Vr o X, w = 1/2 with
+// `sym` (Z in Y's format; Z may be X's storage), else 1 (Z complex128 for kIoF64,
+// complex64 otherwise).
+hipError_t launch_pass1(int nn, int io, bool sym, const void *const *x, void *const *z, int ncols,
+                        const PotArgs &pot, hipStream_t s);
+// Second pass for general vectors: Y = Z + s2 K2 X.
+hipError_t launch_pass2(int nn, int io, const void *x, const void *z, void *y, const MatvecCoef &coef,
                         hipStream_t s);
+// Second pass for X = sign X^T, in place on ncols columns: Y <- Y + sign Y^T.
+hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, hipStream_t s);
 // Generic FP64 path for any odd nn <= 27: six axis passes plus the potential.
 hipError_t launch_matvec_generic(int nn, const Dbl2 *x, Dbl2 *y, const double *vn,
                                  const double *tinv, const MatvecCoef &coef, hipStream_t s);
@@ -130,14 +139,6 @@ hipError_t launch_sym_project(Dbl2 *x, int64_t m, int sign, hipStream_t s);
 hipError_t launch_lowrank(const Dbl2 *t, const Dbl2 *x, Dbl2 *out, int64_t m, int k, hipStream_t s);
 // W = Y X (conj_x: Y conj(X)) for M x M Y and M x K X
 hipError_t launch_ywx(const Dbl2 *y, const Dbl2 *x, Dbl2 *w, int64_t m, int k, int conj_x, hipStream_t s);
-// Second matvec pass for X = sign X^T: Y = s2 (U + sign U^T) + c1 Vr o (X + sign X^T)/2.
-hipError_t launch_symadd(int nn, int io, const void *x, const void *u, void *y,
-                         const double *vn, const double *tinv, const MatvecCoef &coef, int sign,
-                         hipStream_t s);
-// the same on ncols (1..kBatchMax) columns in one launch
-hipError_t launch_symadd_batch(int nn, int io, const void *const *x, const void *const *u, void *const *y,
-                               int ncols, const double *vn, const double *tinv, const MatvecCoef &coef,
-                               int sign, hipStream_t s);
 // One-electron operator Y = s2 tau3D X + c1 vn o X on ncols columns of NN^3 entries.
 hipError_t launch_h1(const Dbl2 *x, Dbl2 *y, int nn, int ncols, const double *vn, const MatvecCoef &coef,
                      hipStream_t s);

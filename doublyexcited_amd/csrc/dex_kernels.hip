@@ -8,13 +8,15 @@
 //     Y = e^{-2 i theta} (T3D x I + I x T3D) X + e^{-i theta} Vr o X,
 // Vr(p, q) = -Z/delta^3 (Tinv(r_p) + Tinv(r_q)) + Tinv(r_q - r_p)/delta^3.
 // tau is a compile-time table, so the kinetic contraction is a stream of
-// FMAs with scalar constants.  Two passes, each over an NN^3 cube held in LDS:
-//   pass 1 (electron 1): U[:, q] = tau3D X[:, q]  (contiguous cubes),
-//   pass 2 (electron 2): Y[p, :] = s2 (U[p, :] + tau3D X[p, :]) + c1 Vr X[p, :]
-// (cubes at stride M; neighbouring p share cache lines, so the workgroup ->
-// p map keeps groups of 8 consecutive p on one XCD).  The kinetic operator is
-// real, so the real and imaginary parts are contracted in turn through two
-// LDS buffers of NN^3 reals each (148 KB at NN = 21 in FP64).
+// FMAs with scalar constants.  Two passes:
+//   pass 1 (electron 1): Z[:, q] = s2 tau3D X[:, q] + w c1 Vr X[:, q]  (contiguous
+//     cubes in LDS),
+//   exchange-(anti)symmetric vectors (w = 1/2): Y = Z + sign Z^T, in place,
+//   general ones (w = 1): Y[p, :] = Z[p, :] + s2 tau3D X[p, :]  (cubes at stride
+//     M; neighbouring p share cache lines, so the workgroup -> p map keeps groups
+//     of 8 consecutive p on one XCD).
+// The kinetic operator is real, so the real and imaginary parts are contracted
+// in turn through two LDS buffers of NN^3 reals each (148 KB at NN = 21 in FP64).
 #include <atomic>
 #include <cstdlib>
 #include <mutex>
@@ -54,6 +56,17 @@ struct Cplx<float> {
   using type = float2;
 };
 
+template <typename T>
+struct Real;
+template <>
+struct Real<double2> {
+  using type = double;
+};
+template <>
+struct Real<float2> {
+  using type = float;
+};
+
 constexpr int round_up(int a, int b) { return (a + b - 1) / b * b; }
 
 template <int NN>
@@ -61,136 +74,122 @@ constexpr int cube_threads() {
   return round_up(NN * NN, 64) > 1024 ? 1024 : round_up(NN * NN, 64);
 }
 
-// b = tau3D a on one NN^3 cube in LDS (a, b: NN^3 reals, i fastest).
-// One thread per line: it reads the NN inputs of its line once and forms all
-// NN outputs with NN^2 FMAs against compile-time coefficients.
-template <int NN, int NT, typename R>
-__device__ __forceinline__ void cube_apply(const R *__restrict__ a, R *__restrict__ b, int tid) {
+// emit(i, y_i) for y = tau x along one axis of NN = 2 H + 1 points.  tau is a
+// symmetric Toeplitz matrix, so it maps the even and the odd part of a line (about
+// its centre) to themselves: with s_m = x_{H+m} + x_{H-m} and d_m = x_{H+m} - x_{H-m},
+//   y_{H+-n} = tau(n) x_H + sum_m (tau(n-m) + tau(n+m)) s_m / 2
+//              +- sum_m (tau(n-m) - tau(n+m)) d_m / 2,
+// (H + 1)^2 + H^2 multiply-adds and 4 H additions a line in place of NN^2
+// multiply-adds (221 + 40 for 441 at NN = 21), with compile-time coefficients.
+template <int NN, typename R, typename F>
+__device__ __forceinline__ void line_apply(const R (&x)[NN], F &&emit) {
+  constexpr int H = NN / 2;
+  R s[H + 1], d[H + 1];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    s[m] = x[H + m] + x[H - m];
+    d[m] = x[H + m] - x[H - m];
+  }
+  R y0 = R(tau_rt(0)) * x[H];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) y0 += R(tau_rt(m)) * s[m];
+  emit(H, y0);
+#pragma unroll
+  for (int n = 1; n <= H; ++n) {
+    R e = R(tau_rt(n)) * x[H], o = R((tau_rt(n - 1) - tau_rt(n + 1)) / 2) * d[1];
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      e += R((tau_rt(n - m) + tau_rt(n + m)) / 2) * s[m];
+      if (m > 1) o += R((tau_rt(n - m) - tau_rt(n + m)) / 2) * d[m];
+    }
+    emit(H + n, e + o);
+    emit(H - n, e - o);
+  }
+}
+
+// The i and j axes of tau3D on one NN^3 cube of reals, one thread per line:
+// thread c < NN^2 holds the k line through (i, j), c = i + NN j, in x (the order
+// of the global loads, so the k axis costs no LDS access).  a is the cube; b
+// collects the two axes' sums, which thread c then finds at b[c + NN^2 k].
+template <int NN, typename R>
+__device__ __forceinline__ void plane_axes(const R (&x)[NN], R *__restrict__ a, R *__restrict__ b, int c) {
   constexpr int N2 = NN * NN;
-  // axis i (stride 1): line c = (j, k), base c * NN
-  for (int c = tid; c < N2; c += NT) {
-    R acc[NN];
+  const bool on = c < N2;
+  if (on) {
 #pragma unroll
-    for (int i = 0; i < NN; ++i) acc[i] = R(0);
-#pragma unroll
-    for (int l = 0; l < NN; ++l) {
-      const R xv = a[c * NN + l];
-#pragma unroll
-      for (int i = 0; i < NN; ++i) acc[i] += R(tau_rt(l - i)) * xv;
-    }
-#pragma unroll
-    for (int i = 0; i < NN; ++i) b[c * NN + i] = acc[i];
+    for (int k = 0; k < NN; ++k) a[c + N2 * k] = x[k];
   }
   __syncthreads();
-  // axis j (stride NN): line c = (i, k)
-  for (int c = tid; c < N2; c += NT) {
-    const int i = c % NN, k = c / NN;
-    const int base = i + N2 * k;
-    R acc[NN];
+  if (on) {  // axis i: line (j, k) = c
+    R v[NN];
 #pragma unroll
-    for (int j = 0; j < NN; ++j) acc[j] = R(0);
-#pragma unroll
-    for (int l = 0; l < NN; ++l) {
-      const R xv = a[base + NN * l];
-#pragma unroll
-      for (int j = 0; j < NN; ++j) acc[j] += R(tau_rt(l - j)) * xv;
-    }
-#pragma unroll
-    for (int j = 0; j < NN; ++j) b[base + NN * j] += acc[j];
+    for (int l = 0; l < NN; ++l) v[l] = a[c * NN + l];
+    line_apply<NN, R>(v, [&](int i, R y) { b[c * NN + i] = y; });
   }
   __syncthreads();
-  // axis k (stride NN^2): line c = (i, j)
-  for (int c = tid; c < N2; c += NT) {
-    R acc[NN];
+  if (on) {  // axis j: line (i, k)
+    const int base = c % NN + N2 * (c / NN);
+    R v[NN];
 #pragma unroll
-    for (int k = 0; k < NN; ++k) acc[k] = R(0);
-#pragma unroll
-    for (int l = 0; l < NN; ++l) {
-      const R xv = a[c + N2 * l];
-#pragma unroll
-      for (int k = 0; k < NN; ++k) acc[k] += R(tau_rt(l - k)) * xv;
-    }
-#pragma unroll
-    for (int k = 0; k < NN; ++k) b[c + N2 * k] += acc[k];
+    for (int l = 0; l < NN; ++l) v[l] = a[base + NN * l];
+    line_apply<NN, R>(v, [&](int j, R y) { b[base + NN * j] += y; });
   }
   __syncthreads();
 }
 
-// Pass 1: electron-1 cubes (contiguous, one per electron-2 index q).
-// U = tau3D X on each cube (no phase, no potential).  Workgroups are
-// persistent: while a workgroup contracts cube q in LDS, the loads of its next
-// cube (q + gridDim.x) are already in flight into registers.
-template <int NN, typename R, typename XT>
-__global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtrsW us, int ncols) {
-  using C = typename Cplx<R>::type;
-  constexpr int NT = cube_threads<NN>();
-  constexpr int N3 = NN * NN * NN;
-  constexpr int PER = (N3 + NT - 1) / NT;
+// Electron-1 pass on the cube of electron-2 index q = blockIdx.x (contiguous) of
+// column blockIdx.y: Z = s2 tau3D X + w c1 Vr o X.  w = 1/2 for
+// exchange-(anti)symmetric vectors (Y = Z + sign Z^T follows, k_symfold), 1 for
+// general ones (Y = Z + s2 K2 X follows, k_pass2).  A workgroup reads its whole
+// cube before it writes, so Z may be X's own storage.
+//
+// One workgroup a cube: the LDS cube and the registers of three lines leave one
+// workgroup (7 waves) on a CU at NN = 21 in FP64, two in FP32, and a new workgroup's
+// loads need not wait for the last one's stores, as they do in a loop over cubes
+// (a wave's memory operations complete in order).  The loop also let the compiler
+// keep vn in registers, which cost the second workgroup: FP32 at NN = 19 ran 277 us
+// a column looped and 175 us not, at NN = 21 487 and 354.
+template <int NN, typename R, typename XT, typename ZT>
+__global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtrsW zs, const double *__restrict__ vn,
+                                                              const double *__restrict__ tinv, MatvecCoef cf,
+                                                              double w) {
+  constexpr int N2 = NN * NN;
+  constexpr int N3 = NN * N2;
+  constexpr int L = 2 * NN + 1;
   extern __shared__ __align__(16) unsigned char smem[];
   R *a = reinterpret_cast<R *>(smem);
   R *b = a + N3;
-  const int tid = threadIdx.x;
-  // work item q: cube q % N3 of column q / N3
-  const int64_t total = int64_t(ncols) * N3;
-  auto xcube = [&](int64_t qq) {
-    const int cc = int(qq / N3);
-    return static_cast<const XT *>(xs.p[cc]) + (qq - int64_t(cc) * N3) * N3;
-  };
-  XT pre[PER];
-  int64_t q = blockIdx.x;
-  if (q < total) {
-    const XT *xq = xcube(q);
+  const int c = threadIdx.x;
+  const bool on = c < N2;
+  const int q = blockIdx.x;
+  const XT *xq = static_cast<const XT *>(xs.p[blockIdx.y]) + int64_t(q) * N3;
+  R xr[NN], xi[NN], kr[NN];
+  if (on) {
 #pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int e = tid + t * NT;
-      if (e < N3) pre[t] = xq[e];
+    for (int k = 0; k < NN; ++k) {
+      const XT v = xq[c + N2 * k];
+      xr[k] = R(v.x);
+      xi[k] = R(v.y);
     }
   }
-  for (; q < total; q += gridDim.x) {
-    R keep[PER];
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int e = tid + t * NT;
-      if (e < N3) {
-        a[e] = R(pre[t].x);
-        keep[t] = R(pre[t].y);
-      }
-    }
-    __syncthreads();
-    const int64_t qn = q + gridDim.x;
-    if (qn < total) {
-      const XT *xq = xcube(qn);
-#pragma unroll
-      for (int t = 0; t < PER; ++t) {
-        const int e = tid + t * NT;
-        if (e < N3) pre[t] = xq[e];
-      }
-    }
-    cube_apply<NN, NT, R>(a, b, tid);
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int e = tid + t * NT;
-      if (e < N3) {
-        const R re = b[e];
-        a[e] = keep[t];
-        keep[t] = re;
-      }
-    }
-    __syncthreads();
-    cube_apply<NN, NT, R>(a, b, tid);
-    const int cq = int(q / N3);
-    C *uq = static_cast<C *>(us.p[cq]) + (q - int64_t(cq) * N3) * N3;
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int e = tid + t * NT;
-      if (e < N3) {
-        C o;
-        o.x = keep[t];
-        o.y = b[e];
-        uq[e] = o;
-      }
-    }
-    __syncthreads();
+  plane_axes<NN, R>(xr, a, b, c);
+  if (on) line_apply<NN, R>(xr, [&](int k, R y) { kr[k] = y + b[c + N2 * k]; });
+  plane_axes<NN, R>(xi, a, b, c);
+  if (on) {
+    const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(w * cf.c1_re), c1i = R(w * cf.c1_im);
+    const int iq = q % NN, jq = (q / NN) % NN, kq = q / N2;
+    const int t0 = (iq - c % NN + NN) + L * ((jq - c / NN + NN) + L * (kq + NN));
+    const double vq = vn[q];
+    ZT *zq = static_cast<ZT *>(zs.p[blockIdx.y]) + int64_t(q) * N3;
+    line_apply<NN, R>(xi, [&](int k, R y) {
+      const R ki = y + b[c + N2 * k];
+      const R vr = R(vn[c + N2 * k] + vq + tinv[t0 - L * L * k] * cf.inv_d3);
+      const R vxr = vr * xr[k], vxi = vr * xi[k];
+      ZT o;
+      o.x = s2r * kr[k] - s2i * ki + c1r * vxr - c1i * vxi;
+      o.y = s2r * ki + s2i * kr[k] + c1r * vxi + c1i * vxr;
+      zq[c + N2 * k] = o;
+    });
   }
 }
 
@@ -205,142 +204,109 @@ __device__ __forceinline__ int64_t xcd_group_map(int64_t b, int64_t m) {
   return 8 * (x + 8 * (s / 8)) + (s % 8);
 }
 
+// Electron-2 pass for general vectors: Y = Z + s2 tau3D X on the stride-M cube
+// of each electron-1 index p (Z from k_pass1 with w = 1).
 template <int NN, typename R, typename XT, typename YT>
 __global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(
-    const XT *__restrict__ x, const typename Cplx<R>::type *__restrict__ u, YT *__restrict__ y,
-    const double *__restrict__ vn, const double *__restrict__ tinv, MatvecCoef cf) {
+    const XT *__restrict__ x, const typename Cplx<R>::type *__restrict__ z, YT *__restrict__ y, MatvecCoef cf) {
   using C = typename Cplx<R>::type;
-  constexpr int NT = cube_threads<NN>();
-  constexpr int N3 = NN * NN * NN;
-  constexpr int PER = (N3 + NT - 1) / NT;
-  constexpr int L = 2 * NN + 1;
+  constexpr int N2 = NN * NN;
+  constexpr int N3 = NN * N2;
   extern __shared__ __align__(16) unsigned char smem[];
   R *a = reinterpret_cast<R *>(smem);
   R *b = a + N3;
-  const int tid = threadIdx.x;
+  const int c = threadIdx.x;
+  const bool on = c < N2;
   const int64_t p = xcd_group_map(blockIdx.x, N3);
   const int64_t M = N3;
-  R keep[PER];
+  R xr[NN], xi[NN], kr[NN];
+  if (on) {
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int e = tid + t * NT;
-    if (e < N3) {
-      const XT v = x[p + M * e];
-      a[e] = R(v.x);
-      keep[t] = R(v.y);
+    for (int k = 0; k < NN; ++k) {
+      const XT v = x[p + M * (c + N2 * k)];
+      xr[k] = R(v.x);
+      xi[k] = R(v.y);
     }
   }
-  __syncthreads();
-  cube_apply<NN, NT, R>(a, b, tid);
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int e = tid + t * NT;
-    if (e < N3) {
-      const R re = b[e];
-      a[e] = keep[t];
-      keep[t] = re;
-    }
-  }
-  __syncthreads();
-  cube_apply<NN, NT, R>(a, b, tid);
-  // epilogue: Y = s2 (U + K) + c1 Vr X
-  const int ip = int(p % NN), jp = int((p / NN) % NN), kp = int(p / (NN * NN));
-  const double vnp = vn[p];
-  const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(cf.c1_re), c1i = R(cf.c1_im);
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int e = tid + t * NT;
-    if (e < N3) {
-      const int iq = e % NN, jq = (e / NN) % NN, kq = e / (NN * NN);
-      const int ti = (iq - ip + NN) + L * ((jq - jp + NN) + L * (kq - kp + NN));
-      const R vr = R(vnp + vn[e] + tinv[ti] * cf.inv_d3);
-      const C uv = u[p + M * e];
-      const XT xv = x[p + M * e];
-      const R sr = uv.x + keep[t], si = uv.y + b[e];
-      const R vxr = vr * R(xv.x), vxi = vr * R(xv.y);
+  plane_axes<NN, R>(xr, a, b, c);
+  if (on) line_apply<NN, R>(xr, [&](int k, R y) { kr[k] = y + b[c + N2 * k]; });
+  plane_axes<NN, R>(xi, a, b, c);
+  if (on) {
+    const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
+    line_apply<NN, R>(xi, [&](int k, R t) {
+      const R ki = t + b[c + N2 * k];
+      const C zv = z[p + M * (c + N2 * k)];
       YT o;
-      o.x = s2r * sr - s2i * si + c1r * vxr - c1i * vxi;
-      o.y = s2r * si + s2i * sr + c1r * vxi + c1i * vxr;
-      y[p + M * e] = o;
-    }
+      o.x = zv.x + (s2r * kr[k] - s2i * ki);
+      o.y = zv.y + (s2r * ki + s2i * kr[k]);
+      y[p + M * (c + N2 * k)] = o;
+    });
   }
 }
 
 // ---- exchange-symmetric second pass ------------------------------------------
 // For X = sign X^T (sign = +1 singlet, -1 triplet) electron 2's kinetic term is
-// the transpose of electron 1's: (I x T3D) X = sign (T3D X)^T.  So after pass 1
-// (U = tau3D X) the result is Y = s2 (U + sign U^T) + c1 Vr o Xs with
-// Xs = (X + sign X^T) / 2, formed tile pair by tile pair: a workgroup owns the
-// 32 x 32 tile (ta, tb), ta <= tb, and its mirror (tb, ta); all global
-// accesses run along p (coalesced) and the transposes go through LDS.  Each
-// unordered pair {(p, q), (q, p)} is computed once and written with its sign,
-// so the output is exactly (anti)symmetric.
+// the transpose of electron 1's: (I x T3D) X = sign (T3D X)^T, and Vr = Vr^T.
+// So after pass 1 (Z = s2 tau3D X + c1 Vr o X / 2, in Y's storage) the result is
+// Y = Z + sign Z^T, in place: a workgroup owns the 32 x 32 tile (ta, tb),
+// ta <= tb, and its mirror (tb, ta); all global accesses run along p (coalesced)
+// and the transposes go through LDS.  Both members of a pair {(p, q), (q, p)} are
+// the same two addends, so the output is exactly (anti)symmetric.
+//
+// M is odd, so a tile's 512-byte runs start at any multiple of 16 bytes and share
+// their first and last 128-byte lines with the next tiles along p.  Tiles go to
+// the XCDs (consecutive workgroups: round robin) in blocks of 4 x 4, so that most
+// shared lines meet in one L2.  Bound by HBM (32 bytes an entry): 4.7 TB/s at NN = 21
+// in FP64, 5.4 TB/s on complex64.  The form before, which read X and U = tau3D X
+// and rebuilt the potential here, moved 48 bytes an entry (1.0 ms a vector at
+// NN = 21 where this takes 0.58).
 constexpr int kSymT = 32;
+constexpr int kSymBlk = 4;
 
-template <typename R, typename XT, typename YT>
-__global__ __launch_bounds__(256) void k_symadd(ColPtrs xs, ColPtrs us, ColPtrsW ys, int64_t m, int nn,
-                                                const double *__restrict__ vn,
-                                                const double *__restrict__ tinv, MatvecCoef cf,
-                                                int sign) {
-  using C = typename Cplx<R>::type;
-  const int ta = blockIdx.x, tb = blockIdx.y;
-  if (ta > tb) return;
-  // column blockIdx.z of the launch
-  const XT *__restrict__ x = static_cast<const XT *>(xs.p[blockIdx.z]);
-  const C *__restrict__ u = static_cast<const C *>(us.p[blockIdx.z]);
-  YT *__restrict__ y = static_cast<YT *>(ys.p[blockIdx.z]);
-  __shared__ C su[kSymT][kSymT + 1], sx[kSymT][kSymT + 1];
-  __shared__ YT sy[kSymT][kSymT + 1];
+template <typename T>
+__global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, int sign) {
+  using R = typename Real<T>::type;
+  const int xcd = blockIdx.x % 8, s = blockIdx.x / 8;
+  const int blk = (s / (kSymBlk * kSymBlk)) * 8 + xcd, in = s % (kSymBlk * kSymBlk);
+  // block (ba, bb), ba <= bb, from its index bb (bb + 1) / 2 + ba
+  int bb = int((sqrtf(8.0f * float(blk) + 1.0f) - 1.0f) * 0.5f);
+  while (bb * (bb + 1) / 2 > blk) --bb;
+  while ((bb + 1) * (bb + 2) / 2 <= blk) ++bb;
+  const int ba = blk - bb * (bb + 1) / 2;
+  const int ta = ba * kSymBlk + in % kSymBlk, tb = bb * kSymBlk + in / kSymBlk;
+  if (bb >= nblk || ta > tb || tb * kSymT >= m) return;
+  T *__restrict__ y = static_cast<T *>(ys.p[blockIdx.y]);
+  __shared__ T s1[kSymT][kSymT + 1], s2[kSymT][kSymT + 1];
   const int tx = threadIdx.x, ty = threadIdx.y;
-  const int64_t pa = int64_t(ta) * kSymT, qb = int64_t(tb) * kSymT;
-  // mirror tile: su[r][c] = U[q + m p] with q = qb + c, p = pa + r
-  for (int r = ty; r < kSymT; r += 8) {
-    const int64_t q = qb + tx, p = pa + r;
-    if (q < m && p < m) {
-      su[r][tx] = u[q + m * p];
-      const XT xv = x[q + m * p];
-      C xc;
-      xc.x = R(xv.x);
-      xc.y = R(xv.y);
-      sx[r][tx] = xc;
-    }
+  const int pa = ta * kSymT, qb = tb * kSymT;
+  constexpr int PER = kSymT / 8;
+  T v1[PER], v2[PER];
+  const bool okp = pa + tx < m, okq = qb + tx < m, diag = ta == tb;
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int r = ty + 8 * u;
+    // main element (pa + tx, qb + r), mirror element (qb + tx, pa + r)
+    if (okp && qb + r < m) v1[u] = y[pa + tx + int64_t(m) * (qb + r)];
+    if (okq && pa + r < m) v2[u] = y[qb + tx + int64_t(m) * (pa + r)];
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    s1[ty + 8 * u][tx] = v1[u];
+    s2[ty + 8 * u][tx] = v2[u];
   }
   __syncthreads();
-  const int L = 2 * nn + 1;
-  const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(cf.c1_re), c1i = R(cf.c1_im);
   const R sg = R(sign);
-  const bool diag = ta == tb;
-  for (int r = ty; r < kSymT; r += 8) {
-    const int64_t p = pa + tx, q = qb + r;  // main element (p, q) at p + m q
-    if (p < m && q < m) {
-      const C uv = u[p + m * q];
-      const XT xv = x[p + m * q];
-      const C um = su[tx][r], xm = sx[tx][r];  // U[q + m p], X[q + m p]
-      const R sr = uv.x + sg * um.x, si = uv.y + sg * um.y;
-      const R xr = R(0.5) * (R(xv.x) + sg * xm.x), xi = R(0.5) * (R(xv.y) + sg * xm.y);
-      const int ip = int(p % nn), jp = int((p / nn) % nn), kp = int(p / (nn * nn));
-      const int iq = int(q % nn), jq = int((q / nn) % nn), kq = int(q / (nn * nn));
-      const int ti = (iq - ip + nn) + L * ((jq - jp + nn) + L * (kq - kp + nn));
-      const R vr = R(vn[p] + vn[q] + tinv[ti] * cf.inv_d3);
-      const R vxr = vr * xr, vxi = vr * xi;
-      YT o;
-      o.x = s2r * sr - s2i * si + c1r * vxr - c1i * vxi;
-      o.y = s2r * si + s2i * sr + c1r * vxi + c1i * vxr;
-      sy[tx][r] = o;
-      if (!diag || tx <= r) y[p + m * q] = o;
-    }
-  }
-  __syncthreads();
-  // mirror write: y[q + m p] = sign * Y(p, q), q = qb + tx, p = pa + r
-  for (int r = ty; r < kSymT; r += 8) {
-    const int64_t q = qb + tx, p = pa + r;
-    if (q < m && p < m && (!diag || r < tx)) {
-      const YT o = sy[r][tx];
-      YT w;
-      w.x = sg * o.x;
-      w.y = sg * o.y;
-      y[q + m * p] = w;
-    }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int r = ty + 8 * u;
+    const T m1 = s2[tx][r], m2 = s1[tx][r];
+    T o1, o2;
+    o1.x = v1[u].x + sg * m1.x;
+    o1.y = v1[u].y + sg * m1.y;
+    o2.x = v2[u].x + sg * m2.x;
+    o2.y = v2[u].y + sg * m2.y;
+    if (okp && qb + r < m) y[pa + tx + int64_t(m) * (qb + r)] = o1;
+    if (!diag && okq && pa + r < m) y[qb + tx + int64_t(m) * (pa + r)] = o2;
   }
 }
 
@@ -416,71 +382,48 @@ hipError_t matvec_generic_nn(const double2 *x, double2 *y, const double *vn, con
 // taking the lock themselves only if prepare_kernels() was never called).
 std::mutex g_setup_mu;
 
-// Workgroups of k_pass1<NN, R, XT> resident on the device at once (its
-// dynamic LDS attribute set on first use).  0 on a HIP error.
-template <int NN, typename R, typename XT>
-int pass1_setup() {
-  static std::atomic<int> resident_cached{0};
-  int resident = resident_cached.load(std::memory_order_acquire);
-  if (resident != 0) return resident;
+// Sets the dynamic LDS limit of one kernel (once: `done` is the kernel's flag).
+bool set_lds(const void *kernel, size_t lds, std::atomic<bool> &done) {
+  if (done.load(std::memory_order_acquire)) return true;
   std::lock_guard<std::mutex> lk(g_setup_mu);
-  resident = resident_cached.load(std::memory_order_acquire);
-  if (resident != 0) return resident;
-  constexpr int N3 = NN * NN * NN;
-  const size_t lds = size_t(2) * N3 * sizeof(R);
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pass1<NN, R, XT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
-    return 0;
-  int dev = 0, cus = 0, per = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void *>(&k_pass1<NN, R, XT>),
-                                                   cube_threads<NN>(), lds) != hipSuccess || per < 1)
-    per = 1;
-  resident = cus * per;
-  resident_cached.store(resident, std::memory_order_release);
-  return resident;
+  if (done.load(std::memory_order_acquire)) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) return false;
+  done.store(true, std::memory_order_release);
+  return true;
+}
+
+// LDS bytes of the passes' two cubes of reals.
+template <int NN, typename R>
+constexpr size_t cube_lds() {
+  return size_t(2) * NN * NN * NN * sizeof(R);
+}
+
+template <int NN, typename R, typename XT, typename ZT>
+bool pass1_setup() {
+  static std::atomic<bool> attr{false};
+  return set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT>), cube_lds<NN, R>(), attr);
 }
 
 template <int NN, typename R, typename XT, typename YT>
 bool pass2_setup() {
   static std::atomic<bool> attr{false};
-  if (attr.load(std::memory_order_acquire)) return true;
-  std::lock_guard<std::mutex> lk(g_setup_mu);
-  if (attr.load(std::memory_order_acquire)) return true;
-  constexpr int N3 = NN * NN * NN;
-  const size_t lds = size_t(2) * N3 * sizeof(R);
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pass2<NN, R, XT, YT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
-    return false;
-  attr.store(true, std::memory_order_release);
-  return true;
+  return set_lds(reinterpret_cast<const void *>(&k_pass2<NN, R, XT, YT>), cube_lds<NN, R>(), attr);
 }
 
-template <int NN, typename R, typename XT>
-hipError_t pass1_nn(const ColPtrs &xs, const ColPtrsW &us, int ncols, hipStream_t s) {
-  constexpr int N3 = NN * NN * NN;
-  const size_t lds = size_t(2) * N3 * sizeof(R);
-  // persistent grid: as many workgroups as fit on the device at once
-  const int resident = pass1_setup<NN, R, XT>();
-  if (resident == 0) return hipErrorInvalidDeviceFunction;
-  const int64_t total = int64_t(ncols) * N3;
-  const int grid = int(resident < total ? resident : total);
-  hipLaunchKernelGGL((k_pass1<NN, R, XT>), dim3(grid), dim3(cube_threads<NN>()), lds, s, xs, us, ncols);
+template <int NN, typename R, typename XT, typename ZT>
+hipError_t pass1_nn(const ColPtrs &xs, const ColPtrsW &zs, int ncols, const PotArgs &pot, double w, hipStream_t s) {
+  if (!pass1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
+  hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT>), dim3(NN * NN * NN, unsigned(ncols)), dim3(cube_threads<NN>()),
+                     (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv, pot.cf, w);
   return hipGetLastError();
 }
 
 template <int NN, typename R, typename XT, typename YT>
-hipError_t pass2_nn(const void *x, const void *u, void *y, const double *vn, const double *tinv,
-                    const MatvecCoef &cf, hipStream_t s) {
+hipError_t pass2_nn(const void *x, const void *z, void *y, const MatvecCoef &cf, hipStream_t s) {
   using C = typename Cplx<R>::type;
-  constexpr int N3 = NN * NN * NN;
-  const size_t lds = size_t(2) * N3 * sizeof(R);
   if (!pass2_setup<NN, R, XT, YT>()) return hipErrorInvalidDeviceFunction;
-  hipLaunchKernelGGL((k_pass2<NN, R, XT, YT>), dim3(N3), dim3(cube_threads<NN>()), lds, s,
-                     static_cast<const XT *>(x), static_cast<const C *>(u), static_cast<YT *>(y), vn,
-                     tinv, cf);
+  hipLaunchKernelGGL((k_pass2<NN, R, XT, YT>), dim3(NN * NN * NN), dim3(cube_threads<NN>()), (cube_lds<NN, R>()), s,
+                     static_cast<const XT *>(x), static_cast<const C *>(z), static_cast<YT *>(y), cf);
   return hipGetLastError();
 }
 
@@ -519,24 +462,27 @@ bool generic_matvec_supported(int nn) {
   }
 }
 
-hipError_t launch_pass1_batch(int nn, int io, const void *const *x, void *const *u, int ncols, hipStream_t s) {
+hipError_t launch_pass1(int nn, int io, bool sym, const void *const *x, void *const *z, int ncols,
+                        const PotArgs &pot, hipStream_t s) {
   if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
   ColPtrs xs{};
-  ColPtrsW us{};
+  ColPtrsW zs{};
   for (int j = 0; j < ncols; ++j) {
     xs.p[j] = x[j];
-    us.p[j] = u[j];
+    zs.p[j] = z[j];
   }
+  const double w = sym ? 0.5 : 1.0;
   switch (nn) {
-#define CASE(N)                                                                             \
-  case N:                                                                                   \
-    if constexpr (fast_fits(N, sizeof(double))) {                                           \
-      if (io == kIoF64) return pass1_nn<N, double, double2>(xs, us, ncols, s);              \
-    }                                                                                       \
-    if constexpr (fast_fits(N, sizeof(float))) {                                            \
-      if (io == kIoF32) return pass1_nn<N, float, float2>(xs, us, ncols, s);                \
-      if (io == kIoMixed) return pass1_nn<N, float, double2>(xs, us, ncols, s);             \
-    }                                                                                       \
+#define CASE(N)                                                                                         \
+  case N:                                                                                               \
+    if constexpr (fast_fits(N, sizeof(double))) {                                                       \
+      if (io == kIoF64) return pass1_nn<N, double, double2, double2>(xs, zs, ncols, pot, w, s);         \
+    }                                                                                                   \
+    if constexpr (fast_fits(N, sizeof(float))) {                                                        \
+      if (io == kIoF32) return pass1_nn<N, float, float2, float2>(xs, zs, ncols, pot, w, s);            \
+      if (io == kIoMixed && sym) return pass1_nn<N, float, double2, double2>(xs, zs, ncols, pot, w, s); \
+      if (io == kIoMixed) return pass1_nn<N, float, double2, float2>(xs, zs, ncols, pot, w, s);         \
+    }                                                                                                   \
     return hipErrorInvalidValue;
     DEX_NN_LIST(CASE)
 #undef CASE
@@ -545,60 +491,39 @@ hipError_t launch_pass1_batch(int nn, int io, const void *const *x, void *const 
   }
 }
 
-hipError_t launch_pass1(int nn, int io, const void *x, void *u, hipStream_t s) {
-  return launch_pass1_batch(nn, io, &x, &u, 1, s);
-}
-
-hipError_t launch_pass2(int nn, int io, const void *x, const void *u, void *y,
-                        const double *vn, const double *tinv, const MatvecCoef &coef,
-                        hipStream_t s) {
-  switch (nn) {
-#define CASE(N)                                                                                   \
-  case N:                                                                                         \
-    if constexpr (fast_fits(N, sizeof(double))) {                                                 \
-      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, u, y, vn, tinv, coef, s); \
-    }                                                                                             \
-    if constexpr (fast_fits(N, sizeof(float))) {                                                  \
-      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, u, y, vn, tinv, coef, s);    \
-      if (io == kIoMixed) return pass2_nn<N, float, double2, double2>(x, u, y, vn, tinv, coef, s); \
-    }                                                                                             \
-    return hipErrorInvalidValue;
-    DEX_NN_LIST(CASE)
-#undef CASE
-    default:
-      return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_symadd_batch(int nn, int io, const void *const *x, const void *const *u, void *const *y,
-                               int ncols, const double *vn, const double *tinv, const MatvecCoef &coef,
-                               int sign, hipStream_t s) {
+hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, hipStream_t s) {
   if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
-  ColPtrs xs{}, us{};
   ColPtrsW ys{};
-  for (int j = 0; j < ncols; ++j) {
-    xs.p[j] = x[j];
-    us.p[j] = u[j];
-    ys.p[j] = y[j];
-  }
-  const int64_t m = int64_t(nn) * nn * nn;
-  const unsigned nt = unsigned((m + kSymT - 1) / kSymT);
-  const dim3 g(nt, nt, unsigned(ncols)), b(kSymT, 8);
-  if (io == kIoF32) {
-    hipLaunchKernelGGL((k_symadd<float, float2, float2>), g, b, 0, s, xs, us, ys, m, nn, vn, tinv, coef, sign);
-  } else if (io == kIoMixed) {
-    hipLaunchKernelGGL((k_symadd<float, double2, double2>), g, b, 0, s, xs, us, ys, m, nn, vn, tinv, coef, sign);
-  } else {
-    hipLaunchKernelGGL((k_symadd<double, double2, double2>), g, b, 0, s, xs, us, ys, m, nn, vn, tinv, coef,
-                       sign);
-  }
+  for (int j = 0; j < ncols; ++j) ys.p[j] = y[j];
+  const int m = nn * nn * nn;
+  const int nt = (m + kSymT - 1) / kSymT, nblk = (nt + kSymBlk - 1) / kSymBlk;
+  const int pairs = nblk * (nblk + 1) / 2;
+  const dim3 g(unsigned(round_up(pairs, 8) * kSymBlk * kSymBlk), unsigned(ncols)), b(kSymT, 8);
+  if (io == kIoF32)
+    hipLaunchKernelGGL((k_symfold<float2>), g, b, 0, s, ys, m, nblk, sign);
+  else
+    hipLaunchKernelGGL((k_symfold<double2>), g, b, 0, s, ys, m, nblk, sign);
   return hipGetLastError();
 }
 
-hipError_t launch_symadd(int nn, int io, const void *x, const void *u, void *y,
-                         const double *vn, const double *tinv, const MatvecCoef &coef, int sign,
-                         hipStream_t s) {
-  return launch_symadd_batch(nn, io, &x, &u, &y, 1, vn, tinv, coef, sign, s);
+hipError_t launch_pass2(int nn, int io, const void *x, const void *z, void *y, const MatvecCoef &coef,
+                        hipStream_t s) {
+  switch (nn) {
+#define CASE(N)                                                                                 \
+  case N:                                                                                       \
+    if constexpr (fast_fits(N, sizeof(double))) {                                               \
+      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, z, y, coef, s);         \
+    }                                                                                           \
+    if constexpr (fast_fits(N, sizeof(float))) {                                                \
+      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, coef, s);            \
+      if (io == kIoMixed) return pass2_nn<N, float, double2, double2>(x, z, y, coef, s);        \
+    }                                                                                           \
+    return hipErrorInvalidValue;
+    DEX_NN_LIST(CASE)
+#undef CASE
+    default:
+      return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_matvec_generic(int nn, const Dbl2 *x, Dbl2 *y, const double *vn,
@@ -1945,11 +1870,12 @@ template <int NN>
 bool prepare_nn() {
   bool ok = true;
   if constexpr (fast_fits(NN, sizeof(double))) {
-    ok = ok && pass1_setup<NN, double, double2>() != 0;
+    ok = ok && pass1_setup<NN, double, double2, double2>();
     ok = ok && pass2_setup<NN, double, double2, double2>();
   }
   if constexpr (fast_fits(NN, sizeof(float))) {
-    ok = ok && pass1_setup<NN, float, float2>() != 0 && pass1_setup<NN, float, double2>() != 0;
+    ok = ok && pass1_setup<NN, float, float2, float2>() && pass1_setup<NN, float, double2, double2>();
+    ok = ok && pass1_setup<NN, float, double2, float2>();
     ok = ok && pass2_setup<NN, float, float2, float2>() && pass2_setup<NN, float, double2, double2>();
   }
   return ok;

@@ -104,13 +104,12 @@ int dex_matvec_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
 /* HAMMULT for exchange-(anti)symmetric vectors, X(P,Q) = symmetry * X(Q,P)
  * (symmetry = +1 singlet, -1 triplet; 0 is dex_matvec_device).  Electron 2's
  * kinetic term is then the transpose of electron 1's, so the second pass is a
- * coalesced transpose-add; the result is Y = H Xs with Xs = (X + symmetry X^T)/2,
- * exactly (anti)symmetric.  This is how the reference's start vectors enter
+ * coalesced transpose-add in Y's own storage; the result is Y = H Xs with
+ * Xs = (X + symmetry X^T)/2, exactly (anti)symmetric.  This is how the reference's start vectors enter
  * (HELIUM_ORBITAL with SIGN = +-1, hammod.F90:1059-1063); HAMMULT itself has
  * no such mode.  Needs the LDS kernels for the grid (dex_info.fast_path).
- * With howmany >= 2 on complex128 columns (and kernel timing off) the columns
- * go through the passes in batches of up to 16 per launch, where the grid is
- * small enough for their intermediates to fit in 512 MiB (NN <= 15). */
+ * With howmany >= 2 (and kernel timing off) the columns go through the passes in
+ * even batches of up to 16 per launch on small grids, 4 on large ones. */
 int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
                           int64_t checksize, int32_t single, int32_t symmetry);
 
@@ -118,11 +117,11 @@ int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howma
  * reference; for callers that cannot allocate (code under HIP graph capture,
  * serving loops that forbid it).  The intermediate U lives in a static 64 MiB
  * device array that the library holds on every GPU it runs on until the
- * process ends, so the LDS kernels' grids are limited to NN <= 11 in an FP64
+ * process ends (exchange-symmetric calls keep to the same limits), so the LDS kernels' grids are limited to NN <= 11 in an FP64
  * context and NN <= 13 in an FP32 one (larger: DEX_ESIZE); FP64 grids without
  * the LDS kernels (NN >= 23) use the six-pass kernels, which need no scratch.
- * Columns go one at a time (no batched launches) and no kernel timing is
- * recorded.  Calls that overlap on one GPU share the array and race: order them
+ * General columns go one at a time, exchange-symmetric ones in batches as above;
+ * no kernel timing is recorded.  Calls that overlap on one GPU share the array and race: order them
  * on one stream or serialise them.  U needs no clearing (each column's first
  * pass writes all of it). */
 int dex_matvec_noalloc(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
