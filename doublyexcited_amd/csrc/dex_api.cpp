@@ -353,19 +353,26 @@ int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int nc
   const double xb = io == dex::kIoF32 ? 8.0 : 16.0;               // X and Y entry bytes
   const double zb = sym != 0 ? xb : (io == dex::kIoF64 ? 16.0 : 8.0);  // Z entry bytes
   const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  const bool planes = sym == 0 && dex::general_by_planes(c->nn);
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[0], c->stream));
   {
-    // reads X, writes Z; three axes of NN real-by-complex MACs an entry and the potential
-    KTimer kt(c, DEX_K_PASS1, (xb + zb) * dd, (12.0 * nn + 16.0) * dd);
-    DEX_HIP(dex::launch_pass1(c->nn, io, sym != 0, x, sym != 0 ? y : &u, ncols, pot, c->stream));
+    // reads X, writes Z; three axes (two by planes) of NN real-by-complex MACs an
+    // entry and the potential
+    KTimer kt(c, DEX_K_PASS1, (xb + zb) * dd, ((planes ? 8.0 : 12.0) * nn + 16.0) * dd);
+    if (sym != 0)
+      DEX_HIP(dex::launch_pass1(c->nn, io, true, x, y, ncols, pot, c->stream));
+    else
+      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], u, pot, c->stream));
   }
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[1], c->stream));
   if (sym != 0) {
     KTimer kt(c, DEX_K_SYMADD, 2.0 * xb * dd, 2.0 * dd);
     DEX_HIP(dex::launch_symfold(c->nn, io, y, ncols, sym, c->stream));
   } else {
-    KTimer kt(c, DEX_K_PASS2, (2.0 * xb + zb) * dd, (12.0 * nn + 8.0) * dd);
-    DEX_HIP(dex::launch_pass2(c->nn, io, x[0], u, y[0], c->coef, c->stream));
+    // reads X and Z, writes Y; by planes two launches, the first writing Z again
+    KTimer kt(c, DEX_K_PASS2, (2.0 * xb + zb + (planes ? xb + 2.0 * zb : 0.0)) * dd,
+              ((planes ? 16.0 : 12.0) * nn + 8.0) * dd);
+    DEX_HIP(dex::launch_general_second(c->nn, io, x[0], u, y[0], c->coef, c->stream));
   }
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[2], c->stream));
   return 0;
@@ -379,6 +386,14 @@ int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, i
     k = batch_cols(c, io, ncols - j);
     if (int st = fast_passes(c, io, x + j, y + j, k, sym, nullptr)) return st;
   }
+  return 0;
+}
+
+// H on one complex128 column in FP64 with the intermediate in Y's own storage
+// (grids without an FP64 cube; x and y must differ).
+int generic_passes(dex_ctx *c, const void *x, void *y) {
+  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, {c->d_vn, c->d_tinv, c->coef}, c->stream));
+  DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, c->coef, c->stream));
   return 0;
 }
 
@@ -396,7 +411,7 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
                        pass_events && c->timing);
   }
   KTimer kt(c, DEX_K_GENERIC, 32.0 * double(c->d), (24.0 * c->nn + 14.0) * double(c->d));
-  DEX_HIP(dex::launch_matvec_generic(c->nn, x, y, c->d_vn, c->d_tinv, c->coef, c->stream));
+  if (int st = generic_passes(c, x, y)) return st;
   // The general operator carries the rounding-level exchange-odd (even) part of
   // an exchange-even (odd) x into y, where the transpose-add kernels, which the
   // mixed form applies to its complex64 blocks, drop it: in a solve that mixes
@@ -754,7 +769,7 @@ int dex_ctx_create(const dex_params *p, dex_ctx **out) {
   c->coef.inv_d3 = 1.0 / (p->delta * p->delta * p->delta);
   c->fast64 = dex::fast_matvec_supported(nn, false);
   c->fast32 = dex::fast_matvec_supported(nn, true);
-  // DEX_MATVEC=generic selects the six-pass FP64 kernels even where the LDS
+  // DEX_MATVEC=generic takes the grids without an FP64 cube's route even where the LDS
   // two-pass kernels exist (used to cross-check the two implementations).
   if (const char *mv = std::getenv("DEX_MATVEC"))
     if (std::strcmp(mv, "generic") == 0) c->fast64 = false;
@@ -991,15 +1006,14 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
       y[i] = static_cast<char *>(out) + size_t(j + i) * size_t(c->d) * xb;
     }
     if (!fast) {
-      DEX_HIP(dex::launch_matvec_generic(c->nn, static_cast<const Dbl2 *>(x[0]), static_cast<Dbl2 *>(y[0]), c->d_vn,
-                                         c->d_tinv, c->coef, c->stream));
+      if (int st = generic_passes(c, x[0], y[0])) return st;
     } else if (symmetry != 0) {
       DEX_HIP(dex::launch_pass1(c->nn, io, true, x, y, k, pot, c->stream));
       DEX_HIP(dex::launch_symfold(c->nn, io, y, k, symmetry, c->stream));
     } else {
       // Z (fully written by the electron-1 pass before the second pass reads it)
-      DEX_HIP(dex::launch_pass1(c->nn, io, false, x, &c->d_scratch, 1, pot, c->stream));
-      DEX_HIP(dex::launch_pass2(c->nn, io, x[0], c->d_scratch, y[0], c->coef, c->stream));
+      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], c->d_scratch, pot, c->stream));
+      DEX_HIP(dex::launch_general_second(c->nn, io, x[0], c->d_scratch, y[0], c->coef, c->stream));
     }
   }
   return DEX_OK;

@@ -90,15 +90,15 @@ struct PotArgs {
 // complex64 otherwise).
 hipError_t launch_pass1(int nn, int io, bool sym, const void *const *x, void *const *z, int ncols,
                         const PotArgs &pot, hipStream_t s);
-// Second pass for general vectors: Y = Z + s2 K2 X.
-hipError_t launch_pass2(int nn, int io, const void *x, const void *z, void *y, const MatvecCoef &coef,
-                        hipStream_t s);
+// General vectors, one column, any grid: the first launch and the rest (z: D
+// entries of the arithmetic's format; x and y may be one array where z is another,
+// z and y where x is another).
+bool general_by_planes(int nn);
+hipError_t launch_general_first(int nn, int io, const void *x, void *z, const PotArgs &pot, hipStream_t s);
+hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, const MatvecCoef &coef,
+                                 hipStream_t s);
 // Second pass for X = sign X^T, in place on ncols columns: Y <- Y + sign Y^T.
 hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, hipStream_t s);
-// Generic FP64 path for any odd nn <= 27: six axis passes plus the potential.
-hipError_t launch_matvec_generic(int nn, const Dbl2 *x, Dbl2 *y, const double *vn,
-                                 const double *tinv, const MatvecCoef &coef, hipStream_t s);
-
 // G(kl x kr, column-major) = L^H R summed over d rows, kl <= 64, kr <= 128.
 // The first `share` columns of R are the L columns themselves (share <= kl);
 // `descs` holds kl L descriptors then kr - share R descriptors.  With

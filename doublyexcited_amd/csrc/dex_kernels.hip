@@ -13,8 +13,8 @@
 //     cubes in LDS),
 //   exchange-(anti)symmetric vectors (w = 1/2): Y = Z + sign Z^T, in place,
 //   general ones (w = 1): Y[p, :] = Z[p, :] + s2 tau3D X[p, :]  (cubes at stride
-//     M; neighbouring p share cache lines, so the workgroup -> p map keeps groups
-//     of 8 consecutive p on one XCD).
+//     M) on the smallest grids; on the others three passes of two axes each
+//     (k_plane1, k_plane2) replace both.
 // The kinetic operator is real, so the real and imaginary parts are contracted
 // in turn through two LDS buffers of NN^3 reals each (148 KB at NN = 21 in FP64).
 #include <atomic>
@@ -310,69 +310,142 @@ __global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, i
   }
 }
 
-// ---- generic FP64 path ------------------------------------------------------
-// One thread per line of the given axis (stride s): y (+)= tau * x along it.
+// ---- two axes at a time --------------------------------------------------------
+// General vectors in three passes of two axes each, for grids whose cube does not
+// fit the LDS (FP64 at NN >= 23) and for those where the stride-M cubes of k_pass2
+// cost more than a third pass: every access runs along a contiguous direction.
+// A workgroup holds NN x NN lines of kPlaneRun entries: each thread keeps one line
+// of the first axis in registers (contracted there), the second axis goes through
+// the LDS buffers a (entries) and b (its sums), one real component at a time.
+// 32 + 48 + 48 bytes an entry over the three passes, 4.0 TB/s of them at NN = 25 in
+// FP64 (7.8 ms a vector; six passes of one axis and the potential's took 16.8), with
+// 8 waves a CU in flight (two workgroups: 80 KB of LDS, 205-240 registers).
+template <typename XT>
+constexpr int plane_run() {
+  return int(128 / sizeof(XT));  // entries of a 128-byte run
+}
 template <int NN>
-__global__ __launch_bounds__(256) void k_axis(const double2 *__restrict__ x, double2 *__restrict__ y,
-                                              int64_t stride, int64_t nlines, int accumulate) {
-  const int64_t line = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (line >= nlines) return;
-  const int64_t off = (line % stride) + (line / stride) * stride * NN;
-  double2 xv[NN];
+constexpr int plane1_planes() {
+  return NN >= 9 ? 8 : 16;  // i1 x j1 planes of a workgroup
+}
+
+// Axes i1 and j1 and the potential: Z = s2 (tau x 1 + 1 x tau) X + w c1 Vr o X.
+// blockIdx: electron-2 index q, group of kp = plane1_planes() planes k1.  Thread (i, g) keeps the
+// j line of plane g.
+template <int NN, typename R, typename XT, typename ZT>
+__global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane1(
+    const XT *__restrict__ x, ZT *__restrict__ z, const double *__restrict__ vn, const double *__restrict__ tinv,
+    MatvecCoef cf) {
+  constexpr int N2 = NN * NN, N3 = NN * N2, L = 2 * NN + 1, G = plane1_planes<NN>();
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int i = threadIdx.x % NN, g = threadIdx.x / NN, k = int(blockIdx.y) * G + g;
+  const bool on = g < G && k < NN;
+  R *a = reinterpret_cast<R *>(smem) + g * N2;
+  R *b = a + G * N2;
+  const int q = blockIdx.x;
+  const int64_t base = int64_t(q) * N3 + N2 * k + i;
+  R xr[NN], xi[NN], kr[NN];
+  if (on) {
 #pragma unroll
-  for (int l = 0; l < NN; ++l) xv[l] = x[off + stride * l];
+    for (int j = 0; j < NN; ++j) {
+      const XT v = x[base + NN * j];
+      xr[j] = R(v.x);
+      xi[j] = R(v.y);
+    }
+  }
+  // i lines of one component through LDS, thread (line j = i, plane g)
+  auto i_axis = [&](const R(&v)[NN]) {
+    if (on) {
 #pragma unroll
-  for (int i = 0; i < NN; ++i) {
-    double ar = 0.0, ai = 0.0;
+      for (int j = 0; j < NN; ++j) a[NN * j + i] = v[j];
+    }
+    __syncthreads();
+    if (on) {
+      R t[NN];
+#pragma unroll
+      for (int l = 0; l < NN; ++l) t[l] = a[NN * i + l];
+      line_apply<NN, R>(t, [&](int l, R y) { b[NN * i + l] = y; });
+    }
+    __syncthreads();
+  };
+  i_axis(xr);
+  if (on) line_apply<NN, R>(xr, [&](int j, R y) { kr[j] = y + b[NN * j + i]; });
+  i_axis(xi);
+  if (on) {
+    const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(cf.c1_re), c1i = R(cf.c1_im);
+    const int iq = q % NN, jq = (q / NN) % NN, kq = q / N2;
+    const int t0 = (iq - i + NN) + L * ((jq + NN) + L * (kq - k + NN));
+    const double vq = vn[q];
+    line_apply<NN, R>(xi, [&](int j, R y) {
+      const R ki = y + b[NN * j + i];
+      const R vr = R(vn[N2 * k + NN * j + i] + vq + tinv[t0 - L * j] * cf.inv_d3);
+      const R vxr = vr * xr[j], vxi = vr * xi[j];
+      ZT o;
+      o.x = s2r * kr[j] - s2i * ki + c1r * vxr - c1i * vxi;
+      o.y = s2r * ki + s2i * kr[j] + c1r * vxi + c1i * vxr;
+      z[base + NN * j] = o;
+    });
+  }
+}
+
+// Two more axes a, b at strides sa, sb: Y = Z + s2 (tau x 1 + 1 x tau) X on
+// entries base + r + sa a + sb b, r < run.  A workgroup takes a run tile of
+// blockIdx.x and the outer index blockIdx.y (stride so); thread (r, b) keeps the a
+// line.  It reads its entries of X and Z before it writes them, so Y may be either.
+// Runs start at any multiple of an entry (M is odd) and share lines with their
+// neighbours: consecutive tiles go to one XCD (workgroups are dealt to the 8 XCDs
+// in turn).
+template <int NN, typename R, typename XT, typename ZT, typename YT>
+__global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(const XT *x, const ZT *z, YT *y,
+                                                                             int64_t run, int64_t sa, int64_t sb,
+                                                                             int64_t so, int64_t per_xcd,
+                                                                             MatvecCoef cf) {
+  constexpr int P = plane_run<XT>(), N2 = NN * NN;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int r = threadIdx.x % P, bb = threadIdx.x / P;
+  const int64_t r0 = ((blockIdx.x % 8) * per_xcd + blockIdx.x / 8) * P;
+  const bool on = bb < NN && r0 + r < run;
+  const int64_t base = r0 + r + so * blockIdx.y + sb * bb;
+  R *a = reinterpret_cast<R *>(smem) + r;
+  R *b = a + N2 * P;
+  R xr[NN], xi[NN], kr[NN];
+  if (on) {
 #pragma unroll
     for (int l = 0; l < NN; ++l) {
-      const double t = tau_rt(l - i);
-      ar += t * xv[l].x;
-      ai += t * xv[l].y;
+      const XT v = x[base + sa * l];
+      xr[l] = R(v.x);
+      xi[l] = R(v.y);
     }
-    double2 o = accumulate ? y[off + stride * i] : make_double2(0.0, 0.0);
-    o.x += ar;
-    o.y += ai;
-    y[off + stride * i] = o;
   }
-}
-
-__global__ void k_potential(const double2 *__restrict__ x, double2 *__restrict__ y,
-                            const double *__restrict__ vn, const double *__restrict__ tinv, int nn,
-                            int64_t m, MatvecCoef cf) {
-  const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= m * m) return;
-  const int64_t p = idx % m, q = idx / m;
-  const int L = 2 * nn + 1;
-  const int ip = int(p % nn), jp = int((p / nn) % nn), kp = int(p / (int64_t(nn) * nn));
-  const int iq = int(q % nn), jq = int((q / nn) % nn), kq = int(q / (int64_t(nn) * nn));
-  const int64_t ti = (iq - ip + nn) + int64_t(L) * ((jq - jp + nn) + int64_t(L) * (kq - kp + nn));
-  const double vr = vn[p] + vn[q] + tinv[ti] * cf.inv_d3;
-  const double2 xv = x[idx];
-  const double2 kv = y[idx];
-  double2 o;
-  o.x = cf.s2_re * kv.x - cf.s2_im * kv.y + vr * (cf.c1_re * xv.x - cf.c1_im * xv.y);
-  o.y = cf.s2_re * kv.y + cf.s2_im * kv.x + vr * (cf.c1_re * xv.y + cf.c1_im * xv.x);
-  y[idx] = o;
-}
-
-template <int NN>
-hipError_t matvec_generic_nn(const double2 *x, double2 *y, const double *vn, const double *tinv,
-                             const MatvecCoef &cf, hipStream_t s) {
-  const int64_t m = int64_t(NN) * NN * NN;
-  const int64_t d = m * m;
-  const int64_t nlines = d / NN;
-  const int bs = 256;
-  const int64_t nb = (nlines + bs - 1) / bs;
-  int64_t stride = 1;
-  for (int axis = 0; axis < 6; ++axis) {
-    hipLaunchKernelGGL(k_axis<NN>, dim3(unsigned(nb)), dim3(bs), 0, s, x, y, stride, nlines,
-                       axis == 0 ? 0 : 1);
-    stride *= NN;
+  // b lines of one component through LDS, thread (r, line a = bb)
+  auto b_axis = [&](const R(&v)[NN]) {
+    if (on) {
+#pragma unroll
+      for (int l = 0; l < NN; ++l) a[(l * NN + bb) * P] = v[l];
+    }
+    __syncthreads();
+    if (on) {
+      R t[NN];
+#pragma unroll
+      for (int l = 0; l < NN; ++l) t[l] = a[(bb * NN + l) * P];
+      line_apply<NN, R>(t, [&](int l, R s) { b[(bb * NN + l) * P] = s; });
+    }
+    __syncthreads();
+  };
+  b_axis(xr);
+  if (on) line_apply<NN, R>(xr, [&](int l, R s) { kr[l] = s + b[(l * NN + bb) * P]; });
+  b_axis(xi);
+  if (on) {
+    const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
+    line_apply<NN, R>(xi, [&](int l, R s) {
+      const R ki = s + b[(l * NN + bb) * P];
+      const ZT zv = z[base + sa * l];
+      YT o;
+      o.x = zv.x + (s2r * kr[l] - s2i * ki);
+      o.y = zv.y + (s2r * ki + s2i * kr[l]);
+      y[base + sa * l] = o;
+    });
   }
-  const int64_t nb2 = (d + bs - 1) / bs;
-  hipLaunchKernelGGL(k_potential, dim3(unsigned(nb2)), dim3(bs), 0, s, x, y, vn, tinv, NN, m, cf);
-  return hipGetLastError();
 }
 
 // Function attributes and occupancy figures are set once per kernel, under
@@ -427,6 +500,56 @@ hipError_t pass2_nn(const void *x, const void *z, void *y, const MatvecCoef &cf,
   return hipGetLastError();
 }
 
+template <int NN, typename R>
+constexpr size_t plane1_lds() {
+  return size_t(2) * plane1_planes<NN>() * NN * NN * sizeof(R);
+}
+template <int NN, typename R, typename XT>
+constexpr size_t plane2_lds() {
+  return size_t(2) * plane_run<XT>() * NN * NN * sizeof(R);
+}
+
+template <int NN, typename R, typename XT, typename ZT>
+bool plane1_setup() {
+  static std::atomic<bool> attr{false};
+  return set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT>), plane1_lds<NN, R>(), attr);
+}
+
+template <int NN, typename R, typename XT, typename ZT, typename YT>
+bool plane2_setup() {
+  static std::atomic<bool> first{false}, second{false};
+  return set_lds(reinterpret_cast<const void *>(&k_plane2<NN, R, XT, ZT, ZT>), plane2_lds<NN, R, XT>(), first) &&
+         set_lds(reinterpret_cast<const void *>(&k_plane2<NN, R, XT, ZT, YT>), plane2_lds<NN, R, XT>(), second);
+}
+
+template <int NN, typename R, typename XT, typename ZT>
+hipError_t plane1_nn(const void *x, void *z, const PotArgs &pot, hipStream_t s) {
+  if (!plane1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
+  constexpr int G = plane1_planes<NN>();
+  hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT>), dim3(NN * NN * NN, (NN + G - 1) / G), dim3(round_up(NN * G, 64)),
+                     (plane1_lds<NN, R>()), s, static_cast<const XT *>(x), static_cast<ZT *>(z), pot.vn, pot.tinv,
+                     pot.cf);
+  return hipGetLastError();
+}
+
+template <int NN, typename R, typename XT, typename ZT, typename YT>
+hipError_t plane2_nn(const void *x, void *z, void *y, const MatvecCoef &cf, hipStream_t s) {
+  if (!plane2_setup<NN, R, XT, ZT, YT>()) return hipErrorInvalidDeviceFunction;
+  constexpr int64_t N2 = NN * NN, N3 = NN * N2, N4 = NN * N3;
+  constexpr int P = plane_run<XT>();
+  const XT *xx = static_cast<const XT *>(x);
+  ZT *zz = static_cast<ZT *>(z);
+  auto per_xcd = [](int64_t run) { return ((run + P - 1) / P + 7) / 8; };  // run tiles an XCD takes
+  // k1 and i2, runs along (i1, j1); then j2 and k2, runs along (i1, j1, k1, i2)
+  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, ZT>), dim3(unsigned(8 * per_xcd(N2)), unsigned(N2)),
+                     dim3(round_up(NN * P, 64)), (plane2_lds<NN, R, XT>()), s, xx, static_cast<const ZT *>(zz), zz, N2,
+                     N2, N3, N4, per_xcd(N2), cf);
+  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, YT>), dim3(unsigned(8 * per_xcd(N4))), dim3(round_up(NN * P, 64)),
+                     (plane2_lds<NN, R, XT>()), s, xx, static_cast<const ZT *>(zz), static_cast<YT *>(y), N4, N4,
+                     N4 * NN, int64_t(0), per_xcd(N4), cf);
+  return hipGetLastError();
+}
+
 // LDS budget per workgroup on gfx950.
 constexpr size_t kMaxLds = 160 * 1024;
 
@@ -435,6 +558,9 @@ constexpr bool fast_fits(int nn, size_t rsize) {
 }
 
 }  // namespace
+
+// Largest grid whose general vectors go through the cubes (launch_general_first).
+constexpr int kCubeMaxNN = 11;
 
 #define DEX_NN_LIST(X) X(3) X(5) X(7) X(9) X(11) X(13) X(15) X(17) X(19) X(21) X(23) X(25)
 
@@ -481,6 +607,8 @@ hipError_t launch_pass1(int nn, int io, bool sym, const void *const *x, void *co
     if constexpr (fast_fits(N, sizeof(float))) {                                                        \
       if (io == kIoF32) return pass1_nn<N, float, float2, float2>(xs, zs, ncols, pot, w, s);            \
       if (io == kIoMixed && sym) return pass1_nn<N, float, double2, double2>(xs, zs, ncols, pot, w, s); \
+    }                                                                                                   \
+    if constexpr (N <= kCubeMaxNN) {                                                                    \
       if (io == kIoMixed) return pass1_nn<N, float, double2, float2>(xs, zs, ncols, pot, w, s);         \
     }                                                                                                   \
     return hipErrorInvalidValue;
@@ -506,18 +634,24 @@ hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, h
   return hipGetLastError();
 }
 
-hipError_t launch_pass2(int nn, int io, const void *x, const void *z, void *y, const MatvecCoef &coef,
-                        hipStream_t s) {
+// General vectors go through the cubes (k_pass1, k_pass2) on the smallest grids and
+// through the planes beyond: k_pass2's stride-M reads take 16 (8) bytes of each
+// 128-byte line, and the neighbours that share it find it in L2 less and less
+// often (3.3 times the bytes from HBM at NN = 13).  Microseconds a vector, cubes
+// and planes: NN = 11 FP64 68 and 69; 13: 165 and 135; 17: 997 and 745; 21: 3270 and
+// 2850; complex64 at 17: 833 and 455; at 25: 7035 and 4300.
+bool general_by_planes(int nn) { return nn > kCubeMaxNN; }
+
+hipError_t launch_general_first(int nn, int io, const void *x, void *z, const PotArgs &pot, hipStream_t s) {
+  if (!general_by_planes(nn)) return launch_pass1(nn, io, false, &x, &z, 1, pot, s);
   switch (nn) {
-#define CASE(N)                                                                                 \
-  case N:                                                                                       \
-    if constexpr (fast_fits(N, sizeof(double))) {                                               \
-      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, z, y, coef, s);         \
-    }                                                                                           \
-    if constexpr (fast_fits(N, sizeof(float))) {                                                \
-      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, coef, s);            \
-      if (io == kIoMixed) return pass2_nn<N, float, double2, double2>(x, z, y, coef, s);        \
-    }                                                                                           \
+#define CASE(N)                                                                           \
+  case N:                                                                                 \
+    if constexpr (N > kCubeMaxNN) {                                                       \
+      if (io == kIoF64) return plane1_nn<N, double, double2, double2>(x, z, pot, s);      \
+      if (io == kIoF32) return plane1_nn<N, float, float2, float2>(x, z, pot, s);         \
+      return plane1_nn<N, float, double2, float2>(x, z, pot, s);                          \
+    }                                                                                     \
     return hipErrorInvalidValue;
     DEX_NN_LIST(CASE)
 #undef CASE
@@ -526,14 +660,20 @@ hipError_t launch_pass2(int nn, int io, const void *x, const void *z, void *y, c
   }
 }
 
-hipError_t launch_matvec_generic(int nn, const Dbl2 *x, Dbl2 *y, const double *vn,
-                                 const double *tinv, const MatvecCoef &coef, hipStream_t s) {
-  const double2 *xx = reinterpret_cast<const double2 *>(x);
-  double2 *yy = reinterpret_cast<double2 *>(y);
+hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, const MatvecCoef &coef,
+                                 hipStream_t s) {
   switch (nn) {
-#define CASE(N) \
-  case N:       \
-    return matvec_generic_nn<N>(xx, yy, vn, tinv, coef, s);
+#define CASE(N)                                                                                       \
+  case N:                                                                                             \
+    if constexpr (N > kCubeMaxNN) {                                                                   \
+      if (io == kIoF64) return plane2_nn<N, double, double2, double2, double2>(x, z, y, coef, s);     \
+      if (io == kIoF32) return plane2_nn<N, float, float2, float2, float2>(x, z, y, coef, s);         \
+      return plane2_nn<N, float, double2, float2, double2>(x, z, y, coef, s);                         \
+    } else {                                                                                          \
+      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, z, y, coef, s);               \
+      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, coef, s);                  \
+      return pass2_nn<N, float, double2, double2>(x, z, y, coef, s);                                  \
+    }
     DEX_NN_LIST(CASE)
 #undef CASE
     default:
@@ -1869,14 +2009,18 @@ namespace {
 template <int NN>
 bool prepare_nn() {
   bool ok = true;
-  if constexpr (fast_fits(NN, sizeof(double))) {
-    ok = ok && pass1_setup<NN, double, double2, double2>();
-    ok = ok && pass2_setup<NN, double, double2, double2>();
-  }
-  if constexpr (fast_fits(NN, sizeof(float))) {
+  if constexpr (fast_fits(NN, sizeof(double))) ok = ok && pass1_setup<NN, double, double2, double2>();
+  if constexpr (fast_fits(NN, sizeof(float)))
     ok = ok && pass1_setup<NN, float, float2, float2>() && pass1_setup<NN, float, double2, double2>();
+  if constexpr (NN > kCubeMaxNN) {
+    ok = ok && plane1_setup<NN, double, double2, double2>() && plane1_setup<NN, float, float2, float2>() &&
+         plane1_setup<NN, float, double2, float2>();
+    ok = ok && plane2_setup<NN, double, double2, double2, double2>() &&
+         plane2_setup<NN, float, float2, float2, float2>() && plane2_setup<NN, float, double2, float2, double2>();
+  } else {
     ok = ok && pass1_setup<NN, float, double2, float2>();
-    ok = ok && pass2_setup<NN, float, float2, float2>() && pass2_setup<NN, float, double2, double2>();
+    ok = ok && pass2_setup<NN, double, double2, double2>() && pass2_setup<NN, float, float2, float2>() &&
+         pass2_setup<NN, float, double2, double2>();
   }
   return ok;
 }

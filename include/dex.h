@@ -105,9 +105,9 @@ int dex_matvec_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
  * (symmetry = +1 singlet, -1 triplet; 0 is dex_matvec_device).  Electron 2's
  * kinetic term is then the transpose of electron 1's, so the second pass is a
  * coalesced transpose-add in Y's own storage; the result is Y = H Xs with
- * Xs = (X + symmetry X^T)/2, exactly (anti)symmetric.  This is how the reference's start vectors enter
- * (HELIUM_ORBITAL with SIGN = +-1, hammod.F90:1059-1063); HAMMULT itself has
- * no such mode.  Needs the LDS kernels for the grid (dex_info.fast_path).
+ * Xs = (X + symmetry X^T)/2, exactly (anti)symmetric.  This is how the reference's start
+ * vectors enter (HELIUM_ORBITAL with SIGN = +-1, hammod.F90:1059-1063); HAMMULT
+ * itself has no such mode.  Needs the LDS kernels for the grid (dex_info.fast_path).
  * With howmany >= 2 (and kernel timing off) the columns go through the passes in
  * even batches of up to 16 per launch on small grids, 4 on large ones. */
 int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
@@ -115,15 +115,15 @@ int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howma
 
 /* dex_matvec_sym_device without any device allocation: no counterpart in the
  * reference; for callers that cannot allocate (code under HIP graph capture,
- * serving loops that forbid it).  The intermediate U lives in a static 64 MiB
- * device array that the library holds on every GPU it runs on until the
- * process ends (exchange-symmetric calls keep to the same limits), so the LDS kernels' grids are limited to NN <= 11 in an FP64
- * context and NN <= 13 in an FP32 one (larger: DEX_ESIZE); FP64 grids without
- * the LDS kernels (NN >= 23) use the six-pass kernels, which need no scratch.
+ * serving loops that forbid it).  The general form's intermediate U lives in a
+ * static 64 MiB device array that the library holds on every GPU it runs on until
+ * the process ends, so grids with the LDS kernels are limited to NN <= 11 in an
+ * FP64 context and NN <= 13 in an FP32 one (larger: DEX_ESIZE), in either
+ * symmetry; FP64 grids without them (NN >= 23) keep U in Y.
  * General columns go one at a time, exchange-symmetric ones in batches as above;
- * no kernel timing is recorded.  Calls that overlap on one GPU share the array and race: order them
- * on one stream or serialise them.  U needs no clearing (each column's first
- * pass writes all of it). */
+ * no kernel timing is recorded.  Calls that overlap on one GPU share the array and
+ * race: order them on one stream or serialise them.  U needs no clearing (each
+ * column's first pass writes all of it). */
 int dex_matvec_noalloc(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
                        int64_t checksize, int32_t single, int32_t symmetry);
 
