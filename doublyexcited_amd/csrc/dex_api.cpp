@@ -46,6 +46,7 @@ double now_s() {
 
 constexpr int kMaxDesc = 512;
 constexpr int kMaxSmall = 96 * 64;
+constexpr int kNormCols = 128;  // residual columns to a wait (two sums each in d_dots)
 
 }  // namespace
 
@@ -2451,6 +2452,24 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
   DEX_HIP(blocks.take(&v, size_t(c->d) * sizeof(Dbl2)));
   Dbl2 *ax = static_cast<Dbl2 *>(v);
   int st = DEX_OK;
+  if (dex::general_by_planes(c->nn)) {
+    // the sums come from the matvec's last pass, 128 columns to a wait
+    const double dd = double(c->d);
+    for (int j0 = 0; j0 < nev; j0 += kNormCols) {
+      const int k = std::min(nev - j0, kNormCols);
+      for (int j = j0; j < j0 + k; ++j) {
+        KTimer kt(c, DEX_K_GENERIC, 112.0 * dd, (24.0 * c->nn + 24.0) * dd);
+        DEX_HIP(dex::launch_general_norms(c->nn, static_cast<const Dbl2 *>(x_dev) + size_t(j) * c->d, ax, e[2 * j],
+                                          e[2 * j + 1], static_cast<double *>(c->d_partial), c->d_dots + 2 * (j - j0),
+                                          {c->d_vn, c->d_tinv, c->coef}, c->stream));
+      }
+      double h[2 * kNormCols];
+      DEX_HIP(hipMemcpyAsync(h, c->d_dots, size_t(2 * k) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+      DEX_HIP(hipStreamSynchronize(c->stream));
+      for (int j = 0; j < k; ++j) res_out[j0 + j] = std::sqrt(h[2 * j]) / std::sqrt(h[2 * j + 1]);
+    }
+    return DEX_OK;
+  }
   for (int j = 0; j < nev && st == DEX_OK; ++j) {
     const Dbl2 *xj = static_cast<const Dbl2 *>(x_dev) + size_t(j) * c->d;
     st = apply_h(c, xj, ax, false);

@@ -394,12 +394,16 @@ __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane
 // line.  It reads its entries of X and Z before it writes them, so Y may be either.
 // Runs start at any multiple of an entry (M is odd) and share lines with their
 // neighbours: consecutive tiles go to one XCD (workgroups are dealt to the 8 XCDs
-// in turn).
-template <int NN, typename R, typename XT, typename ZT, typename YT>
+// in turn).  With NORMS nothing is written but each workgroup's sums of |Y - e X|^2 and
+// |X|^2 in norms[2 blockIdx.x]: a residual needs no more of Y (112 bytes an entry over
+// the three passes where writing Y and reading it back with X took 160; 8 pairs at
+// NN = 17: 7.4 ms before).
+template <int NN, typename R, typename XT, typename ZT, typename YT, bool NORMS = false>
 __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(const XT *x, const ZT *z, YT *y,
                                                                              int64_t run, int64_t sa, int64_t sb,
                                                                              int64_t so, int64_t per_xcd,
-                                                                             MatvecCoef cf) {
+                                                                             MatvecCoef cf, double e_re, double e_im,
+                                                                             double *norms) {
   constexpr int P = plane_run<XT>(), N2 = NN * NN;
   extern __shared__ __align__(16) unsigned char smem[];
   const int r = threadIdx.x % P, bb = threadIdx.x / P;
@@ -435,6 +439,7 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
   b_axis(xr);
   if (on) line_apply<NN, R>(xr, [&](int l, R s) { kr[l] = s + b[(l * NN + bb) * P]; });
   b_axis(xi);
+  double rr = 0.0, xx = 0.0;
   if (on) {
     const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
     line_apply<NN, R>(xi, [&](int l, R s) {
@@ -443,8 +448,48 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
       YT o;
       o.x = zv.x + (s2r * kr[l] - s2i * ki);
       o.y = zv.y + (s2r * ki + s2i * kr[l]);
-      y[base + sa * l] = o;
+      if constexpr (NORMS) {
+        const double dr = o.x - (e_re * xr[l] - e_im * xi[l]), di = o.y - (e_re * xi[l] + e_im * xr[l]);
+        rr += dr * dr + di * di;
+        xx += double(xr[l]) * xr[l] + double(xi[l]) * xi[l];
+      } else {
+        y[base + sa * l] = o;
+      }
     });
+  }
+  if constexpr (NORMS) {
+    constexpr int W = round_up(NN * P, 64) / 64;
+    __shared__ double red[W][2];
+    for (int off = 32; off > 0; off >>= 1) {
+      rr += __shfl_down(rr, off);
+      xx += __shfl_down(xx, off);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      red[threadIdx.x >> 6][0] = rr;
+      red[threadIdx.x >> 6][1] = xx;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      double t = 0.0;
+      for (int w = 0; w < W; ++w) t += red[w][threadIdx.x];
+      norms[2 * size_t(blockIdx.x) + threadIdx.x] = t;
+    }
+  }
+}
+
+// out[e] = sum over nparts of partial[b nelem + e], one workgroup an element.
+__global__ __launch_bounds__(1024) void k_reduce_wide(const double *__restrict__ partial, int nparts, int nelem,
+                                                      double *__restrict__ out) {
+  __shared__ double red[16];
+  double s = 0.0;
+  for (int b = threadIdx.x; b < nparts; b += 1024) s += partial[size_t(b) * nelem + blockIdx.x];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s = 0.0;
+    for (int w = 0; w < 16; ++w) s += red[w];
+    out[blockIdx.x] = s;
   }
 }
 
@@ -517,7 +562,11 @@ bool plane1_setup() {
 
 template <int NN, typename R, typename XT, typename ZT, typename YT>
 bool plane2_setup() {
-  static std::atomic<bool> first{false}, second{false};
+  static std::atomic<bool> first{false}, second{false}, sums{false};
+  if constexpr (sizeof(R) == 8) {
+    if (!set_lds(reinterpret_cast<const void *>(&k_plane2<NN, R, XT, ZT, YT, true>), plane2_lds<NN, R, XT>(), sums))
+      return false;
+  }
   return set_lds(reinterpret_cast<const void *>(&k_plane2<NN, R, XT, ZT, ZT>), plane2_lds<NN, R, XT>(), first) &&
          set_lds(reinterpret_cast<const void *>(&k_plane2<NN, R, XT, ZT, YT>), plane2_lds<NN, R, XT>(), second);
 }
@@ -532,21 +581,33 @@ hipError_t plane1_nn(const void *x, void *z, const PotArgs &pot, hipStream_t s) 
   return hipGetLastError();
 }
 
+// k1 and i2, runs along (i1, j1); then j2 and k2, runs along (i1, j1, k1, i2): into Y,
+// or (norms, FP64) into the sums of |Y - e X|^2 and |X|^2 in out.
 template <int NN, typename R, typename XT, typename ZT, typename YT>
-hipError_t plane2_nn(const void *x, void *z, void *y, const MatvecCoef &cf, hipStream_t s) {
+hipError_t plane2_nn(const void *x, void *z, void *y, const MatvecCoef &cf, hipStream_t s, double *norms = nullptr,
+                     double e_re = 0.0, double e_im = 0.0, double *out = nullptr) {
   if (!plane2_setup<NN, R, XT, ZT, YT>()) return hipErrorInvalidDeviceFunction;
   constexpr int64_t N2 = NN * NN, N3 = NN * N2, N4 = NN * N3;
   constexpr int P = plane_run<XT>();
   const XT *xx = static_cast<const XT *>(x);
   ZT *zz = static_cast<ZT *>(z);
   auto per_xcd = [](int64_t run) { return ((run + P - 1) / P + 7) / 8; };  // run tiles an XCD takes
-  // k1 and i2, runs along (i1, j1); then j2 and k2, runs along (i1, j1, k1, i2)
-  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, ZT>), dim3(unsigned(8 * per_xcd(N2)), unsigned(N2)),
-                     dim3(round_up(NN * P, 64)), (plane2_lds<NN, R, XT>()), s, xx, static_cast<const ZT *>(zz), zz, N2,
-                     N2, N3, N4, per_xcd(N2), cf);
-  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, YT>), dim3(unsigned(8 * per_xcd(N4))), dim3(round_up(NN * P, 64)),
-                     (plane2_lds<NN, R, XT>()), s, xx, static_cast<const ZT *>(zz), static_cast<YT *>(y), N4, N4,
-                     N4 * NN, int64_t(0), per_xcd(N4), cf);
+  const dim3 block(round_up(NN * P, 64)), last(unsigned(8 * per_xcd(N4)));
+  const size_t lds = plane2_lds<NN, R, XT>();
+  double *none = nullptr;
+  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, ZT>), dim3(unsigned(8 * per_xcd(N2)), unsigned(N2)), block, lds, s, xx,
+                     static_cast<const ZT *>(zz), zz, N2, N2, N3, N4, per_xcd(N2), cf, 0.0, 0.0, none);
+  if constexpr (sizeof(R) == 8) {
+    if (norms) {
+      YT *noy = nullptr;
+      hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, YT, true>), last, block, lds, s, xx, static_cast<const ZT *>(zz),
+                         noy, N4, N4, N4 * NN, int64_t(0), per_xcd(N4), cf, e_re, e_im, norms);
+      hipLaunchKernelGGL(k_reduce_wide, dim3(2), dim3(1024), 0, s, norms, int(last.x), 2, out);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((k_plane2<NN, R, XT, ZT, YT>), last, block, lds, s, xx, static_cast<const ZT *>(zz),
+                     static_cast<YT *>(y), N4, N4, N4 * NN, int64_t(0), per_xcd(N4), cf, 0.0, 0.0, none);
   return hipGetLastError();
 }
 
@@ -674,6 +735,24 @@ hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y
       if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, coef, s);                  \
       return pass2_nn<N, float, double2, double2>(x, z, y, coef, s);                                  \
     }
+    DEX_NN_LIST(CASE)
+#undef CASE
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_general_norms(int nn, const Dbl2 *x, Dbl2 *z, double e_re, double e_im, double *partial,
+                                double *out, const PotArgs &pot, hipStream_t s) {
+  if (!general_by_planes(nn)) return hipErrorInvalidValue;
+  const hipError_t e = launch_general_first(nn, kIoF64, x, z, pot, s);
+  if (e != hipSuccess) return e;
+  switch (nn) {
+#define CASE(N)                                                                                                  \
+  case N:                                                                                                        \
+    if constexpr (N > kCubeMaxNN)                                                                                \
+      return plane2_nn<N, double, double2, double2, double2>(x, z, nullptr, pot.cf, s, partial, e_re, e_im, out); \
+    return hipErrorInvalidValue;
     DEX_NN_LIST(CASE)
 #undef CASE
     default:

@@ -84,3 +84,22 @@ def test_output_over_the_input(dex, n, prec, single, sym, cols):
         g.matvec_device(x, y, cols, single=single, symmetry=sym)
         g.matvec_device(x, x, cols, single=single, symmetry=sym)
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("n,prec,cols", [(3, "fp64", 3), (6, "fp64", 3), (6, "fp32", 130), (8, "fp64", 2),
+                                         (11, "fp64", 1)])
+def test_residuals_against_the_dense_product(dex, n, prec, cols):
+    """||H x - e x|| / ||x|| within 1e-13 of the dense product's (sums of D squares
+    of values that differ from the dense ones by 1e-15 of their largest)."""
+    import numpy as np
+
+    print(f"case: residuals N={n} {prec} cols={cols}", flush=True)
+    with dex.HeliumGrid(n, 0.45, 0.3, precision=prec) as g:
+        x = _block(g, min(cols, 3), 0, torch.complex128, n)
+        x = x.repeat((cols + 2) // 3)[:cols * g.d].contiguous() if cols > 3 else x
+        e = -0.7 + 0.01 * np.arange(cols) - 0.02j * np.arange(cols)
+        got = g.residuals_device(x, e)
+        for j in {0, cols // 2, cols - 1}:
+            v = x[j * g.d:(j + 1) * g.d]
+            ref = (torch.linalg.vector_norm(_dense(g, v) - complex(e[j]) * v) / torch.linalg.vector_norm(v)).item()
+            assert abs(got[j] - ref) <= 1e-13 * ref, j
