@@ -196,7 +196,8 @@ struct dex_ctx {
   dex::MatvecCoef coef{};
   hipStream_t stream = nullptr;
   bool fast64 = false, fast32 = false;
-  void *d_u = nullptr;  // the general matvec's intermediate, D complex128 (also used as D complex64)
+  void *d_u = nullptr;  // the general matvec's intermediates (ensure_u)
+  size_t u_bytes = 0;
   void *d_scratch = nullptr;  // this device's copy of `scratch` (dex_matvec_noalloc)
   ColDesc *d_desc = nullptr;
   unsigned char *d_args = nullptr;  // a combine's descriptors, C and beta, packed (one upload)
@@ -320,9 +321,35 @@ hipError_t stage_upload(dex_ctx *c, void *dev, const void *src, size_t bytes) {
   return hipMemcpyAsync(dev, h, bytes, hipMemcpyHostToDevice, c->stream);
 }
 
-int ensure_u(dex_ctx *c) {
-  if (c->d_u) return 0;
-  DEX_HIP(device_malloc(c->p.device, &c->d_u, size_t(c->d) * sizeof(Dbl2)));
+// Whether a call's outputs are, at an offset, its inputs: its columns then go one at a
+// time, each reading what the one before wrote (out = in + D: H x, H^2 x, ...).
+bool chained(const void *in, const void *out, size_t bytes) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(in), b = reinterpret_cast<uintptr_t>(out);
+  return a != b && a < b + bytes && b < a + bytes;
+}
+
+// Consecutive general columns of a pair of launches: as many as the 64 MiB of the
+// allocation-free entry point's array holds intermediates for, so that both entry
+// points take a call alike (16 up to NN = 7; 7 at NN = 9 and 2 at NN = 11 in FP64).
+// 16 columns at NN = 5: 33 us, 145 singly.
+int general_cols(const dex_ctx *c, int io, int left) {
+  if (dex::general_by_planes(c->nn)) return 1;
+  const size_t b = kScratchBytes / (size_t(c->d) * (io == dex::kIoF64 ? 16 : 8));
+  return std::min(int(std::min<size_t>(std::max<size_t>(b, 1), size_t(dex::kBatchMax))), left);
+}
+
+// Intermediates of `ncols` general columns (one complex128 column at least, which
+// other callers use too).
+int ensure_u(dex_ctx *c, int ncols = 1, int io = dex::kIoF64) {
+  const size_t bytes = std::max(size_t(c->d) * 16, size_t(ncols) * size_t(c->d) * (io == dex::kIoF64 ? 16 : 8));
+  if (c->d_u && c->u_bytes >= bytes) return 0;
+  if (c->d_u) {
+    DEX_HIP(hipStreamSynchronize(c->stream));
+    DEX_HIP(hipFree(c->d_u));
+    c->d_u = nullptr;
+  }
+  DEX_HIP(device_malloc(c->p.device, &c->d_u, bytes));
+  c->u_bytes = bytes;
   return 0;
 }
 
@@ -363,7 +390,7 @@ int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int nc
     if (sym != 0)
       DEX_HIP(dex::launch_pass1(c->nn, io, true, x, y, ncols, pot, c->stream));
     else
-      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], u, pot, c->stream));
+      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], u, ncols, pot, c->stream));
   }
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[1], c->stream));
   if (sym != 0) {
@@ -373,19 +400,22 @@ int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int nc
     // reads X and Z, writes Y; by planes two launches, the first writing Z again
     KTimer kt(c, DEX_K_PASS2, (2.0 * xb + zb + (planes ? xb + 2.0 * zb : 0.0)) * dd,
               ((planes ? 16.0 : 12.0) * nn + 8.0) * dd);
-    DEX_HIP(dex::launch_general_second(c->nn, io, x[0], u, y[0], c->coef, c->stream));
+    DEX_HIP(dex::launch_general_second(c->nn, io, x[0], u, y[0], ncols, c->coef, c->stream));
   }
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[2], c->stream));
   return 0;
 }
 
-// H on exchange-(anti)symmetric columns, a batch per pair of launches.
+// H on columns that have the LDS kernels, a batch per pair of launches.  General
+// columns must be consecutive (x[j], y[j] at D entries from x[j - 1], y[j - 1]).
 int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, int io, int sym) {
-  if (ncols < 0 || sym == 0 || !(io != dex::kIoF64 ? c->fast32 : c->fast64))
+  if (ncols < 0 || !(io != dex::kIoF64 ? c->fast32 : c->fast64))
     return fail(DEX_EINVAL, "batched matvec: bad column count or form");
   for (int j = 0, k = 0; j < ncols; j += k) {
-    k = batch_cols(c, io, ncols - j);
-    if (int st = fast_passes(c, io, x + j, y + j, k, sym, nullptr)) return st;
+    k = sym != 0 ? batch_cols(c, io, ncols - j) : general_cols(c, io, ncols - j);
+    if (sym == 0)
+      if (int st = ensure_u(c, k, io)) return st;
+    if (int st = fast_passes(c, io, x + j, y + j, k, sym, c->d_u)) return st;
   }
   return 0;
 }
@@ -393,8 +423,8 @@ int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, i
 // H on one complex128 column in FP64 with the intermediate in Y's own storage
 // (grids without an FP64 cube; x and y must differ).
 int generic_passes(dex_ctx *c, const void *x, void *y) {
-  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, {c->d_vn, c->d_tinv, c->coef}, c->stream));
-  DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, c->coef, c->stream));
+  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, {c->d_vn, c->d_tinv, c->coef}, c->stream));
+  DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, 1, c->coef, c->stream));
   return 0;
 }
 
@@ -950,8 +980,9 @@ int dex_matvec_sym_device(dex_ctx *c, const void *in, void *out, int32_t howmany
   if (sp && !c->fast32) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
   const bool f32 = c->p.precision == DEX_FP32;
   const size_t xb = sp ? 8 : 16;
-  if (symmetry != 0 && !c->timing && howmany >= 2) {
-    // exchange-symmetric columns, a batch per pair of launches
+  if ((f32 ? c->fast32 : c->fast64) && !c->timing && howmany >= 2 &&
+      !chained(in, out, size_t(howmany) * size_t(c->d) * xb)) {
+    // a batch of columns per pair of launches
     std::vector<const void *> xs(howmany);
     std::vector<void *> ys(howmany);
     for (int j = 0; j < howmany; ++j) {
@@ -998,8 +1029,9 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
   const int io = sp ? dex::kIoF32 : (f32 ? dex::kIoMixed : dex::kIoF64);
   const size_t xb = sp ? 8 : 16;  // bytes per entry of X and Y
   const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  const bool single_file = chained(in, out, size_t(howmany) * size_t(c->d) * xb);
   for (int j = 0, k = 0; j < howmany; j += k) {
-    k = fast && symmetry != 0 ? batch_cols(c, io, howmany - j) : 1;
+    k = !fast || single_file ? 1 : symmetry != 0 ? batch_cols(c, io, howmany - j) : general_cols(c, io, howmany - j);
     const void *x[dex::kBatchMax];
     void *y[dex::kBatchMax];
     for (int i = 0; i < k; ++i) {
@@ -1013,8 +1045,8 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
       DEX_HIP(dex::launch_symfold(c->nn, io, y, k, symmetry, c->stream));
     } else {
       // Z (fully written by the electron-1 pass before the second pass reads it)
-      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], c->d_scratch, pot, c->stream));
-      DEX_HIP(dex::launch_general_second(c->nn, io, x[0], c->d_scratch, y[0], c->coef, c->stream));
+      DEX_HIP(dex::launch_general_first(c->nn, io, x[0], c->d_scratch, k, pot, c->stream));
+      DEX_HIP(dex::launch_general_second(c->nn, io, x[0], c->d_scratch, y[0], k, c->coef, c->stream));
     }
   }
   return DEX_OK;

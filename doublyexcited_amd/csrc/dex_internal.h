@@ -90,12 +90,13 @@ struct PotArgs {
 // complex64 otherwise).
 hipError_t launch_pass1(int nn, int io, bool sym, const void *const *x, void *const *z, int ncols,
                         const PotArgs &pot, hipStream_t s);
-// General vectors, one column, any grid: the first launch and the rest (z: D
-// entries of the arithmetic's format; x and y may be one array where z is another,
-// z and y where x is another).
+// General vectors: the first launch and the rest, on ncols consecutive columns: one
+// where general_by_planes, up to kBatchMax elsewhere (z: D entries of the
+// arithmetic's format a column; x and y may be one array where z is another, z and y
+// where x is another).
 bool general_by_planes(int nn);
-hipError_t launch_general_first(int nn, int io, const void *x, void *z, const PotArgs &pot, hipStream_t s);
-hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, const MatvecCoef &coef,
+hipError_t launch_general_first(int nn, int io, const void *x, void *z, int ncols, const PotArgs &pot, hipStream_t s);
+hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, int ncols, const MatvecCoef &coef,
                                  hipStream_t s);
 // out[0] = ||H x - e x||^2 and out[1] = ||x||^2 of one complex128 column in FP64
 // (general_by_planes grids; z: D entries; partial: 2 doubles a run tile, at most

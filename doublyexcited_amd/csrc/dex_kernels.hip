@@ -205,10 +205,14 @@ __device__ __forceinline__ int64_t xcd_group_map(int64_t b, int64_t m) {
 }
 
 // Electron-2 pass for general vectors: Y = Z + s2 tau3D X on the stride-M cube
-// of each electron-1 index p (Z from k_pass1 with w = 1).
+// of each electron-1 index p of column blockIdx.y (columns M^2 entries apart; Z from
+// k_pass1 with w = 1; Y may
+// be X's or Z's storage: a thread reads each entry of Z before it writes that of Y,
+// and the workgroup's entries of X before any).
 template <int NN, typename R, typename XT, typename YT>
-__global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(
-    const XT *__restrict__ x, const typename Cplx<R>::type *__restrict__ z, YT *__restrict__ y, MatvecCoef cf) {
+__global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *__restrict__ x,
+                                                              const typename Cplx<R>::type *__restrict__ z,
+                                                              YT *__restrict__ y, MatvecCoef cf) {
   using C = typename Cplx<R>::type;
   constexpr int N2 = NN * NN;
   constexpr int N3 = NN * N2;
@@ -217,7 +221,7 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(
   R *b = a + N3;
   const int c = threadIdx.x;
   const bool on = c < N2;
-  const int64_t p = xcd_group_map(blockIdx.x, N3);
+  const int64_t p = xcd_group_map(blockIdx.x, N3) + int64_t(N3) * N3 * blockIdx.y;
   const int64_t M = N3;
   R xr[NN], xi[NN], kr[NN];
   if (on) {
@@ -537,11 +541,12 @@ hipError_t pass1_nn(const ColPtrs &xs, const ColPtrsW &zs, int ncols, const PotA
 }
 
 template <int NN, typename R, typename XT, typename YT>
-hipError_t pass2_nn(const void *x, const void *z, void *y, const MatvecCoef &cf, hipStream_t s) {
+hipError_t pass2_nn(const void *x, const void *z, void *y, int ncols, const MatvecCoef &cf, hipStream_t s) {
   using C = typename Cplx<R>::type;
   if (!pass2_setup<NN, R, XT, YT>()) return hipErrorInvalidDeviceFunction;
-  hipLaunchKernelGGL((k_pass2<NN, R, XT, YT>), dim3(NN * NN * NN), dim3(cube_threads<NN>()), (cube_lds<NN, R>()), s,
-                     static_cast<const XT *>(x), static_cast<const C *>(z), static_cast<YT *>(y), cf);
+  hipLaunchKernelGGL((k_pass2<NN, R, XT, YT>), dim3(NN * NN * NN, unsigned(ncols)), dim3(cube_threads<NN>()),
+                     (cube_lds<NN, R>()), s, static_cast<const XT *>(x), static_cast<const C *>(z),
+                     static_cast<YT *>(y), cf);
   return hipGetLastError();
 }
 
@@ -703,8 +708,19 @@ hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, h
 // 2850; complex64 at 17: 833 and 455; at 25: 7035 and 4300.
 bool general_by_planes(int nn) { return nn > kCubeMaxNN; }
 
-hipError_t launch_general_first(int nn, int io, const void *x, void *z, const PotArgs &pot, hipStream_t s) {
-  if (!general_by_planes(nn)) return launch_pass1(nn, io, false, &x, &z, 1, pot, s);
+hipError_t launch_general_first(int nn, int io, const void *x, void *z, int ncols, const PotArgs &pot, hipStream_t s) {
+  if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
+  if (!general_by_planes(nn)) {
+    const size_t d = size_t(nn) * nn * nn * nn * nn * nn;
+    const void *xs[kBatchMax];
+    void *zs[kBatchMax];
+    for (int j = 0; j < ncols; ++j) {
+      xs[j] = static_cast<const char *>(x) + size_t(j) * d * (io == kIoF32 ? 8 : 16);
+      zs[j] = static_cast<char *>(z) + size_t(j) * d * (io == kIoF64 ? 16 : 8);
+    }
+    return launch_pass1(nn, io, false, xs, zs, ncols, pot, s);
+  }
+  if (ncols != 1) return hipErrorInvalidValue;
   switch (nn) {
 #define CASE(N)                                                                           \
   case N:                                                                                 \
@@ -721,8 +737,9 @@ hipError_t launch_general_first(int nn, int io, const void *x, void *z, const Po
   }
 }
 
-hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, const MatvecCoef &coef,
+hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, int ncols, const MatvecCoef &coef,
                                  hipStream_t s) {
+  if (ncols < 1 || ncols > kBatchMax || (ncols != 1 && general_by_planes(nn))) return hipErrorInvalidValue;
   switch (nn) {
 #define CASE(N)                                                                                       \
   case N:                                                                                             \
@@ -731,9 +748,9 @@ hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y
       if (io == kIoF32) return plane2_nn<N, float, float2, float2, float2>(x, z, y, coef, s);         \
       return plane2_nn<N, float, double2, float2, double2>(x, z, y, coef, s);                         \
     } else {                                                                                          \
-      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, z, y, coef, s);               \
-      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, coef, s);                  \
-      return pass2_nn<N, float, double2, double2>(x, z, y, coef, s);                                  \
+      if (io == kIoF64) return pass2_nn<N, double, double2, double2>(x, z, y, ncols, coef, s);     \
+      if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, ncols, coef, s);        \
+      return pass2_nn<N, float, double2, double2>(x, z, y, ncols, coef, s);                        \
     }
     DEX_NN_LIST(CASE)
 #undef CASE
@@ -745,7 +762,7 @@ hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y
 hipError_t launch_general_norms(int nn, const Dbl2 *x, Dbl2 *z, double e_re, double e_im, double *partial,
                                 double *out, const PotArgs &pot, hipStream_t s) {
   if (!general_by_planes(nn)) return hipErrorInvalidValue;
-  const hipError_t e = launch_general_first(nn, kIoF64, x, z, pot, s);
+  const hipError_t e = launch_general_first(nn, kIoF64, x, z, 1, pot, s);
   if (e != hipSuccess) return e;
   switch (nn) {
 #define CASE(N)                                                                                                  \

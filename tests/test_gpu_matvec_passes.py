@@ -52,7 +52,8 @@ def _block(g, cols, sym, dtype, seed):
 
 @pytest.mark.parametrize("n,prec,single,sym,cols", [
     (1, "fp64", False, 1, 3), (1, "fp64", False, 0, 2), (2, "fp64", False, -1, 17), (2, "fp32", True, 1, 17),
-    (3, "fp64", False, 0, 3), (4, "fp64", False, 1, 2), (4, "fp32", True, 0, 2), (6, "fp64", False, -1, 3),
+    (3, "fp64", False, 0, 3), (4, "fp64", False, 1, 2), (4, "fp32", True, 0, 2), (4, "fp32", True, 0, 16),
+    (4, "fp64", False, 0, 15), (5, "fp32", False, 0, 5), (6, "fp64", False, -1, 3),
     (6, "fp32", True, -1, 5), (6, "fp32", False, 1, 2), (6, "fp32", False, 0, 1), (7, "fp64", False, 0, 1),
     (8, "fp64", False, 1, 2), (9, "fp32", True, 1, 2), (10, "fp64", False, -1, 1), (11, "fp32", True, 1, 1),
     (11, "fp32", True, 0, 1), (11, "fp64", False, 0, 1), (12, "fp32", True, -1, 1), (12, "fp64", False, 0, 1)])
@@ -103,3 +104,19 @@ def test_residuals_against_the_dense_product(dex, n, prec, cols):
             v = x[j * g.d:(j + 1) * g.d]
             ref = (torch.linalg.vector_norm(_dense(g, v) - complex(e[j]) * v) / torch.linalg.vector_norm(v)).item()
             assert abs(got[j] - ref) <= 1e-13 * ref, j
+
+
+@pytest.mark.parametrize("n,sym", [(2, 0), (2, 1), (5, 1)])
+def test_outputs_one_column_along_the_inputs(dex, n, sym):
+    """Y one column along X: each column takes the product of the one before."""
+    print(f"case: chained columns N={n} sym={sym}", flush=True)
+    with dex.HeliumGrid(n, 0.45, 0.3) as g:
+        buf = torch.zeros(4 * g.d, dtype=torch.complex128, device="cuda")
+        buf[:g.d] = _block(g, 1, sym, torch.complex128, n)
+        ref = [buf[:g.d].clone()]
+        for _ in range(3):
+            y = torch.empty_like(ref[-1])
+            g.matvec_device(ref[-1], y, 1, symmetry=sym)
+            ref.append(y)
+        g.matvec_device(buf[:3 * g.d], buf[g.d:], 3, symmetry=sym)
+        assert torch.equal(buf, torch.cat(ref))
