@@ -511,18 +511,23 @@ double distinct_entry_bytes(const std::vector<ColDesc> &ds, size_t n) {
   return b;
 }
 
+// sym (in the block operations below): 0, or +-1 where every column involved is an
+// exchange-symmetric (antisymmetric) vector: its two halves are each other's mirror
+// images, so Grams and combinations read one (half_blocks grids).
+
 // Runs one Gram launch (kl <= 64, kr <= 128) and copies the kl x kr result
 // into g (leading dimension ldg) at (i0, j0).  With share > 0 the skipped lower
 // blocks of the Hermitian share x share part are filled by conjugate symmetry.
 int gram_launch_copy(dex_ctx *c, const std::vector<ColDesc> &ds, int kl, int kr, int share,
-                     std::vector<cd> &g, int ldg, int i0, int j0) {
+                     std::vector<cd> &g, int ldg, int i0, int j0, int sym) {
   if (int st = upload_descs(c, ds)) return st;
   {
     const double hskip = share > 0 ? 0.5 * double(share) * double(share - 1) : 0.0;
-    KTimer kt(c, DEX_K_GRAM, double(c->d) * distinct_entry_bytes(ds, ds.size()),
-              8.0 * double(c->d) * (double(kl) * kr - hskip));
-    DEX_HIP(dex::launch_gram(c->d_desc, kl, kr, share, c->d, reinterpret_cast<Dbl2 *>(c->d_partial),
-                             c->d_gram_out, c->stream));
+    const bool half = sym != 0 && dex::half_blocks(c->m);
+    const double rows = double(c->d) * (half ? 0.5 : 1.0);
+    KTimer kt(c, DEX_K_GRAM, rows * distinct_entry_bytes(ds, ds.size()), 8.0 * rows * (double(kl) * kr - hskip));
+    DEX_HIP(dex::launch_gram(c->d_desc, kl, kr, share, c->d, half ? int(c->m) : 0,
+                             reinterpret_cast<Dbl2 *>(c->d_partial), c->d_gram_out, c->stream));
   }
   std::vector<cd> part(size_t(kl) * kr);
   DEX_HIP(hipMemcpyAsync(part.data(), c->d_gram_out, part.size() * sizeof(Dbl2), hipMemcpyDeviceToHost,
@@ -538,8 +543,7 @@ int gram_launch_copy(dex_ctx *c, const std::vector<ColDesc> &ds, int kl, int kr,
 }
 
 // G = L^H R (kl x kr, column-major) on the host; any sizes (chunked launches).
-int gram(dex_ctx *c, const std::vector<ColDesc> &l, const std::vector<ColDesc> &r,
-         std::vector<cd> &g) {
+int gram(dex_ctx *c, const std::vector<ColDesc> &l, const std::vector<ColDesc> &r, std::vector<cd> &g, int sym) {
   const int kl = int(l.size()), kr = int(r.size());
   g.assign(size_t(kl) * kr, 0.0);
   for (int i0 = 0; i0 < kl; i0 += 64)
@@ -547,25 +551,23 @@ int gram(dex_ctx *c, const std::vector<ColDesc> &l, const std::vector<ColDesc> &
       const int bl = std::min(64, kl - i0), br = std::min(128, kr - j0);
       std::vector<ColDesc> ds(l.begin() + i0, l.begin() + i0 + bl);
       ds.insert(ds.end(), r.begin() + j0, r.begin() + j0 + br);
-      if (int st = gram_launch_copy(c, ds, bl, br, 0, g, kl, i0, j0)) return st;
+      if (int st = gram_launch_copy(c, ds, bl, br, 0, g, kl, i0, j0, sym)) return st;
     }
   return 0;
 }
 
 // G = X^H X for k <= 64 columns: every column is read once.
-int gram_self(dex_ctx *c, const std::vector<ColDesc> &x, std::vector<cd> &g) {
+int gram_self(dex_ctx *c, const std::vector<ColDesc> &x, std::vector<cd> &g, int sym) {
   const int k = int(x.size());
-  if (k > 64) return gram(c, x, x, g);
+  if (k > 64) return gram(c, x, x, g, sym);
   g.assign(size_t(k) * k, 0.0);
-  return gram_launch_copy(c, x, k, k, k, g, k, 0, 0);
+  return gram_launch_copy(c, x, k, k, k, g, k, 0, 0, sym);
 }
 
 // [K | M] = B^H [B | Q] with B = AQ - sigma Q: for nq <= 64 one launch that reads
 // AQ and Q once; wider bases (up to 96) go through the chunked general Gram.
-int gram(dex_ctx *c, const std::vector<ColDesc> &l, const std::vector<ColDesc> &r, std::vector<cd> &g);
-
 int gram_harmonic(dex_ctx *c, const std::vector<Dbl2 *> &q, const std::vector<Dbl2 *> &aq, cd sigma,
-                  std::vector<cd> &g) {
+                  std::vector<cd> &g, int sym) {
   const int nq = int(q.size());
   if (nq < 1 || nq > 96) return fail(DEX_EINVAL, "projected basis must have 1..96 columns");
   if (nq > 64) {
@@ -574,7 +576,7 @@ int gram_harmonic(dex_ctx *c, const std::vector<Dbl2 *> &q, const std::vector<Db
     for (int j = 0; j < nq; ++j) l.push_back(shifted(aq[j], q[j], sigma));
     r = l;
     for (int j = 0; j < nq; ++j) r.push_back(plain(q[j]));
-    return gram(c, l, r, g);
+    return gram(c, l, r, g, sym);
   }
   const int ma = (nq + 15) / 16;
   std::vector<ColDesc> ds;
@@ -585,7 +587,7 @@ int gram_harmonic(dex_ctx *c, const std::vector<Dbl2 *> &q, const std::vector<Db
   }
   for (int j = 0; j < nq; ++j) ds.push_back(ColDesc{nullptr, nullptr, 0, 0, -1, 0});
   g.assign(size_t(nq) * 2 * nq, 0.0);
-  return gram_launch_copy(c, ds, nq, 2 * nq, nq, g, nq, 0, 0);
+  return gram_launch_copy(c, ds, nq, 2 * nq, nq, g, nq, 0, 0, sym);
 }
 
 // The iteration's X/P update as two launches of up to 16 outputs (on unless
@@ -601,7 +603,7 @@ bool split_update() {
 // out_j = sum_i in_i C(i, j) (+ beta_j out_j), row-local, in-place safe; each
 // output column is stored in its own pointer's format.
 int combine(dex_ctx *c, const std::vector<ColDesc> &in, const std::vector<Dbl2 *> &out,
-            const std::vector<cd> &cm, const std::vector<cd> *beta = nullptr) {
+            const std::vector<cd> &cm, const std::vector<cd> *beta, int sym) {
   const int nin = int(in.size()), nout = int(out.size());
   if (nout == 0) return 0;
   if (nin * nout > kMaxSmall || cm.size() < size_t(nin) * nout || cm.size() > size_t(kMaxSmall) ||
@@ -623,13 +625,18 @@ int combine(dex_ctx *c, const std::vector<ColDesc> &in, const std::vector<Dbl2 *
   std::memcpy(img.data() + bd, cm.data(), cm.size() * sizeof(Dbl2));
   if (beta) std::memcpy(img.data() + bd + bc, beta->data(), bb);
   DEX_HIP(stage_upload(c, c->d_args, img.data(), img.size()));
+  const bool half = sym != 0 && dex::half_blocks(c->m) && dex::combine_halves(nout);
+  const double rows = double(c->d) * (half ? 0.5 : 1.0);  // read (all outputs are written)
   KTimer kt(c, DEX_K_COMBINE,
-            double(c->d) * (distinct_entry_bytes(in, in.size()) + out_bytes * (beta ? 2.0 : 1.0)),
-            8.0 * double(c->d) * nin * nout);
+            rows * (distinct_entry_bytes(in, in.size()) + (beta ? out_bytes : 0.0)) + double(c->d) * out_bytes,
+            8.0 * rows * nin * nout);
+  const auto *dd = reinterpret_cast<const ColDesc *>(c->d_args);
   const Dbl2 *dc = reinterpret_cast<const Dbl2 *>(c->d_args + bd);
   const Dbl2 *dbeta = beta ? reinterpret_cast<const Dbl2 *>(c->d_args + bd + bc) : nullptr;
-  DEX_HIP(dex::launch_combine(reinterpret_cast<const ColDesc *>(c->d_args), nin, nout, dc, dbeta, c->d,
-                              c->stream));
+  if (half)
+    DEX_HIP(dex::launch_combine_sym(dd, nin, nout, dc, dbeta, int(c->m), sym, c->stream));
+  else
+    DEX_HIP(dex::launch_combine(dd, nin, nout, dc, dbeta, c->d, c->stream));
   return 0;
 }
 
@@ -1148,7 +1155,7 @@ int dex_dots_device(dex_ctx *c, const void *bras, const void *kets, int64_t size
   for (int i = 0; i < nn; ++i) l.push_back(plain(static_cast<const Dbl2 *>(bras) + size_t(i) * size));
   for (int j = 0; j < mm; ++j) r.push_back(plain(static_cast<const Dbl2 *>(kets) + size_t(j) * size));
   std::vector<cd> g;
-  if (int st = gram(c, l, r, g)) return st;
+  if (int st = gram(c, l, r, g, 0)) return st;
   std::memcpy(out, g.data(), g.size() * sizeof(cd));
   return DEX_OK;
 }
@@ -1234,7 +1241,7 @@ struct Solver {
     const int k = x.size();
     std::vector<cd> g;
     double t0 = now_s();
-    if (int st = gram_self(c, descs_of(x), g)) return st;
+    if (int st = gram_self(c, descs_of(x), g, sym)) return st;
     t_gram += now_s() - t0;
     t0 = now_s();
     double asum = 0.0;
@@ -1308,11 +1315,11 @@ struct Solver {
       if (kout > 0) {
         std::vector<ColDesc> in = descs_of(x);
         std::vector<Dbl2 *> out(x.cols.begin(), x.cols.begin() + kout);
-        if (int st = combine(c, in, out, t, nullptr)) return -st;
+        if (int st = combine(c, in, out, t, nullptr, sym)) return -st;
         if (ax) {
           std::vector<ColDesc> ain = descs_of(*ax);
           std::vector<Dbl2 *> aout(ax->cols.begin(), ax->cols.begin() + kout);
-          if (int st = combine(c, ain, aout, t, nullptr)) return -st;
+          if (int st = combine(c, ain, aout, t, nullptr, sym)) return -st;
         }
       }
       t_update += now_s() - t0;
@@ -1332,7 +1339,7 @@ struct Solver {
     if (q.size() == 0 || b.size() == 0) return 0;
     std::vector<cd> g;
     double t0 = now_s();
-    if (int st = gram(c, descs_of(q), descs_of(b), g)) return st;
+    if (int st = gram(c, descs_of(q), descs_of(b), g, sym)) return st;
     t_gram += now_s() - t0;
     t0 = now_s();
     const int kq = q.size(), kb = b.size();
@@ -1352,12 +1359,12 @@ struct Solver {
       std::vector<ColDesc> in;
       if (first) in = descs_of(b);
       for (int i = 0; i < nq; ++i) in.push_back(plain(q.cols[q0 + i]));
-      if (int st = combine(c, in, b.cols, cm, first ? nullptr : &one)) return st;
+      if (int st = combine(c, in, b.cols, cm, first ? nullptr : &one, sym)) return st;
       if (ab) {
         std::vector<ColDesc> ain;
         if (first) ain = descs_of(*ab);
         for (int i = 0; i < nq; ++i) ain.push_back(plain(aq->cols[q0 + i]));
-        if (int st = combine(c, ain, ab->cols, cm, first ? nullptr : &one)) return st;
+        if (int st = combine(c, ain, ab->cols, cm, first ? nullptr : &one, sym)) return st;
       }
       q0 += nq;
     }
@@ -1375,13 +1382,13 @@ struct Solver {
     const int n1 = std::min(kq, 64 - k);
     std::vector<ColDesc> ds(w);
     for (int i = 0; i < n1; ++i) ds.push_back(plain(q.cols[i]));
-    if (int st = gram_launch_copy(c, ds, k + n1, k, k, g, rows, 0, 0)) return st;
+    if (int st = gram_launch_copy(c, ds, k + n1, k, k, g, rows, 0, 0, sym)) return st;
     for (int i0 = n1; i0 < kq; i0 += 64) {
       const int bl = std::min(64, kq - i0);
       std::vector<ColDesc> d2;
       for (int i = 0; i < bl; ++i) d2.push_back(plain(q.cols[i0 + i]));
       d2.insert(d2.end(), w.begin(), w.end());
-      if (int st = gram_launch_copy(c, d2, bl, k, 0, g, rows, k + i0, 0)) return st;
+      if (int st = gram_launch_copy(c, d2, bl, k, 0, g, rows, k + i0, 0, sym)) return st;
     }
     t_gram += now_s() - t0;
     return 0;
@@ -1418,7 +1425,7 @@ struct Solver {
       std::vector<ColDesc> in;
       if (first) in = w;
       for (int i = 0; i < nq; ++i) in.push_back(plain(q.cols[q0 + i]));
-      if (int st = combine(c, in, out.cols, cm, first ? nullptr : &one)) return st;
+      if (int st = combine(c, in, out.cols, cm, first ? nullptr : &one, sym)) return st;
       q0 += nq;
       if (nq == 0) break;
     }
@@ -1608,7 +1615,7 @@ struct Solver {
         return 0;  // b = 0: x = 0, which b already holds
       }
       const double tg = now_s();
-      if (int st = gram(c, descs_of(q1), descs_of(b), r0)) return st;
+      if (int st = gram(c, descs_of(q1), descs_of(b), r0, sym)) return st;
       t_gram += now_s() - tg;
     }
     qall = q1;
@@ -1688,7 +1695,7 @@ struct Solver {
       for (int j = 0; j < nout; ++j)
         for (int i = 0; i < bi; ++i) sub[i + size_t(bi) * j] = cm[i0 + i + size_t(nin) * j];
       std::vector<cd> one(nout, 1.0);
-      if (int st = combine(c, ds, out.cols, sub, i0 > 0 ? &one : nullptr)) return st;
+      if (int st = combine(c, ds, out.cols, sub, i0 > 0 ? &one : nullptr, sym)) return st;
     }
     return 0;
   }
@@ -1764,7 +1771,7 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
       if (!(aa[j] > 0)) return fail(DEX_EZEROBLOCK, "zero start vector");
       dm[j + size_t(nev) * j] = 1.0 / std::sqrt(aa[j]);
     }
-    if (int st = combine(c, descs_of(X), X.cols, dm)) return st;
+    if (int st = combine(c, descs_of(X), X.cols, dm, nullptr, S.sym)) return st;
   }
   auto precblock = [&](Block &b) -> int {
     if (inner == 0 || b.size() == 0) return 0;
@@ -1903,7 +1910,7 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
         }
         std::vector<ColDesc> in = descs_of(aprev);
         for (Dbl2 *p : prev.cols) in.push_back(plain(p));
-        if (int st = combine(c, in, sl.cols, cm)) return st;
+        if (int st = combine(c, in, sl.cols, cm, nullptr, S.sym)) return st;
       }
       if (int st = precblock(sl)) return st;  // :118-126, :148-156
       {
@@ -1940,7 +1947,7 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
     if (nq > 96) return fail(DEX_EINVAL, "projected basis larger than 96");
     std::vector<cd> km;
     double t0 = now_s();
-    if (int st = gram_harmonic(c, Q.cols, AQ.cols, sigma, km)) return st;
+    if (int st = gram_harmonic(c, Q.cols, AQ.cols, sigma, km, S.sym)) return st;
     S.t_gram += now_s() - t0;
     t0 = now_s();
     std::vector<cd> kp(size_t(nq) * nq), mp(size_t(nq) * nq);
@@ -2018,18 +2025,18 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
           for (int j = 0; j < npo; ++j)
             for (int k = 0; k < bp; ++k) subp[k + size_t(bp) * j] = sub[rows_p[k] + size_t(bi) * (nev + j)];
           std::vector<cd> onex(nev, 1.0), onep(npo, 1.0);
-          if (int st = combine(c, qd, outx, subx, i0 > 0 ? &onex : nullptr)) return st;
-          if (int st = combine(c, aqd, aoutx, subx, i0 > 0 ? &onex : nullptr)) return st;
+          if (int st = combine(c, qd, outx, subx, i0 > 0 ? &onex : nullptr, S.sym)) return st;
+          if (int st = combine(c, aqd, aoutx, subx, i0 > 0 ? &onex : nullptr, S.sym)) return st;
           if (bp > 0) {
-            if (int st = combine(c, qdp, outp, subp, i0 > 0 ? &onep : nullptr)) return st;
-            if (int st = combine(c, aqdp, aoutp, subp, i0 > 0 ? &onep : nullptr)) return st;
+            if (int st = combine(c, qdp, outp, subp, i0 > 0 ? &onep : nullptr, S.sym)) return st;
+            if (int st = combine(c, aqdp, aoutp, subp, i0 > 0 ? &onep : nullptr, S.sym)) return st;
           } else if (i0 == 0) {
             return fail(DEX_EINVAL, "update: no input for the new P in the first chunk");
           }
           continue;
         }
-        if (int st = combine(c, qd, out, sub, i0 > 0 ? &one : nullptr)) return st;
-        if (int st = combine(c, aqd, aout, sub, i0 > 0 ? &one : nullptr)) return st;
+        if (int st = combine(c, qd, out, sub, i0 > 0 ? &one : nullptr, S.sym)) return st;
+        if (int st = combine(c, aqd, aout, sub, i0 > 0 ? &one : nullptr, S.sym)) return st;
       }
     }
     for (int j = nact; j < np; ++j) {
@@ -2257,6 +2264,11 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
     const size_t bytes = size_t(c->d) * nev * sizeof(Dbl2);
     if (hipMemcpyAsync(px_dev, x_dev, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
       st = fail(DEX_EHIP, "device copy failed");
+    // the block operations read one half of an exchange-symmetric vector: any other X
+    // counts as Xs, as in the matvec (no change to an exactly symmetric one)
+    for (int j = 0; j < nev && symmetry != 0 && !st; ++j)
+      if (dex::launch_sym_project(out.cols[j], c->m, symmetry, c->stream) != hipSuccess)
+        st = fail(DEX_EHIP, "exchange projection failed");
     if (!st) st = S.inner_solve(out, inner_iter, cd(sigma_re, sigma_im));
   }
   if (hipStreamSynchronize(c->stream) != hipSuccess && !st) st = fail(DEX_EHIP, "stream synchronise failed");
@@ -2402,7 +2414,7 @@ extern "C" int dex_diagsubspace_device(dex_ctx *c, const double *orbitals, int32
         break;
       }
       std::vector<cd> sc(1, 1.0 / std::sqrt(aa[0]));
-      if (int e = combine(c, {plain(out)}, {out}, sc)) {
+      if (int e = combine(c, {plain(out)}, {out}, sc, nullptr, 0)) {
         st = e;
         break;
       }

@@ -110,11 +110,17 @@ hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, h
 // `descs` holds kl L descriptors then kr - share R descriptors.  With
 // share > 0 the leading share x share block is Hermitian and only its upper
 // 16 x 16 blocks are computed (the rest of that block is left unset).
-// `partial` must hold gram_partial_elems(kl, kr) Dbl2.
+// `partial` must hold gram_partial_elems(kl, kr) Dbl2.  m > 0: every column is an
+// exchange-symmetric or every one an exchange-antisymmetric M x M matrix (d = m m),
+// read on and above the diagonal only; m = 0: all rows of any columns.
 int gram_blocks();
 size_t gram_partial_elems(int kl, int kr);
-hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t d, Dbl2 *partial,
+hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, Dbl2 *partial,
                        Dbl2 *out, hipStream_t s);
+
+// Blocks of exchange-(anti)symmetric columns are read by halves from NN = 11 on.
+constexpr int64_t kHalfMinM = 1331;
+bool half_blocks(int64_t m);
 
 // out_j = beta_j out_j + sum_i in_i C(i, j) row by row; in-place aliasing of
 // an output with an input is allowed.  `descs`: nin input descriptors then
@@ -122,6 +128,12 @@ hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t 
 // null) are device arrays.  nin <= 64, nout <= 48.
 hipError_t launch_combine(const ColDesc *descs, int nin, int nout, const Dbl2 *c,
                           const Dbl2 *beta, int64_t d, hipStream_t s);
+
+// launch_combine on columns that all are exchange-symmetric (sign 1) or antisymmetric
+// (-1) M x M matrices, inputs read on one side of the diagonal; where combine_halves.
+bool combine_halves(int nout);
+hipError_t launch_combine_sym(const ColDesc *descs, int nin, int nout, const Dbl2 *c, const Dbl2 *beta, int m,
+                              int sign, hipStream_t s);
 
 // Per column j: sum |a_j|^2, sum conj(a_j) b_j, sum |b_j|^2 (b from descs[k + j]).
 size_t coldots_partial_elems(int k);

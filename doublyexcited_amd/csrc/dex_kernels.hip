@@ -267,9 +267,8 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *__restri
 constexpr int kSymT = 32;
 constexpr int kSymBlk = 4;
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, int sign) {
-  using R = typename Real<T>::type;
+// Tile pair (ta, tb), ta <= tb, of this workgroup; false beyond the matrix.
+__device__ __forceinline__ bool sym_tile(int m, int nblk, int &ta, int &tb) {
   const int xcd = blockIdx.x % 8, s = blockIdx.x / 8;
   const int blk = (s / (kSymBlk * kSymBlk)) * 8 + xcd, in = s % (kSymBlk * kSymBlk);
   // block (ba, bb), ba <= bb, from its index bb (bb + 1) / 2 + ba
@@ -277,8 +276,20 @@ __global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, i
   while (bb * (bb + 1) / 2 > blk) --bb;
   while ((bb + 1) * (bb + 2) / 2 <= blk) ++bb;
   const int ba = blk - bb * (bb + 1) / 2;
-  const int ta = ba * kSymBlk + in % kSymBlk, tb = bb * kSymBlk + in / kSymBlk;
-  if (bb >= nblk || ta > tb || tb * kSymT >= m) return;
+  ta = ba * kSymBlk + in % kSymBlk;
+  tb = bb * kSymBlk + in / kSymBlk;
+  return bb < nblk && ta <= tb && tb * kSymT < m;
+}
+
+// Blocks along an axis, and workgroups of a launch over the tile pairs.
+constexpr int sym_blocks(int m) { return ((m + kSymT - 1) / kSymT + kSymBlk - 1) / kSymBlk; }
+constexpr int sym_grid(int m) { return round_up(sym_blocks(m) * (sym_blocks(m) + 1) / 2, 8) * kSymBlk * kSymBlk; }
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, int sign) {
+  using R = typename Real<T>::type;
+  int ta, tb;
+  if (!sym_tile(m, nblk, ta, tb)) return;
   T *__restrict__ y = static_cast<T *>(ys.p[blockIdx.y]);
   __shared__ T s1[kSymT][kSymT + 1], s2[kSymT][kSymT + 1];
   const int tx = threadIdx.x, ty = threadIdx.y;
@@ -689,10 +700,8 @@ hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, h
   if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
   ColPtrsW ys{};
   for (int j = 0; j < ncols; ++j) ys.p[j] = y[j];
-  const int m = nn * nn * nn;
-  const int nt = (m + kSymT - 1) / kSymT, nblk = (nt + kSymBlk - 1) / kSymBlk;
-  const int pairs = nblk * (nblk + 1) / 2;
-  const dim3 g(unsigned(round_up(pairs, 8) * kSymBlk * kSymBlk), unsigned(ncols)), b(kSymT, 8);
+  const int m = nn * nn * nn, nblk = sym_blocks(m);
+  const dim3 g(unsigned(sym_grid(m)), unsigned(ncols)), b(kSymT, 8);
   if (io == kIoF32)
     hipLaunchKernelGGL((k_symfold<float2>), g, b, 0, s, ys, m, nblk, sign);
   else
@@ -801,6 +810,9 @@ __device__ __forceinline__ void st_col(void *p, int fmt, int64_t r, double2 v) {
     reinterpret_cast<double2 *>(p)[r] = v;
 }
 
+// Four floats at 8-byte alignment (a row pair that starts at an odd row).
+typedef float dex_v4f __attribute__((ext_vector_type(4), aligned(8)));
+
 // Two adjacent rows r, r + 1 of a complex128 (fmt 0) or complex64 (fmt 1)
 // column in FP64; `two` false reads only row r (the last row of an odd-length
 // column).  A complex64 pair is one 16-byte load, a complex128 pair two.
@@ -808,7 +820,7 @@ __device__ __forceinline__ void ld_col2(const void *p, int fmt, int64_t r, bool 
   if (fmt != 0) {
     const float2 *q = reinterpret_cast<const float2 *>(p) + r;
     if (two) {
-      const float4 w = *reinterpret_cast<const float4 *>(q);
+      const dex_v4f w = *reinterpret_cast<const dex_v4f *>(q);
       v0 = make_double2(double(w.x), double(w.y));
       v1 = make_double2(double(w.z), double(w.w));
     } else {
@@ -847,7 +859,85 @@ __device__ __forceinline__ double2 col_value(const ColDesc &c, int64_t r) {
   return o;
 }
 
-// Partial Gram G = L^H R over a contiguous row range per workgroup, on the FP64
+// The row tiles a workgroup of the Gram kernels takes, in order.
+//   !TRI: rows 0 .. d - 1, tiles round robin over the grid.
+//   TRI: the columns are exchange-(anti)symmetric M x M matrices, whose products
+//     conj(l) r are symmetric: only the 64 x 64 blocks on and above the diagonal
+//     are read, those above first (`diag` false: the caller doubles their sum), then
+//     the diagonal ones.  A unit is 64 consecutive rows of one matrix column (fewer in
+//     the last block); consecutive units go to one XCD, where the lines that two of
+//     them share (M is odd) meet in L2.  Tiles cut at whole lines instead: no faster
+//     (280 for 290 us at 64 x 10 columns, M = 1331), and 5% slower where 64-row tiles
+//     become five a unit.
+constexpr int kTriT = 64;
+
+template <int ROWS, bool TRI>
+struct RowWalk {
+  static_assert(kTriT % ROWS == 0, "whole tiles in a unit");
+  int64_t row = 0;  // first row of the tile
+  int rows = 0;     // its rows, 0 when none is left
+  bool diag = false;
+
+  __device__ RowWalk(int64_t d, int m) : m_(m) {
+    if constexpr (!TRI) {
+      row = int64_t(blockIdx.x) * ROWS;
+      left_ = d - row;
+    } else {
+      const int b = m / kTriT;
+      n_ = kTriT / 2 * b * (b - 1) + (m - kTriT * b) * b;
+      i_ = blockIdx.x / 8;
+      unit();
+    }
+    rows = left_ < ROWS ? (left_ > 0 ? int(left_) : 0) : ROWS;
+  }
+  __device__ void next() {
+    const int64_t by = TRI ? int64_t(ROWS) : int64_t(gridDim.x) * ROWS;
+    row += by;
+    left_ -= by;
+    if (TRI && left_ <= 0) {
+      i_ += gridDim.x / 8;
+      unit();
+    }
+    rows = left_ < ROWS ? (left_ > 0 ? int(left_) : 0) : ROWS;
+  }
+
+ private:
+
+  int64_t left_ = 0;  // rows from `row` to the end (of the unit)
+  int m_, i_ = 0, n_ = 0;
+
+  // The first tile of this workgroup's unit i_, or of a later phase.
+  __device__ void unit() {
+    for (;;) {
+      const int per = (n_ + 7) / 8, u = int(blockIdx.x % 8) * per + i_;
+      if (i_ < per && u < n_) {
+        if (!diag) {
+          // block column j from its first unit, 32 j (j - 1)
+          int j = int((1.0f + sqrtf(1.0f + float(u) * (8.0f / kTriT))) * 0.5f);
+          while (kTriT / 2 * j * (j - 1) > u) --j;
+          while (kTriT / 2 * j * (j + 1) <= u) ++j;
+          const int v = u - kTriT / 2 * j * (j - 1);
+          row = int64_t(kTriT * j + v / j) * m_ + kTriT * (v % j);
+          left_ = kTriT;
+        } else {
+          const int p0 = u / kTriT * kTriT;
+          row = int64_t(u) * m_ + p0;
+          left_ = m_ - p0 < kTriT ? m_ - p0 : kTriT;
+        }
+        return;
+      }
+      if (diag) {
+        left_ = 0;
+        return;
+      }
+      diag = true;
+      n_ = m_;
+      i_ = blockIdx.x / 8;
+    }
+  }
+};
+
+// Partial Gram G = L^H R of each workgroup's row tiles (RowWalk), on the FP64
 // matrix cores.  G = L^H R is a GEMM whose
 // inner dimension is the vector length: per 4 rows, v_mfma_f64_16x16x4f64
 // multiplies a 16 x 4 slice of L^T by a 4 x 16 slice of R into a 16 x 16
@@ -874,10 +964,9 @@ constexpr int gram_mfma_rows(int mt, int nt, int tall = 16) {
   return r;
 }
 
-template <int MT, int NT, int TALL = 16>
+template <int MT, int NT, int TALL, bool TRI>
 __global__ __launch_bounds__(kGramThreads) void k_gram_mfma(const ColDesc *__restrict__ descs, int kl,
-                                                            int kr, int share, int64_t d,
-                                                            int64_t rows_per_block,
+                                                            int kr, int share, int64_t d, int m,
                                                             double2 *__restrict__ partial) {
   constexpr int LD = 16 * MT + 16 * NT + 1;
   constexpr int ROWS = gram_mfma_rows(MT, NT, TALL);
@@ -937,24 +1026,18 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_mfma(const ColDesc *__res
       pf[p] = dc.fmt;
     }
   }
-  // rows_per_block > 0: this workgroup's rows are one contiguous range; 0: the
-  // workgroups take tiles round robin (tile t to workgroup t % gridDim.x), so
-  // the grid sweeps every column together through a narrow window of rows
-  const bool strided = rows_per_block == 0;
-  const int64_t r0 = strided ? int64_t(blockIdx.x) * ROWS : int64_t(blockIdx.x) * rows_per_block;
-  const int64_t r1 = strided ? d : (r0 + rows_per_block < d ? r0 + rows_per_block : d);
-  const int64_t rstep = strided ? int64_t(gridDim.x) * ROWS : ROWS;
   // One tile in flight per workgroup while the matrix cores work on the
   // previous one: three register stages (more bytes in flight per workgroup)
   // measured 4-8% slower on the narrow shapes (fewer resident workgroups)
   double2 va[PMAX][2], vb[PMAX][2];
-  auto fetch = [&](int64_t rb) {
+  auto fetch = [&](const RowWalk<ROWS, TRI> &w) {
 #pragma unroll
     for (int p = 0; p < PMAX; ++p) {
-      const int64_t row = rb + 2 * ((tid + kGramThreads * p) % HALF);
+      const int lr = 2 * ((tid + kGramThreads * p) % HALF);
+      const int64_t row = w.row + lr;
       va[p][0] = va[p][1] = vb[p][0] = vb[p][1] = make_double2(0.0, 0.0);
-      if (pa[p] != nullptr && row < r1) {
-        const bool two = row + 1 < r1;
+      if (pa[p] != nullptr && lr < w.rows) {
+        const bool two = lr + 1 < w.rows;
         ld_col2(pa[p], pf[p], row, two, va[p][0], va[p][1]);
         if (pb[p] != nullptr) ld_col2(pb[p], pf[p], row, two, vb[p][0], vb[p][1]);
       }
@@ -982,11 +1065,24 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_mfma(const ColDesc *__res
       }
     }
   };
-  if (r0 < r1) fetch(r0);
-  for (int64_t rb = r0; rb < r1; rb += rstep) {
+  bool halves = TRI;  // the sums so far count half
+  auto twice = [&]() {
+#pragma unroll
+    for (int q = 0; q < QMAX; ++q) {
+      accr[q] += accr[q];
+      acci[q] += acci[q];
+    }
+    halves = false;
+  };
+  RowWalk<ROWS, TRI> walk(d, m);  // one tile ahead: the tile in flight
+  if (walk.rows) fetch(walk);
+  while (walk.rows) {
+    const bool diag = walk.diag;
+    walk.next();
     store();
     __syncthreads();
-    if (rb + rstep < r1) fetch(rb + rstep);
+    if (walk.rows) fetch(walk);
+    if (halves && diag) twice();
     // this wave's row steps: k0 = 4 (ks + KS s)
 #pragma unroll
     for (int st = 0; st < ROWS / (4 * KS); ++st) {
@@ -1006,6 +1102,7 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_mfma(const ColDesc *__res
     }
     __syncthreads();
   }
+  if (halves) twice();
   if constexpr (KS > 1) {
     // the waves with ks > 0 hand their sums to the tile's ks = 0 wave (the last
     // __syncthreads of the loop has freed the row tile)
@@ -1057,9 +1154,10 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_mfma(const ColDesc *__res
 // grid); KS waves share each 8 x 8 block and split its row steps.  Right
 // columns are unshared (share 0) or all shared with the first left columns
 // (share == kr).  Layout of the partials as k_gram_mfma's.
-template <int M8, int ROWS>
+template <int M8, int ROWS, bool TRI>
 __global__ __launch_bounds__(kGramThreads) void k_gram_pk(const ColDesc *__restrict__ descs, int kl, int kr,
-                                                          int share, int64_t d, double2 *__restrict__ partial) {
+                                                          int share, int64_t d, int m,
+                                                          double2 *__restrict__ partial) {
   constexpr int LD = 8 * M8 + 8 + 1;
   constexpr int KS = M8 == 1 ? 4 : (M8 == 2 ? 2 : 1);
   static_assert(ROWS % (4 * KS) == 0, "every wave takes whole row steps");
@@ -1092,16 +1190,15 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_pk(const ColDesc *__restr
       pf[p] = dc.fmt;
     }
   }
-  const int64_t r0 = int64_t(blockIdx.x) * ROWS;
-  const int64_t rstep = int64_t(gridDim.x) * ROWS;
   double2 va[PMAX][2], vb[PMAX][2];
-  auto fetch = [&](int64_t rb) {
+  auto fetch = [&](const RowWalk<ROWS, TRI> &w) {
 #pragma unroll
     for (int p = 0; p < PMAX; ++p) {
-      const int64_t row = rb + 2 * ((tid + kGramThreads * p) % HALF);
+      const int lr = 2 * ((tid + kGramThreads * p) % HALF);
+      const int64_t row = w.row + lr;
       va[p][0] = va[p][1] = vb[p][0] = vb[p][1] = make_double2(0.0, 0.0);
-      if (pa[p] != nullptr && row < d) {
-        const bool two = row + 1 < d;
+      if (pa[p] != nullptr && lr < w.rows) {
+        const bool two = lr + 1 < w.rows;
         ld_col2(pa[p], pf[p], row, two, va[p][0], va[p][1]);
         if (pb[p] != nullptr) ld_col2(pb[p], pf[p], row, two, vb[p][0], vb[p][1]);
       }
@@ -1132,11 +1229,19 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_pk(const ColDesc *__restr
   const int rj = li & 7;
   const int bcol = rj < share ? rj : 8 * M8 + (rj - share);
   const bool im = li >= 8;
-  if (r0 < d) fetch(r0);
-  for (int64_t rb = r0; rb < d; rb += rstep) {
+  bool halves = TRI;  // the sums so far count half
+  RowWalk<ROWS, TRI> walk(d, m);  // one tile ahead: the tile in flight
+  if (walk.rows) fetch(walk);
+  while (walk.rows) {
+    const bool diag = walk.diag;
+    walk.next();
     store();
     __syncthreads();
-    if (rb + rstep < d) fetch(rb + rstep);
+    if (walk.rows) fetch(walk);
+    if (halves && diag) {
+      acc += acc;
+      halves = false;
+    }
     if (tv) {
 #pragma unroll
       for (int st = 0; st < ROWS / (4 * KS); ++st) {
@@ -1148,6 +1253,7 @@ __global__ __launch_bounds__(kGramThreads) void k_gram_pk(const ColDesc *__restr
     }
     __syncthreads();
   }
+  if (halves) acc += acc;
   // every wave's 16 x 16 sums to LDS (the loop's last __syncthreads freed the
   // tile); element (i, j) of the block, i = 4 v + lk, j = li, sits at
   // [v * 64 + lane] of the wave's 256 doubles
@@ -1416,6 +1522,93 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
           st_col2(o, od.fmt, r0, ok1, out[0], out[RPL - 1]);
         else
           st_col(o, od.fmt, r0, out[0]);
+      }
+    }
+  }
+}
+
+// The combine on exchange-(anti)symmetric columns (M x M matrices, X(q, p) = sign
+// X(p, q)): a workgroup reads every input on its 32 x 32 tile (ta <= tb) only, forms
+// the outputs there and writes them to the tile and, transposed through LDS, to its
+// mirror: half the bytes of the inputs, all of the outputs'.  A thread owns two
+// entries of the tile and every output (coefficients wave-uniform, as in
+// k_combine_w); it reads all its inputs before it writes, and nobody reads a mirror
+// tile, so outputs may alias inputs.  Each output's mirror is the same value: the
+// outputs are exactly (anti)symmetric, as the inputs are.  HBM-bound: 3.6-4.6 TB/s (64
+// inputs into 10 outputs at NN = 11: 327 us).
+template <int JN, int UNR>
+__global__ __launch_bounds__(512) void k_combine_sym(const ColDesc *__restrict__ descs, int nin, int nout,
+                                                     const double2 *__restrict__ cm,
+                                                     const double2 *__restrict__ beta, int m, int nblk, int sign) {
+  int ta, tb;
+  if (!sym_tile(m, nblk, ta, tb)) return;
+  __shared__ double2 tile[2][kSymT][kSymT + 1];
+  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int p = ta * kSymT + tx, q0 = tb * kSymT + ty;  // entries (p, q0) and (p, q0 + 16)
+  const bool ok[2] = {p < m && q0 < m, p < m && q0 + 16 < m};
+  const int64_t at[2] = {p + int64_t(m) * q0, p + int64_t(m) * (q0 + 16)};
+  double ax[2][JN], ay[2][JN];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int j = 0; j < JN; ++j) ax[k][j] = ay[k][j] = 0.0;
+#pragma unroll UNR
+  for (int i = 0; i < nin; ++i) {
+    const ColDesc dc = descs[i];
+    double2 v[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      v[k] = make_double2(0.0, 0.0);
+      if (ok[k]) {
+        v[k] = ld_col(dc.a, dc.fmt, at[k]);
+        if (dc.b != nullptr) {
+          const double2 w = ld_col(dc.b, dc.fmt, at[k]);
+          v[k].x -= dc.sig_re * w.x - dc.sig_im * w.y;
+          v[k].y -= dc.sig_re * w.y + dc.sig_im * w.x;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < JN; ++j) {
+      if (j < nout) {
+        const double2 c = cm[i + size_t(nin) * j];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          ax[k][j] = fma(v[k].x, c.x, ax[k][j]);
+          ax[k][j] = fma(-v[k].y, c.y, ax[k][j]);
+          ay[k][j] = fma(v[k].x, c.y, ay[k][j]);
+          ay[k][j] = fma(v[k].y, c.x, ay[k][j]);
+        }
+      }
+    }
+  }
+  const int pm = tb * kSymT + tx, qm = ta * kSymT + ty;  // mirror entries (pm, qm) and (pm, qm + 16)
+  const double sg = double(sign);
+#pragma unroll
+  for (int j = 0; j < JN; ++j) {
+    if (j < nout) {
+      const ColDesc &od = descs[nin + j];
+      void *o = const_cast<Dbl2 *>(od.a);
+      double2 (*t)[kSymT + 1] = tile[j & 1];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        double2 r = make_double2(ax[k][j], ay[k][j]);
+        if (beta != nullptr && ok[k]) {
+          const double2 b = beta[j], ov = ld_col(o, od.fmt, at[k]);
+          r.x += b.x * ov.x - b.y * ov.y;
+          r.y += b.x * ov.y + b.y * ov.x;
+        }
+        if (ok[k]) st_col(o, od.fmt, at[k], r);
+        t[ty + 16 * k][tx] = r;
+      }
+      if (ta != tb) {
+        __syncthreads();  // the other buffer's readers are past the previous one
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const double2 r = t[tx][ty + 16 * k];
+          if (pm < m && qm + 16 * k < m)
+            st_col(o, od.fmt, pm + int64_t(m) * (qm + 16 * k), make_double2(sg * r.x, sg * r.y));
+        }
       }
     }
   }
@@ -1752,13 +1945,11 @@ int gram_blocks() { return kGramBlocks; }
 size_t gram_partial_elems(int kl, int kr) { return size_t(kGramBlocks) * kl * kr; }
 
 namespace {
-// Workgroups of k_gram_mfma<MA, NB> that fit on the device at once (LDS sets
-// it: 3 or 4 per CU), capped at kGramBlocks.  A grid of exactly that many runs
-// in one wave of workgroups; 1024 workgroups at 3 per CU would leave a second
-// round on a third of the chip.
-template <int MA, int NB, int TALL>
-int gram_grid() {
-  static std::atomic<int> cached{0};
+// Workgroups of a Gram kernel that fit on the device at once (LDS sets it: 3 or 4
+// per CU), capped at kGramBlocks, a multiple of the 8 XCDs.  A grid of exactly that
+// many runs in one wave of workgroups; 1024 workgroups at 3 per CU would leave a
+// second round on a third of the chip.
+int resident_grid(const void *kernel, std::atomic<int> &cached) {
   int grid = cached.load(std::memory_order_acquire);
   if (grid != 0) return grid;
   std::lock_guard<std::mutex> lk(g_setup_mu);
@@ -1767,24 +1958,13 @@ int gram_grid() {
   int dev = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per_cu, reinterpret_cast<const void *>(&k_gram_mfma<MA, NB, TALL>), kGramThreads, 0) != hipSuccess ||
-      cus < 1 || per_cu < 1)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kGramThreads, 0) != hipSuccess || cus < 1 ||
+      per_cu < 1)
     return kGramBlocks;
   grid = cus * per_cu < kGramBlocks ? cus * per_cu : kGramBlocks;
+  grid = grid < 8 ? 8 : grid / 8 * 8;
   cached.store(grid, std::memory_order_release);
   return grid;
-}
-
-// Tile height choice (read once): DEX_GRAM_ROWS=16 keeps 16-row tiles
-// everywhere, 64 takes up-to-64-row tiles (64 KB of LDS) for every shape;
-// otherwise 32-row tiles for single-tile Grams and 16 elsewhere.
-int gram_rows_choice() {
-  static const int rows = [] {
-    const char *v = std::getenv("DEX_GRAM_ROWS");
-    return v ? std::atoi(v) : 32;
-  }();
-  return rows;
 }
 
 // The packed narrow Gram (on unless DEX_GRAM_PK=0, read once).
@@ -1796,138 +1976,100 @@ bool gram_pk_on() {
   return on;
 }
 
-// Row-tile height of the packed Gram: 64, or DEX_PK_ROWS = 32 or 128 (read once).
-// Measured on whole NN=21 block-16 solves: 64 rows took 5-7% less Gram time
-// than 32, 128 rows 1-3% less.
-int pk_rows_choice() {
-  static const int rows = [] {
-    const char *v = std::getenv("DEX_PK_ROWS");
-    const int r = v ? std::atoi(v) : 64;
-    return r == 32 || r == 128 ? r : 64;
-  }();
-  return rows;
-}
+// Row-tile heights: 64 in the packed Gram (5-7% less time than 32 on whole NN=21
+// block-16 solves, 128 1-3% less); 32 for one-tile Grams, 16 elsewhere (gram_mfma_rows).
+constexpr int kPkRows = 64;
 
-template <int M8, int ROWS>
+template <int M8, bool TRI>
 int gram_pk_grid() {
   static std::atomic<int> cached{0};
-  int grid = cached.load(std::memory_order_acquire);
-  if (grid != 0) return grid;
-  std::lock_guard<std::mutex> lk(g_setup_mu);
-  grid = cached.load(std::memory_order_acquire);
-  if (grid != 0) return grid;
-  int dev = 0, cus = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per_cu, reinterpret_cast<const void *>(&k_gram_pk<M8, ROWS>), kGramThreads, 0) != hipSuccess ||
-      cus < 1 || per_cu < 1)
-    return kGramBlocks;
-  grid = cus * per_cu < kGramBlocks ? cus * per_cu : kGramBlocks;
-  cached.store(grid, std::memory_order_release);
-  return grid;
+  return resident_grid(reinterpret_cast<const void *>(&k_gram_pk<M8, kPkRows, TRI>), cached);
 }
 
-template <int M8, int ROWS>
-int gram_pk_launch_r(const ColDesc *descs, int kl, int kr, int share, int64_t d, double2 *partial,
-                     hipStream_t s) {
-  const int grid = gram_pk_grid<M8, ROWS>();
-  hipLaunchKernelGGL((k_gram_pk<M8, ROWS>), dim3(grid), dim3(kGramThreads), 0, s, descs, kl, kr, share, d,
-                     partial);
+template <int M8, bool TRI>
+int gram_pk_start(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, double2 *partial,
+                  hipStream_t s) {
+  const int grid = gram_pk_grid<M8, TRI>();
+  hipLaunchKernelGGL((k_gram_pk<M8, kPkRows, TRI>), dim3(grid), dim3(kGramThreads), 0, s, descs, kl, kr, share, d,
+                     m, partial);
   return grid;
 }
 
 template <int M8>
-int gram_pk_launch(const ColDesc *descs, int kl, int kr, int share, int64_t d, double2 *partial, hipStream_t s) {
-  switch (pk_rows_choice()) {
-    case 128: return gram_pk_launch_r<M8, 128>(descs, kl, kr, share, d, partial, s);
-    case 64: return gram_pk_launch_r<M8, 64>(descs, kl, kr, share, d, partial, s);
-    default: return gram_pk_launch_r<M8, 32>(descs, kl, kr, share, d, partial, s);
-  }
+int gram_pk_launch(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, double2 *partial,
+                   hipStream_t s) {
+  return m > 0 ? gram_pk_start<M8, true>(descs, kl, kr, share, d, m, partial, s)
+               : gram_pk_start<M8, false>(descs, kl, kr, share, d, m, partial, s);
 }
 
-template <int M8>
-void gram_pk_grids() {
-  const int r = pk_rows_choice();
-  if (r == 128) (void)gram_pk_grid<M8, 128>();
-  else if (r == 64) (void)gram_pk_grid<M8, 64>();
-  else (void)gram_pk_grid<M8, 32>();
+template <int MA, int NB>
+constexpr int gram_tall() {
+  return MA == 1 && NB == 1 ? 32 : 16;
+}
+
+template <int MA, int NB, bool TRI>
+int gram_grid() {
+  static std::atomic<int> cached{0};
+  return resident_grid(reinterpret_cast<const void *>(&k_gram_mfma<MA, NB, gram_tall<MA, NB>(), TRI>), cached);
+}
+
+template <int MA, int NB>
+void gram_grids() {
+  (void)gram_grid<MA, NB, false>();
+  (void)gram_grid<MA, NB, true>();
 }
 
 template <int MA>
 void gram_grids_nb() {
-  if (gram_rows_choice() == 64) {
-    (void)gram_grid<MA, 1, 64>();
-    (void)gram_grid<MA, 2, 64>();
-    (void)gram_grid<MA, 3, 64>();
-    (void)gram_grid<MA, 4, 64>();
-    (void)gram_grid<MA, 5, 64>();
-    (void)gram_grid<MA, 6, 64>();
-    (void)gram_grid<MA, 7, 64>();
-    (void)gram_grid<MA, 8, 64>();
-  }
-  (void)gram_grid<MA, 1, 16>();
-  (void)gram_grid<MA, 2, 16>();
-  (void)gram_grid<MA, 3, 16>();
-  (void)gram_grid<MA, 4, 16>();
-  (void)gram_grid<MA, 5, 16>();
-  (void)gram_grid<MA, 6, 16>();
-  (void)gram_grid<MA, 7, 16>();
-  (void)gram_grid<MA, 8, 16>();
-  if constexpr (MA == 1) (void)gram_grid<MA, 1, 32>();
+  gram_grids<MA, 1>();
+  gram_grids<MA, 2>();
+  gram_grids<MA, 3>();
+  gram_grids<MA, 4>();
+  gram_grids<MA, 5>();
+  gram_grids<MA, 6>();
+  gram_grids<MA, 7>();
+  gram_grids<MA, 8>();
+  (void)gram_pk_grid<MA, false>();
+  (void)gram_pk_grid<MA, true>();
 }
 
-// Round-robin tiles (the default) or, with DEX_GRAM_STRIDE=0 (read once), one
-// contiguous row range per workgroup.  Measured on whole NN=21 block-16 solves:
-// Gram time within 1% either way (complex128 and complex64 columns).
-bool gram_stride_on() {
-  static const bool on = [] {
-    const char *v = std::getenv("DEX_GRAM_STRIDE");
-    return !(v && std::atoi(v) == 0);
-  }();
-  return on;
-}
-
-template <int MA, int NB, int TALL>
-int gram_launch_t(const ColDesc *descs, int kl, int kr, int share, int64_t d, double2 *partial,
-                  hipStream_t s) {
-  const int grid = gram_grid<MA, NB, TALL>();
-  int64_t rpb = (d + grid - 1) / grid;
-  rpb = (rpb + 63) / 64 * 64;  // a whole number of tiles for every tile height
-  if (gram_stride_on()) rpb = 0;
-  hipLaunchKernelGGL((k_gram_mfma<MA, NB, TALL>), dim3(grid), dim3(kGramThreads), 0, s, descs, kl, kr, share,
-                     d, rpb, partial);
+template <int MA, int NB, bool TRI>
+int gram_start(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, double2 *partial,
+               hipStream_t s) {
+  const int grid = gram_grid<MA, NB, TRI>();
+  hipLaunchKernelGGL((k_gram_mfma<MA, NB, gram_tall<MA, NB>(), TRI>), dim3(grid), dim3(kGramThreads), 0, s, descs,
+                     kl, kr, share, d, m, partial);
   return grid;
 }
 
 template <int MA, int NB>
-int gram_launch(const ColDesc *descs, int kl, int kr, int share, int64_t d, double2 *partial,
+int gram_launch(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, double2 *partial,
                 hipStream_t s) {
-  const int rows = gram_rows_choice();
-  if (rows == 64) return gram_launch_t<MA, NB, 64>(descs, kl, kr, share, d, partial, s);
-  if constexpr (MA == 1 && NB == 1) {
-    if (rows != 16) return gram_launch_t<MA, NB, 32>(descs, kl, kr, share, d, partial, s);
-  }
-  return gram_launch_t<MA, NB, 16>(descs, kl, kr, share, d, partial, s);
+  return m > 0 ? gram_start<MA, NB, true>(descs, kl, kr, share, d, m, partial, s)
+               : gram_start<MA, NB, false>(descs, kl, kr, share, d, m, partial, s);
 }
 
 template <int MA>
-int gram_launch_nb(int nb, const ColDesc *descs, int kl, int kr, int share, int64_t d, double2 *partial,
+int gram_launch_nb(int nb, const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, double2 *partial,
                    hipStream_t s) {
   switch (nb) {
-    case 1: return gram_launch<MA, 1>(descs, kl, kr, share, d, partial, s);
-    case 2: return gram_launch<MA, 2>(descs, kl, kr, share, d, partial, s);
-    case 3: return gram_launch<MA, 3>(descs, kl, kr, share, d, partial, s);
-    case 4: return gram_launch<MA, 4>(descs, kl, kr, share, d, partial, s);
-    case 5: return gram_launch<MA, 5>(descs, kl, kr, share, d, partial, s);
-    case 6: return gram_launch<MA, 6>(descs, kl, kr, share, d, partial, s);
-    case 7: return gram_launch<MA, 7>(descs, kl, kr, share, d, partial, s);
-    default: return gram_launch<MA, 8>(descs, kl, kr, share, d, partial, s);
+    case 1: return gram_launch<MA, 1>(descs, kl, kr, share, d, m, partial, s);
+    case 2: return gram_launch<MA, 2>(descs, kl, kr, share, d, m, partial, s);
+    case 3: return gram_launch<MA, 3>(descs, kl, kr, share, d, m, partial, s);
+    case 4: return gram_launch<MA, 4>(descs, kl, kr, share, d, m, partial, s);
+    case 5: return gram_launch<MA, 5>(descs, kl, kr, share, d, m, partial, s);
+    case 6: return gram_launch<MA, 6>(descs, kl, kr, share, d, m, partial, s);
+    case 7: return gram_launch<MA, 7>(descs, kl, kr, share, d, m, partial, s);
+    default: return gram_launch<MA, 8>(descs, kl, kr, share, d, m, partial, s);
   }
 }
 }  // namespace
 
-hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t d, Dbl2 *partial,
+// Halves from NN = 11 on: there 290 us for a 64 x 10 Gram where all rows take 410, and the
+// Grams and combinations of two iterations of an 8 + 2 column solve 53 + 53 -> 32 + 34 ms.
+bool half_blocks(int64_t m) { return m >= kHalfMinM; }
+
+hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t d, int m, Dbl2 *partial,
                        Dbl2 *out, hipStream_t s) {
   if (kl < 1 || kr < 1 || kl > kGramMaxL || kr > kGramMaxR) return hipErrorInvalidValue;
   if (share < 0 || share > kl || share > kr) return hipErrorInvalidValue;
@@ -1936,10 +2078,10 @@ hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t 
   int nparts = 0;
   if (kr <= 8 && kl <= 32 && (share == 0 || share == kr) && gram_pk_on()) {
     switch ((kl + 7) / 8) {
-      case 1: nparts = gram_pk_launch<1>(descs, kl, kr, share, d, pp, s); break;
-      case 2: nparts = gram_pk_launch<2>(descs, kl, kr, share, d, pp, s); break;
-      case 3: nparts = gram_pk_launch<3>(descs, kl, kr, share, d, pp, s); break;
-      default: nparts = gram_pk_launch<4>(descs, kl, kr, share, d, pp, s); break;
+      case 1: nparts = gram_pk_launch<1>(descs, kl, kr, share, d, m, pp, s); break;
+      case 2: nparts = gram_pk_launch<2>(descs, kl, kr, share, d, m, pp, s); break;
+      case 3: nparts = gram_pk_launch<3>(descs, kl, kr, share, d, m, pp, s); break;
+      default: nparts = gram_pk_launch<4>(descs, kl, kr, share, d, m, pp, s); break;
     }
     const int nelem = kl * kr;
     hipLaunchKernelGGL(k_reduce_partials, dim3((nelem + 3) / 4), dim3(256), 0, s,
@@ -1948,10 +2090,10 @@ hipError_t launch_gram(const ColDesc *descs, int kl, int kr, int share, int64_t 
     return hipGetLastError();
   }
   switch (ma) {
-    case 1: nparts = gram_launch_nb<1>(nb, descs, kl, kr, share, d, pp, s); break;
-    case 2: nparts = gram_launch_nb<2>(nb, descs, kl, kr, share, d, pp, s); break;
-    case 3: nparts = gram_launch_nb<3>(nb, descs, kl, kr, share, d, pp, s); break;
-    default: nparts = gram_launch_nb<4>(nb, descs, kl, kr, share, d, pp, s); break;
+    case 1: nparts = gram_launch_nb<1>(nb, descs, kl, kr, share, d, m, pp, s); break;
+    case 2: nparts = gram_launch_nb<2>(nb, descs, kl, kr, share, d, m, pp, s); break;
+    case 3: nparts = gram_launch_nb<3>(nb, descs, kl, kr, share, d, m, pp, s); break;
+    default: nparts = gram_launch_nb<4>(nb, descs, kl, kr, share, d, m, pp, s); break;
   }
   const int nelem = kl * kr;
   hipLaunchKernelGGL(k_reduce_partials, dim3((nelem + 3) / 4), dim3(256), 0, s,
@@ -2016,6 +2158,26 @@ hipError_t launch_combine(const ColDesc *descs, int nin, int nout, const Dbl2 *c
     case 3: return combine_launch<3>(descs, nin, nout, c, beta, d, s);
     default: return combine_launch<4>(descs, nin, nout, c, beta, d, s);
   }
+}
+
+bool combine_halves(int nout) { return nout <= 16; }
+
+hipError_t launch_combine_sym(const ColDesc *descs, int nin, int nout, const Dbl2 *c, const Dbl2 *beta, int m,
+                              int sign, hipStream_t s) {
+  if (nin < 1 || nin > kCombMaxIn || nout < 1 || !combine_halves(nout)) return hipErrorInvalidValue;
+  const double2 *cc = reinterpret_cast<const double2 *>(c);
+  const double2 *bb = reinterpret_cast<const double2 *>(beta);
+  const dim3 g(unsigned(sym_grid(m))), b(kSymT, 16);
+  const int nblk = sym_blocks(m);
+  if (nout <= 4)
+    hipLaunchKernelGGL((k_combine_sym<4, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+  else if (nout <= 8)
+    hipLaunchKernelGGL((k_combine_sym<8, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+  else if (nout <= 12)
+    hipLaunchKernelGGL((k_combine_sym<12, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+  else
+    hipLaunchKernelGGL((k_combine_sym<16, 4>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+  return hipGetLastError();
 }
 
 size_t coldots_partial_elems(int k) { return size_t(kDotBlocks) * k * 4; }
@@ -2133,10 +2295,6 @@ hipError_t prepare_kernels() {
   gram_grids_nb<2>();
   gram_grids_nb<3>();
   gram_grids_nb<4>();
-  gram_pk_grids<1>();
-  gram_pk_grids<2>();
-  gram_pk_grids<3>();
-  gram_pk_grids<4>();
   return ok ? hipSuccess : hipErrorInvalidDeviceFunction;
 }
 

@@ -248,7 +248,8 @@ int dex_residuals_device(dex_ctx *ctx, const void *x_dev, const double *e, int32
  * ||(H - sigma) PX - X|| (PRECBLOCK_BASIC -> basicblocklansolve,
  * gplmr.F90:674-770, harmonic_ritz_small.F90:258-324), every column
  * multiplied.  inner_iter = 0 is an error, as in the reference (:487-489).
- * symmetry: 0, or +-1 for exchange-(anti)symmetric X. */
+ * symmetry: 0, or +-1 for exchange-(anti)symmetric X (any other X counts as
+ * Xs = (X + symmetry X^T)/2). */
 int dex_precblock_device(dex_ctx *ctx, const void *x_dev, void *px_dev, int32_t m, int32_t mb,
                          int32_t nev, double sigma_re, double sigma_im, int32_t inner_iter,
                          int32_t symmetry);
