@@ -332,8 +332,8 @@ __global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, i
 // A workgroup holds NN x NN lines of kPlaneRun entries: each thread keeps one line
 // of the first axis in registers (contracted there), the second axis goes through
 // the LDS buffers a (entries) and b (its sums), one real component at a time.
-// 32 + 48 + 48 bytes an entry over the three passes, 4.0 TB/s of them at NN = 25 in
-// FP64 (7.8 ms a vector; six passes of one axis and the potential's took 16.8), with
+// 32 + 48 + 48 bytes an entry over the three passes, 4.6 TB/s of them at NN = 25 in
+// FP64 (6.8 ms a vector; six passes of one axis and the potential's took 16.8), with
 // 8 waves a CU in flight (two workgroups: 80 KB of LDS, 205-240 registers).
 template <typename XT>
 constexpr int plane_run() {
@@ -413,6 +413,12 @@ __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane
 // |X|^2 in norms[2 blockIdx.x]: a residual needs no more of Y (112 bytes an entry over
 // the three passes where writing Y and reading it back with X took 160; 8 pairs at
 // NN = 17: 7.4 ms before).
+//
+// HBM-bound (48 bytes an entry), 4.7 TB/s at NN = 25 in FP64.  From NN = 17 on Z is read
+// while the second component still has to go through LDS, and what is known of Y is
+// summed onto it: read in the last loop, each entry's wait stood before its store
+// (NN = 25 3.02 -> 2.48 ms a launch, NN = 21 1.13 -> 0.93).  On the smaller grids that
+// costs a wave of each SIMD (registers) and 0-4%, as it would with NORMS from NN = 23 on.
 template <int NN, typename R, typename XT, typename ZT, typename YT, bool NORMS = false>
 __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(const XT *x, const ZT *z, YT *y,
                                                                              int64_t run, int64_t sa, int64_t sb,
@@ -427,7 +433,9 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
   const int64_t base = r0 + r + so * blockIdx.y + sb * bb;
   R *a = reinterpret_cast<R *>(smem) + r;
   R *b = a + N2 * P;
+  constexpr bool EARLY = NN >= 17 && !(NORMS && NN >= 23);
   R xr[NN], xi[NN], kr[NN];
+  ZT o[NN];  // EARLY: Y's sum so far, in kr's place
   if (on) {
 #pragma unroll
     for (int l = 0; l < NN; ++l) {
@@ -437,7 +445,7 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
     }
   }
   // b lines of one component through LDS, thread (r, line a = bb)
-  auto b_axis = [&](const R(&v)[NN]) {
+  auto b_lines = [&](const R(&v)[NN]) {
     if (on) {
 #pragma unroll
       for (int l = 0; l < NN; ++l) a[(l * NN + bb) * P] = v[l];
@@ -449,26 +457,56 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
       for (int l = 0; l < NN; ++l) t[l] = a[(bb * NN + l) * P];
       line_apply<NN, R>(t, [&](int l, R s) { b[(bb * NN + l) * P] = s; });
     }
-    __syncthreads();
   };
-  b_axis(xr);
-  if (on) line_apply<NN, R>(xr, [&](int l, R s) { kr[l] = s + b[(l * NN + bb) * P]; });
-  b_axis(xi);
+  const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
   double rr = 0.0, xx = 0.0;
+  b_lines(xr);
+  if constexpr (EARLY) {
+    if (on) {
+#pragma unroll
+      for (int l = 0; l < NN; ++l) o[l] = z[base + sa * l];
+    }
+  }
+  __syncthreads();
   if (on) {
-    const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
+    line_apply<NN, R>(xr, [&](int l, R s) {
+      kr[l] = s + b[(l * NN + bb) * P];
+      if constexpr (EARLY) {
+        o[l].x += s2r * kr[l];
+        o[l].y += s2i * kr[l];
+        if constexpr (NORMS) {
+          o[l].x -= e_re * xr[l];
+          o[l].y -= e_im * xr[l];
+          xx += double(xr[l]) * xr[l];
+        }
+      }
+    });
+  }
+  b_lines(xi);
+  __syncthreads();
+  if (on) {
     line_apply<NN, R>(xi, [&](int l, R s) {
       const R ki = s + b[(l * NN + bb) * P];
-      const ZT zv = z[base + sa * l];
-      YT o;
-      o.x = zv.x + (s2r * kr[l] - s2i * ki);
-      o.y = zv.y + (s2r * ki + s2i * kr[l]);
-      if constexpr (NORMS) {
-        const double dr = o.x - (e_re * xr[l] - e_im * xi[l]), di = o.y - (e_re * xi[l] + e_im * xr[l]);
-        rr += dr * dr + di * di;
-        xx += double(xr[l]) * xr[l] + double(xi[l]) * xi[l];
+      YT out;
+      if constexpr (EARLY) {
+        out.x = o[l].x - s2i * ki;
+        out.y = o[l].y + s2r * ki;
       } else {
-        y[base + sa * l] = o;
+        const ZT zv = z[base + sa * l];
+        out.x = zv.x + (s2r * kr[l] - s2i * ki);
+        out.y = zv.y + (s2r * ki + s2i * kr[l]);
+      }
+      if constexpr (NORMS) {
+        if constexpr (!EARLY) {
+          out.x -= e_re * xr[l];
+          out.y -= e_im * xr[l];
+          xx += double(xr[l]) * xr[l];
+        }
+        const double dr = out.x + e_im * xi[l], di = out.y - e_re * xi[l];
+        rr += dr * dr + di * di;
+        xx += double(xi[l]) * xi[l];
+      } else {
+        y[base + sa * l] = out;
       }
     });
   }
