@@ -370,17 +370,25 @@ int batch_cols(const dex_ctx *c, int io, int left) {
   return launches > 1 ? (left + launches - 1) / launches : left;
 }
 
-// H on one column, or with sym = +-1 (X = sym X^T) on up to dex::kBatchMax
+// What the passes of H - shift read beside the vectors.
+dex::PotArgs pot_args(const dex_ctx *c, cd shift) {
+  dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  pot.cf.sh_re = shift.real();
+  pot.cf.sh_im = shift.imag();
+  return pot;
+}
+
+// H - shift on one column, or with sym = +-1 (X = sym X^T) on up to dex::kBatchMax
 // columns, by the LDS kernels.  io: kIoF64 (complex128, FP64), kIoMixed
 // (complex128, FP32 arithmetic) or kIoF32 (complex64 columns, FP32).  u: the
 // general form's intermediate.  pass_events: also record c->ev[0..2] around the
 // passes (the matvec entry point's per-pass timing).
 int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int ncols, int sym, void *u,
-                bool pass_events = false) {
+                bool pass_events = false, cd shift = 0.0) {
   const double dd = double(c->d) * ncols, nn = double(c->nn);
   const double xb = io == dex::kIoF32 ? 8.0 : 16.0;               // X and Y entry bytes
   const double zb = sym != 0 ? xb : (io == dex::kIoF64 ? 16.0 : 8.0);  // Z entry bytes
-  const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  const dex::PotArgs pot = pot_args(c, shift);
   const bool planes = sym == 0 && dex::general_by_planes(c->nn);
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[0], c->stream));
   {
@@ -406,31 +414,31 @@ int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int nc
   return 0;
 }
 
-// H on columns that have the LDS kernels, a batch per pair of launches.  General
+// H - shift on columns that have the LDS kernels, a batch per pair of launches.  General
 // columns must be consecutive (x[j], y[j] at D entries from x[j - 1], y[j - 1]).
-int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, int io, int sym) {
+int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, int io, int sym, cd shift = 0.0) {
   if (ncols < 0 || !(io != dex::kIoF64 ? c->fast32 : c->fast64))
     return fail(DEX_EINVAL, "batched matvec: bad column count or form");
   for (int j = 0, k = 0; j < ncols; j += k) {
     k = sym != 0 ? batch_cols(c, io, ncols - j) : general_cols(c, io, ncols - j);
     if (sym == 0)
       if (int st = ensure_u(c, k, io)) return st;
-    if (int st = fast_passes(c, io, x + j, y + j, k, sym, c->d_u)) return st;
+    if (int st = fast_passes(c, io, x + j, y + j, k, sym, c->d_u, false, shift)) return st;
   }
   return 0;
 }
 
-// H on one complex128 column in FP64 with the intermediate in Y's own storage
+// H - shift on one complex128 column in FP64 with the intermediate in Y's own storage
 // (grids without an FP64 cube; x and y must differ).
-int generic_passes(dex_ctx *c, const void *x, void *y) {
-  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, {c->d_vn, c->d_tinv, c->coef}, c->stream));
+int generic_passes(dex_ctx *c, const void *x, void *y, cd shift = 0.0) {
+  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, pot_args(c, shift), c->stream));
   DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, 1, c->coef, c->stream));
   return 0;
 }
 
-// One application of H on complex128 device vectors; `single` selects FP32
+// One application of H - shift on complex128 device vectors; `single` selects FP32
 // arithmetic (complex128 in and out).
-int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool pass_events = false) {
+int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool pass_events = false, cd shift = 0.0) {
   const bool fast = single ? c->fast32 : c->fast64;
   if (single && !fast) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
   if (fast) {
@@ -439,10 +447,10 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
     const void *xp = x;
     void *yp = y;
     return fast_passes(c, single ? dex::kIoMixed : dex::kIoF64, &xp, &yp, 1, sym, c->d_u,
-                       pass_events && c->timing);
+                       pass_events && c->timing, shift);
   }
   KTimer kt(c, DEX_K_GENERIC, 32.0 * double(c->d), (24.0 * c->nn + 14.0) * double(c->d));
-  if (int st = generic_passes(c, x, y)) return st;
+  if (int st = generic_passes(c, x, y, shift)) return st;
   // The general operator carries the rounding-level exchange-odd (even) part of
   // an exchange-even (odd) x into y, where the transpose-add kernels, which the
   // mixed form applies to its complex64 blocks, drop it: in a solve that mixes
@@ -454,14 +462,14 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
   return 0;
 }
 
-// H on complex64 device vectors in FP32 arithmetic (x, y hold D complex64).
-int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym, bool pass_events = false) {
+// H - shift on complex64 device vectors in FP32 arithmetic (x, y hold D complex64).
+int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym, bool pass_events = false, cd shift = 0.0) {
   if (!c->fast32) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
   if (sym == 0)
     if (int st = ensure_u(c)) return st;
   const void *xp = x;
   void *yp = y;
-  return fast_passes(c, dex::kIoF32, &xp, &yp, 1, sym, c->d_u, pass_events && c->timing);
+  return fast_passes(c, dex::kIoF32, &xp, &yp, 1, sym, c->d_u, pass_events && c->timing, shift);
 }
 
 // ---- block helpers on one context ------------------------------------------
@@ -1035,7 +1043,7 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
   DEX_HIP(hipSetDevice(c->p.device));
   const int io = sp ? dex::kIoF32 : (f32 ? dex::kIoMixed : dex::kIoF64);
   const size_t xb = sp ? 8 : 16;  // bytes per entry of X and Y
-  const dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
+  const dex::PotArgs pot = pot_args(c, 0.0);
   const bool single_file = chained(in, out, size_t(howmany) * size_t(c->d) * xb);
   for (int j = 0, k = 0; j < howmany; j += k) {
     k = !fast || single_file ? 1 : symmetry != 0 ? batch_cols(c, io, howmany - j) : general_cols(c, io, howmany - j);
@@ -1197,9 +1205,9 @@ struct Solver {
   std::vector<Dbl2 *> pool;    // free complex128 work vectors
   std::vector<Dbl2 *> pool32;  // free complex64 work vectors (tagged pointers)
 
-  // H on every column of `in` into `out`.  complex128 columns get the FP64
+  // H - shift on every column of `in` into `out`.  complex128 columns get the FP64
   // matvec, complex64 columns (both sides) the FP32 one.
-  int matblock(const Block &in, const Block &out) {
+  int matblock(const Block &in, const Block &out, cd shift = 0.0) {
     const double t0 = now_s();
     if (out.size() < in.size()) return fail(DEX_EINVAL, "matblock: output block too small");
     bool same = true;
@@ -1214,7 +1222,8 @@ struct Solver {
         xi.push_back(untag(in.cols[j]));
         yo.push_back(untag(out.cols[j]));
       }
-      if (int st = apply_h_batch(c, xi.data(), yo.data(), in.size(), lo ? dex::kIoF32 : dex::kIoF64, sym)) return st;
+      if (int st = apply_h_batch(c, xi.data(), yo.data(), in.size(), lo ? dex::kIoF32 : dex::kIoF64, sym, shift))
+        return st;
       matvecs += in.size();
       t_matvec += now_s() - t0;
       return 0;
@@ -1222,8 +1231,8 @@ struct Solver {
     for (int j = 0; j < in.size(); ++j) {
       if (is32(in.cols[j]) != is32(out.cols[j])) return fail(DEX_EINVAL, "matblock: mixed storage formats");
       if (is32(in.cols[j])) {
-        if (int st = apply_h32(c, untag(in.cols[j]), untag(out.cols[j]), sym)) return st;
-      } else if (int st = apply_h(c, in.cols[j], out.cols[j], false, sym)) {
+        if (int st = apply_h32(c, untag(in.cols[j]), untag(out.cols[j]), sym, false, shift)) return st;
+      } else if (int st = apply_h(c, in.cols[j], out.cols[j], false, sym, false, shift)) {
         return st;
       }
       ++matvecs;
@@ -1479,7 +1488,7 @@ struct Solver {
   // 0.5 is the criterion of Daniel, Gragg, Kaufman and Stewart (Math. Comp. 30
   // (1976) 772-795); the subtraction loses about eps / keep of relative
   // accuracy in R, so a smaller keep_min trades orthogonality for a pass.  q
-  // must be orthonormal.  The input is `wd` (descriptors: plain columns or a - sigma b),
+  // must be orthonormal.  The input is `wd` (plain descriptors),
   // the result goes to `w` (which may be the storage wd reads).  On success
   // `cq` and `r` satisfy w_in = q cq + w_out r; `ok` is false when the
   // projected block is numerically rank deficient (then w holds the projected,
@@ -1631,14 +1640,14 @@ struct Solver {
       Block hq;
       hq.fmt = bf;
       if (int st = grow(hq, kb)) return st;
-      if (int st = matblock(qj, hq)) return st;
-      std::vector<ColDesc> wd;
-      for (int i = 0; i < kb; ++i) wd.push_back(shifted(hq.cols[i], qj.cols[i], sigma));
+      // the matvec applies the shift: formed by the Grams and combinations as
+      // H Q_j - sigma Q_j, Q_j went through each of them a second time
+      if (int st = matblock(qj, hq, sigma)) return st;
       std::vector<cd> cj, rj;
       const bool last = j == m - 1;
       // a preconditioner's basis: one pass unless the projection cancels
       // more than 99.9% of a column (R keeps ~1e-13 relative accuracy)
-      if (int st = cgs_cholqr(qall, wd, hq, cj, rj, ok, !last, 1e-3)) return st;
+      if (int st = cgs_cholqr(qall, descs_of(hq), hq, cj, rj, ok, !last, 1e-3)) return st;
       if (!ok) rj.assign(size_t(kb) * kb, 0.0);  // (H - sigma) Q_j lies in span(Q): the space is exhausted
       hc.push_back(cj);
       hr.push_back(rj);

@@ -138,7 +138,7 @@ __device__ __forceinline__ void plane_axes(const R (&x)[NN], R *__restrict__ a, 
 }
 
 // Electron-1 pass on the cube of electron-2 index q = blockIdx.x (contiguous) of
-// column blockIdx.y: Z = s2 tau3D X + w c1 Vr o X.  w = 1/2 for
+// column blockIdx.y: Z = s2 tau3D X + w (c1 Vr - shift) o X.  w = 1/2 for
 // exchange-(anti)symmetric vectors (Y = Z + sign Z^T follows, k_symfold), 1 for
 // general ones (Y = Z + s2 K2 X follows, k_pass2).  A workgroup reads its whole
 // cube before it writes, so Z may be X's own storage.
@@ -177,6 +177,7 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtr
   plane_axes<NN, R>(xi, a, b, c);
   if (on) {
     const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(w * cf.c1_re), c1i = R(w * cf.c1_im);
+    const R shr = R(w * cf.sh_re), shi = R(w * cf.sh_im);
     const int iq = q % NN, jq = (q / NN) % NN, kq = q / N2;
     const int t0 = (iq - c % NN + NN) + L * ((jq - c / NN + NN) + L * (kq + NN));
     const double vq = vn[q];
@@ -184,10 +185,10 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtr
     line_apply<NN, R>(xi, [&](int k, R y) {
       const R ki = y + b[c + N2 * k];
       const R vr = R(vn[c + N2 * k] + vq + tinv[t0 - L * L * k] * cf.inv_d3);
-      const R vxr = vr * xr[k], vxi = vr * xi[k];
+      const R vcr = c1r * vr - shr, vci = c1i * vr - shi;
       ZT o;
-      o.x = s2r * kr[k] - s2i * ki + c1r * vxr - c1i * vxi;
-      o.y = s2r * ki + s2i * kr[k] + c1r * vxi + c1i * vxr;
+      o.x = s2r * kr[k] - s2i * ki + vcr * xr[k] - vci * xi[k];
+      o.y = s2r * ki + s2i * kr[k] + vcr * xi[k] + vci * xr[k];
       zq[c + N2 * k] = o;
     });
   }
@@ -344,7 +345,7 @@ constexpr int plane1_planes() {
   return NN >= 9 ? 8 : 16;  // i1 x j1 planes of a workgroup
 }
 
-// Axes i1 and j1 and the potential: Z = s2 (tau x 1 + 1 x tau) X + w c1 Vr o X.
+// Axes i1 and j1 and the potential: Z = s2 (tau x 1 + 1 x tau) X + (c1 Vr - shift) o X.
 // blockIdx: electron-2 index q, group of kp = plane1_planes() planes k1.  Thread (i, g) keeps the
 // j line of plane g.
 template <int NN, typename R, typename XT, typename ZT>
@@ -388,16 +389,17 @@ __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane
   i_axis(xi);
   if (on) {
     const R s2r = R(cf.s2_re), s2i = R(cf.s2_im), c1r = R(cf.c1_re), c1i = R(cf.c1_im);
+    const R shr = R(cf.sh_re), shi = R(cf.sh_im);
     const int iq = q % NN, jq = (q / NN) % NN, kq = q / N2;
     const int t0 = (iq - i + NN) + L * ((jq + NN) + L * (kq - k + NN));
     const double vq = vn[q];
     line_apply<NN, R>(xi, [&](int j, R y) {
       const R ki = y + b[NN * j + i];
       const R vr = R(vn[N2 * k + NN * j + i] + vq + tinv[t0 - L * j] * cf.inv_d3);
-      const R vxr = vr * xr[j], vxi = vr * xi[j];
+      const R vcr = c1r * vr - shr, vci = c1i * vr - shi;
       ZT o;
-      o.x = s2r * kr[j] - s2i * ki + c1r * vxr - c1i * vxi;
-      o.y = s2r * ki + s2i * kr[j] + c1r * vxi + c1i * vxr;
+      o.x = s2r * kr[j] - s2i * ki + vcr * xr[j] - vci * xi[j];
+      o.y = s2r * ki + s2i * kr[j] + vcr * xi[j] + vci * xr[j];
       z[base + NN * j] = o;
     });
   }
@@ -1374,30 +1376,24 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
   }
   // element p of this thread: row pair e % HALF of input column e / HALF
   const void *pa[PMAX];
-  const void *pb[PMAX];
   int pf[PMAX];
 #pragma unroll
   for (int p = 0; p < PMAX; ++p) {
     const int e = tid + kCombThreads * p;
     pa[p] = nullptr;
-    pb[p] = nullptr;
     pf[p] = 0;
     if (e < HALF * nin) {
       const ColDesc &dc = descs[e / HALF];
       pa[p] = dc.a;
-      pb[p] = dc.b;
       pf[p] = dc.fmt;
     }
   }
-  double2 va[PMAX][2], vb[PMAX][2];
+  double2 va[PMAX][2];
   auto fetch = [&](int64_t rb) {
 #pragma unroll
     for (int p = 0; p < PMAX; ++p) {
       const int64_t r = rb + 2 * ((tid + kCombThreads * p) % HALF);
-      if (pa[p] != nullptr && r < d) {
-        ld_col2(pa[p], pf[p], r, r + 1 < d, va[p][0], va[p][1]);
-        if (pb[p] != nullptr) ld_col2(pb[p], pf[p], r, r + 1 < d, vb[p][0], vb[p][1]);
-      }
+      if (pa[p] != nullptr && r < d) ld_col2(pa[p], pf[p], r, r + 1 < d, va[p][0], va[p][1]);
     }
   };
   const int64_t ntile = (d + kCombRows - 1) / kCombRows;
@@ -1413,14 +1409,7 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
       const int r = 2 * (e % HALF), c = e / HALF;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (r + h >= nr) continue;
-        double2 v = va[p][h];
-        if (pb[p] != nullptr) {
-          const ColDesc &dc = descs[c];
-          v.x -= dc.sig_re * vb[p][h].x - dc.sig_im * vb[p][h].y;
-          v.y -= dc.sig_re * vb[p][h].y + dc.sig_im * vb[p][h].x;
-        }
-        tin[c * kCombRows + r + h] = v;
+        if (r + h < nr) tin[c * kCombRows + r + h] = va[p][h];
       }
     }
     __syncthreads();
@@ -1503,21 +1492,8 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
       if (ok0) {
         if constexpr (RPL == 2) {
           ld_col2(dc.a, dc.fmt, r0, ok1, v[0], v[RPL - 1]);
-          if (dc.b != nullptr) {
-            double2 b0, b1;
-            ld_col2(dc.b, dc.fmt, r0, ok1, b0, b1);
-            v[0].x -= dc.sig_re * b0.x - dc.sig_im * b0.y;
-            v[0].y -= dc.sig_re * b0.y + dc.sig_im * b0.x;
-            v[RPL - 1].x -= dc.sig_re * b1.x - dc.sig_im * b1.y;
-            v[RPL - 1].y -= dc.sig_re * b1.y + dc.sig_im * b1.x;
-          }
         } else {
           v[0] = ld_col(dc.a, dc.fmt, r0);
-          if (dc.b != nullptr) {
-            const double2 vb = ld_col(dc.b, dc.fmt, r0);
-            v[0].x -= dc.sig_re * vb.x - dc.sig_im * vb.y;
-            v[0].y -= dc.sig_re * vb.y + dc.sig_im * vb.x;
-          }
         }
       }
 #pragma unroll
@@ -1597,14 +1573,7 @@ __global__ __launch_bounds__(512) void k_combine_sym(const ColDesc *__restrict__
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       v[k] = make_double2(0.0, 0.0);
-      if (ok[k]) {
-        v[k] = ld_col(dc.a, dc.fmt, at[k]);
-        if (dc.b != nullptr) {
-          const double2 w = ld_col(dc.b, dc.fmt, at[k]);
-          v[k].x -= dc.sig_re * w.x - dc.sig_im * w.y;
-          v[k].y -= dc.sig_re * w.y + dc.sig_im * w.x;
-        }
-      }
+      if (ok[k]) v[k] = ld_col(dc.a, dc.fmt, at[k]);
     }
 #pragma unroll
     for (int j = 0; j < JN; ++j) {
