@@ -519,6 +519,11 @@ double distinct_entry_bytes(const std::vector<ColDesc> &ds, size_t n) {
   return b;
 }
 
+// Every column is complex128 and stands for itself: the block kernels' direct form.
+bool all_complex128(const std::vector<ColDesc> &ds) {
+  return std::all_of(ds.begin(), ds.end(), [](const ColDesc &d) { return d.a && !d.b && d.fmt == 0; });
+}
+
 // sym (in the block operations below): 0, or +-1 where every column involved is an
 // exchange-symmetric (antisymmetric) vector: its two halves are each other's mirror
 // images, so Grams and combinations read one (half_blocks grids).
@@ -626,11 +631,15 @@ int combine(dex_ctx *c, const std::vector<ColDesc> &in, const std::vector<Dbl2 *
   if (int(ds.size()) > kMaxDesc) return fail(DEX_EINVAL, "too many block columns");
   // descriptors | C | beta in one image, one copy
   const size_t bd = (ds.size() * sizeof(ColDesc) + 255) / 256 * 256;
-  const size_t bc = (cm.size() * sizeof(Dbl2) + 255) / 256 * 256;
+  const int ld = dex::combine_ld(nout);  // C goes row by row
+  if (nin * ld > kMaxSmall) return fail(DEX_EINVAL, "combine matrix size");
+  const size_t bc = (size_t(nin) * ld * sizeof(Dbl2) + 255) / 256 * 256;
   const size_t bb = beta ? beta->size() * sizeof(Dbl2) : 0;
   std::vector<unsigned char> img(bd + bc + bb);
   std::memcpy(img.data(), ds.data(), ds.size() * sizeof(ColDesc));
-  std::memcpy(img.data() + bd, cm.data(), cm.size() * sizeof(Dbl2));
+  cd *rows_c = reinterpret_cast<cd *>(img.data() + bd);
+  for (int j = 0; j < nout; ++j)
+    for (int i = 0; i < nin; ++i) rows_c[size_t(ld) * i + j] = cm[i + size_t(nin) * j];
   if (beta) std::memcpy(img.data() + bd + bc, beta->data(), bb);
   DEX_HIP(stage_upload(c, c->d_args, img.data(), img.size()));
   const bool half = sym != 0 && dex::half_blocks(c->m) && dex::combine_halves(nout);
@@ -641,10 +650,11 @@ int combine(dex_ctx *c, const std::vector<ColDesc> &in, const std::vector<Dbl2 *
   const auto *dd = reinterpret_cast<const ColDesc *>(c->d_args);
   const Dbl2 *dc = reinterpret_cast<const Dbl2 *>(c->d_args + bd);
   const Dbl2 *dbeta = beta ? reinterpret_cast<const Dbl2 *>(c->d_args + bd + bc) : nullptr;
+  const bool plain = all_complex128(ds);
   if (half)
-    DEX_HIP(dex::launch_combine_sym(dd, nin, nout, dc, dbeta, int(c->m), sym, c->stream));
+    DEX_HIP(dex::launch_combine_sym(dd, nin, nout, dc, dbeta, int(c->m), sym, plain, c->stream));
   else
-    DEX_HIP(dex::launch_combine(dd, nin, nout, dc, dbeta, c->d, c->stream));
+    DEX_HIP(dex::launch_combine(dd, nin, nout, dc, dbeta, c->d, plain, c->stream));
   return 0;
 }
 

@@ -126,16 +126,17 @@ bool half_blocks(int64_t m);
 
 // out_j = beta_j out_j + sum_i in_i C(i, j) row by row; in-place aliasing of
 // an output with an input is allowed.  `descs`: nin input descriptors then
-// nout output pointers (as ColDesc.a); C (nin x nout) and beta (nout, may be
-// null) are device arrays.  nin <= 64, nout <= 48.
+// nout output pointers (as ColDesc.a); C (nin rows of combine_ld(nout), zeros beyond
+// nout) and beta (nout, may be null) are device arrays.  nin <= 64, nout <= 48.  plain: every column is complex128.
+int combine_ld(int nout);
 hipError_t launch_combine(const ColDesc *descs, int nin, int nout, const Dbl2 *c,
-                          const Dbl2 *beta, int64_t d, hipStream_t s);
+                          const Dbl2 *beta, int64_t d, bool plain, hipStream_t s);
 
 // launch_combine on columns that all are exchange-symmetric (sign 1) or antisymmetric
 // (-1) M x M matrices, inputs read on one side of the diagonal; where combine_halves.
 bool combine_halves(int nout);
 hipError_t launch_combine_sym(const ColDesc *descs, int nin, int nout, const Dbl2 *c, const Dbl2 *beta, int m,
-                              int sign, hipStream_t s);
+                              int sign, bool plain, hipStream_t s);
 
 // Per column j: sum |a_j|^2, sum conj(a_j) b_j, sum |b_j|^2 (b from descs[k + j]).
 size_t coldots_partial_elems(int k);

@@ -1372,7 +1372,7 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
   const int grp = tid / kCombRows;
   for (int e = tid; e < nin * NP; e += kCombThreads) {
     const int i = e / NP, j = e % NP;
-    sc[e] = j < nout ? cm[i + size_t(nin) * j] : make_double2(0.0, 0.0);
+    sc[e] = j < nout ? cm[size_t(nout) * i + j] : make_double2(0.0, 0.0);
   }
   // element p of this thread: row pair e % HALF of input column e / HALF
   const void *pa[PMAX];
@@ -1452,6 +1452,52 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
   }
 }
 
+// a_k += v_k C(i, .) over the JN outputs (c: C(i, 0), C stored by rows of JN).
+template <int JN, int RPL>
+__device__ __forceinline__ void add_products(const double2 (&v)[RPL], const double2 *__restrict__ c,
+                                             double (&ax)[RPL][JN], double (&ay)[RPL][JN]) {
+#pragma unroll
+  for (int q = 0; q < JN; ++q) {
+    const double2 f = c[q];
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) {
+      ax[k][q] = fma(v[k].x, f.x, ax[k][q]);
+      ax[k][q] = fma(-v[k].y, f.y, ax[k][q]);
+      ay[k][q] = fma(v[k].x, f.y, ay[k][q]);
+      ay[k][q] = fma(v[k].y, f.x, ay[k][q]);
+    }
+  }
+}
+
+// The same over complex128 inputs at the entries `at`: UNR inputs are loaded while the
+// UNR before them are used.
+template <int JN, int RPL, int UNR>
+__device__ __forceinline__ void plain_inputs(const ColDesc *__restrict__ descs, int nin,
+                                             const double2 *__restrict__ cm, const int64_t (&at)[2],
+                                             double (&ax)[RPL][JN], double (&ay)[RPL][JN]) {
+  double2 v[UNR][RPL], next[UNR][RPL];
+  auto load = [&](int i, double2(&w)[UNR][RPL]) {
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const double2 *a = reinterpret_cast<const double2 *>(descs[i + u < nin ? i + u : nin - 1].a);
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) w[u][k] = a[at[k]];
+    }
+  };
+  load(0, v);
+  for (int i = 0; i < nin; i += UNR) {
+    load(i + UNR, next);
+    __builtin_amdgcn_sched_barrier(0);  // else the loads sink to their uses
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+      if (i + u < nin) add_products<JN, RPL>(v[u], cm + size_t(JN) * (i + u), ax, ay);
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) v[u][k] = next[u][k];
+  }
+}
+
 // The combine for narrow outputs (nout <= 16; also 33..48, where the LDS
 // kernel's staging would exceed 64 KB per workgroup), without LDS: a wavefront
 // owns 64 * RPL consecutive rows and every output column of them, so the
@@ -1463,11 +1509,19 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
 // with one complex64 row per lane the loads were 8 bytes wide and the kernel
 // moved half the bytes per instruction.  With RPL = 1 a lane owns one row.
 // JN, the output width the registers hold, is the smallest of 4, 8, 12, 16, 48
-// that covers nout: spare accumulators cost occupancy.  UNR inputs are
-// unrolled.  All inputs of a row are read before any output of it is written,
-// so outputs may alias inputs.  Columns start 256-byte aligned and row pairs
-// start at even rows, so the 16-byte accesses are aligned.
-template <int JN, int RPL, int UNR>
+// that covers nout: spare accumulators cost occupancy.  C comes by rows of JN, zeros
+// past nout, so an input's coefficients are a few wide scalar loads without a branch
+// (by columns they were one load and one branch an output: two iterations of an 8 + 2
+// column solve at NN = 9 took 51 ms, now 48).  All inputs of a row are read before any
+// output of it is written, so outputs may alias inputs.  Columns start 256-byte
+// aligned and row pairs start at even rows, so the 16-byte accesses are aligned.
+//
+// PLAIN: every column is complex128.  A lane's rows are then 64 apart (each load of a
+// wavefront is one 1 KB run) and UNR inputs are loaded while the UNR before them are
+// used; with a branch on each column's format the loads of one input waited for the
+// products of the one before.  UNR is what measured fastest, loads in flight against
+// wavefronts a SIMD: 8, 4 and 1 inputs for 4, 8 and 12 outputs.
+template <int JN, int RPL, int UNR, bool PLAIN>
 __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ descs, int nin, int nout,
                                                    const double2 *__restrict__ cm,
                                                    const double2 *__restrict__ beta, int64_t d) {
@@ -1476,38 +1530,32 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
   const int64_t wave = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t stride = int64_t(gridDim.x) * 4 * 64 * RPL;
   for (int64_t rb = wave * 64 * RPL; rb < d; rb += stride) {
-    const int64_t r0 = rb + RPL * lane;  // this lane's first row
-    const bool ok0 = r0 < d, ok1 = RPL == 2 && r0 + 1 < d;
+    const int64_t r0 = rb + (PLAIN ? 1 : RPL) * lane;  // this lane's first row
+    const bool ok0 = r0 < d, ok1 = RPL == 2 && r0 + (PLAIN ? 64 : 1) < d;
     double ax[RPL][JN], ay[RPL][JN];
 #pragma unroll
     for (int k = 0; k < RPL; ++k)
 #pragma unroll
       for (int q = 0; q < JN; ++q) ax[k][q] = ay[k][q] = 0.0;
+    if constexpr (PLAIN) {
+      // rows past the end read row 0 and are not written
+      const int64_t at[2] = {ok0 ? r0 : 0, ok1 ? r0 + 64 : 0};
+      plain_inputs<JN, RPL, UNR>(descs, nin, cm, at, ax, ay);
+    } else {
 #pragma unroll UNR
-    for (int i = 0; i < nin; ++i) {
-      const ColDesc dc = descs[i];
-      double2 v[RPL];
+      for (int i = 0; i < nin; ++i) {
+        const ColDesc dc = descs[i];
+        double2 v[RPL];
 #pragma unroll
-      for (int k = 0; k < RPL; ++k) v[k] = make_double2(0.0, 0.0);
-      if (ok0) {
-        if constexpr (RPL == 2) {
-          ld_col2(dc.a, dc.fmt, r0, ok1, v[0], v[RPL - 1]);
-        } else {
-          v[0] = ld_col(dc.a, dc.fmt, r0);
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < JN; ++q) {
-        if (q < nout) {
-          const double2 c = cm[i + size_t(nin) * q];
-#pragma unroll
-          for (int k = 0; k < RPL; ++k) {
-            ax[k][q] = fma(v[k].x, c.x, ax[k][q]);
-            ax[k][q] = fma(-v[k].y, c.y, ax[k][q]);
-            ay[k][q] = fma(v[k].x, c.y, ay[k][q]);
-            ay[k][q] = fma(v[k].y, c.x, ay[k][q]);
+        for (int k = 0; k < RPL; ++k) v[k] = make_double2(0.0, 0.0);
+        if (ok0) {
+          if constexpr (RPL == 2) {
+            ld_col2(dc.a, dc.fmt, r0, ok1, v[0], v[RPL - 1]);
+          } else {
+            v[0] = ld_col(dc.a, dc.fmt, r0);
           }
         }
+        add_products<JN, RPL>(v, cm + size_t(JN) * i, ax, ay);
       }
     }
     if (!ok0) continue;
@@ -1522,20 +1570,32 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
         if (beta != nullptr) {
           const double2 bq = beta[q];
           double2 ov[RPL];
-          if constexpr (RPL == 2)
+          if constexpr (PLAIN) {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k)
+              ov[k] = static_cast<const double2 *>(o)[k == 0 || ok1 ? r0 + 64 * k : r0];
+          } else if constexpr (RPL == 2) {
             ld_col2(o, od.fmt, r0, ok1, ov[0], ov[RPL - 1]);
-          else
+          } else {
             ov[0] = ld_col(o, od.fmt, r0);
+          }
 #pragma unroll
           for (int k = 0; k < RPL; ++k) {
             out[k].x += bq.x * ov[k].x - bq.y * ov[k].y;
             out[k].y += bq.x * ov[k].y + bq.y * ov[k].x;
           }
         }
-        if constexpr (RPL == 2)
+        if constexpr (PLAIN) {
+          double2 *w = static_cast<double2 *>(o) + r0;
+          w[0] = out[0];
+          if constexpr (RPL == 2) {
+            if (ok1) w[64] = out[1];
+          }
+        } else if constexpr (RPL == 2) {
           st_col2(o, od.fmt, r0, ok1, out[0], out[RPL - 1]);
-        else
+        } else {
           st_col(o, od.fmt, r0, out[0]);
+        }
       }
     }
   }
@@ -1548,9 +1608,10 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
 // entries of the tile and every output (coefficients wave-uniform, as in
 // k_combine_w); it reads all its inputs before it writes, and nobody reads a mirror
 // tile, so outputs may alias inputs.  Each output's mirror is the same value: the
-// outputs are exactly (anti)symmetric, as the inputs are.  HBM-bound: 3.6-4.6 TB/s (64
-// inputs into 10 outputs at NN = 11: 327 us).
-template <int JN, int UNR>
+// outputs are exactly (anti)symmetric, as the inputs are.  HBM-bound: 5.0 TB/s at 10
+// outputs of NN = 11 (two iterations of an 8 + 2 column solve: 34.7 -> 29.9 ms of
+// these), 4.5 at 4 outputs of NN = 21 (an order-4 inner solve: 16.8 -> 15.5 ms).
+template <int JN, int UNR, bool PLAIN>
 __global__ __launch_bounds__(512) void k_combine_sym(const ColDesc *__restrict__ descs, int nin, int nout,
                                                      const double2 *__restrict__ cm,
                                                      const double2 *__restrict__ beta, int m, int nblk, int sign) {
@@ -1566,27 +1627,21 @@ __global__ __launch_bounds__(512) void k_combine_sym(const ColDesc *__restrict__
   for (int k = 0; k < 2; ++k)
 #pragma unroll
     for (int j = 0; j < JN; ++j) ax[k][j] = ay[k][j] = 0.0;
+  if constexpr (PLAIN) {
+    // entries past the edge read entry 0 and are not written
+    const int64_t from[2] = {ok[0] ? at[0] : 0, ok[1] ? at[1] : 0};
+    plain_inputs<JN, 2, UNR>(descs, nin, cm, from, ax, ay);
+  } else {
 #pragma unroll UNR
-  for (int i = 0; i < nin; ++i) {
-    const ColDesc dc = descs[i];
-    double2 v[2];
+    for (int i = 0; i < nin; ++i) {
+      const ColDesc dc = descs[i];
+      double2 v[2];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      v[k] = make_double2(0.0, 0.0);
-      if (ok[k]) v[k] = ld_col(dc.a, dc.fmt, at[k]);
-    }
-#pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      if (j < nout) {
-        const double2 c = cm[i + size_t(nin) * j];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          ax[k][j] = fma(v[k].x, c.x, ax[k][j]);
-          ax[k][j] = fma(-v[k].y, c.y, ax[k][j]);
-          ay[k][j] = fma(v[k].x, c.y, ay[k][j]);
-          ay[k][j] = fma(v[k].y, c.x, ay[k][j]);
-        }
+      for (int k = 0; k < 2; ++k) {
+        v[k] = make_double2(0.0, 0.0);
+        if (ok[k]) v[k] = ld_col(dc.a, dc.fmt, at[k]);
       }
+      add_products<JN, 2>(v, cm + size_t(JN) * i, ax, ay);
     }
   }
   const int pm = tb * kSymT + tx, qm = ta * kSymT + ty;  // mirror entries (pm, qm) and (pm, qm + 16)
@@ -2136,28 +2191,54 @@ hipError_t combine_launch(const ColDesc *descs, int nin, int nout, const Dbl2 *c
 }
 }  // namespace
 
+namespace {
+template <bool PLAIN>
+void combine_w_launch(const ColDesc *descs, int nin, int nout, const double2 *c, const double2 *beta, int64_t d,
+                      hipStream_t s) {
+  // one wavefront per 64 * RPL rows, at most 2048 workgroups of 4 (grid-stride beyond)
+  auto grid = [d](int rpl) {
+    const int64_t waves = (d + 64 * rpl - 1) / (64 * rpl);
+    return dim3(unsigned((waves + 3) / 4 < 2048 ? (waves + 3) / 4 : 2048));
+  };
+  const dim3 b(256);
+  if (nout <= 4)
+    hipLaunchKernelGGL((k_combine_w<4, 2, 8, PLAIN>), grid(2), b, 0, s, descs, nin, nout, c, beta, d);
+  else if (nout <= 8)
+    hipLaunchKernelGGL((k_combine_w<8, 2, 4, PLAIN>), grid(2), b, 0, s, descs, nin, nout, c, beta, d);
+  else if (nout <= 12)
+    hipLaunchKernelGGL((k_combine_w<12, 2, PLAIN ? 1 : 2, PLAIN>), grid(2), b, 0, s, descs, nin, nout, c, beta, d);
+  else if (nout <= 16)
+    hipLaunchKernelGGL((k_combine_w<16, 2, PLAIN ? 1 : 2, PLAIN>), grid(2), b, 0, s, descs, nin, nout, c, beta, d);
+  else
+    hipLaunchKernelGGL((k_combine_w<kCombMaxOut, 1, 1, PLAIN>), grid(1), b, 0, s, descs, nin, nout, c, beta, d);
+}
+
+template <bool PLAIN>
+void combine_sym_launch(const ColDesc *descs, int nin, int nout, const double2 *c, const double2 *beta, int m,
+                        int sign, hipStream_t s) {
+  const dim3 g(unsigned(sym_grid(m))), b(kSymT, 16);
+  const int nblk = sym_blocks(m);
+  if (nout <= 4)
+    hipLaunchKernelGGL((k_combine_sym<4, 8, PLAIN>), g, b, 0, s, descs, nin, nout, c, beta, m, nblk, sign);
+  else if (nout <= 8)
+    hipLaunchKernelGGL((k_combine_sym<8, 4, PLAIN>), g, b, 0, s, descs, nin, nout, c, beta, m, nblk, sign);
+  else if (nout <= 12)
+    hipLaunchKernelGGL((k_combine_sym<12, PLAIN ? 1 : 2, PLAIN>), g, b, 0, s, descs, nin, nout, c, beta, m, nblk, sign);
+  else
+    hipLaunchKernelGGL((k_combine_sym<16, PLAIN ? 1 : 2, PLAIN>), g, b, 0, s, descs, nin, nout, c, beta, m, nblk, sign);
+}
+}  // namespace
+
 hipError_t launch_combine(const ColDesc *descs, int nin, int nout, const Dbl2 *c, const Dbl2 *beta,
-                          int64_t d, hipStream_t s) {
+                          int64_t d, bool plain, hipStream_t s) {
   if (nin < 1 || nin > kCombMaxIn || nout < 1 || nout > kCombMaxOut) return hipErrorInvalidValue;
   if (nout <= 16 || nout > kCombGroups * 4) {
     const double2 *cc = reinterpret_cast<const double2 *>(c);
     const double2 *bb = reinterpret_cast<const double2 *>(beta);
-    // one wavefront per 64 * RPL rows, at most 2048 workgroups of 4 (grid-stride beyond)
-    auto grid = [d](int rpl) {
-      const int64_t waves = (d + 64 * rpl - 1) / (64 * rpl);
-      return dim3(unsigned((waves + 3) / 4 < 2048 ? (waves + 3) / 4 : 2048));
-    };
-    if (nout <= 4)
-      hipLaunchKernelGGL((k_combine_w<4, 2, 8>), grid(2), dim3(256), 0, s, descs, nin, nout, cc, bb, d);
-    else if (nout <= 8)
-      hipLaunchKernelGGL((k_combine_w<8, 2, 8>), grid(2), dim3(256), 0, s, descs, nin, nout, cc, bb, d);
-    else if (nout <= 12)
-      hipLaunchKernelGGL((k_combine_w<12, 2, 8>), grid(2), dim3(256), 0, s, descs, nin, nout, cc, bb, d);
-    else if (nout <= 16)
-      hipLaunchKernelGGL((k_combine_w<16, 2, 16>), grid(2), dim3(256), 0, s, descs, nin, nout, cc, bb, d);
+    if (plain)
+      combine_w_launch<true>(descs, nin, nout, cc, bb, d, s);
     else
-      hipLaunchKernelGGL((k_combine_w<kCombMaxOut, 1, 4>), grid(1), dim3(256), 0, s, descs, nin, nout, cc, bb,
-                         d);
+      combine_w_launch<false>(descs, nin, nout, cc, bb, d, s);
     return hipGetLastError();
   }
   // 17..32 outputs: C and one row tile in LDS, (64 * 8 * 4 + 32 * 64) * 16 B = 64 KB at most
@@ -2169,21 +2250,20 @@ hipError_t launch_combine(const ColDesc *descs, int nin, int nout, const Dbl2 *c
 
 bool combine_halves(int nout) { return nout <= 16; }
 
+int combine_ld(int nout) {
+  if (nout <= 16) return (nout + 3) / 4 * 4;
+  return nout > kCombGroups * 4 ? kCombMaxOut : nout;
+}
+
 hipError_t launch_combine_sym(const ColDesc *descs, int nin, int nout, const Dbl2 *c, const Dbl2 *beta, int m,
-                              int sign, hipStream_t s) {
+                              int sign, bool plain, hipStream_t s) {
   if (nin < 1 || nin > kCombMaxIn || nout < 1 || !combine_halves(nout)) return hipErrorInvalidValue;
   const double2 *cc = reinterpret_cast<const double2 *>(c);
   const double2 *bb = reinterpret_cast<const double2 *>(beta);
-  const dim3 g(unsigned(sym_grid(m))), b(kSymT, 16);
-  const int nblk = sym_blocks(m);
-  if (nout <= 4)
-    hipLaunchKernelGGL((k_combine_sym<4, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
-  else if (nout <= 8)
-    hipLaunchKernelGGL((k_combine_sym<8, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
-  else if (nout <= 12)
-    hipLaunchKernelGGL((k_combine_sym<12, 8>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+  if (plain)
+    combine_sym_launch<true>(descs, nin, nout, cc, bb, m, sign, s);
   else
-    hipLaunchKernelGGL((k_combine_sym<16, 4>), g, b, 0, s, descs, nin, nout, cc, bb, m, nblk, sign);
+    combine_sym_launch<false>(descs, nin, nout, cc, bb, m, sign, s);
   return hipGetLastError();
 }
 
