@@ -458,7 +458,7 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
   // part, and the iteration drifts away from the wanted levels after tens of
   // iterations (seen at NN=25, where FP64 has only these kernels).  Projecting y
   // keeps both paths on the exchange-symmetric subspace.
-  if (sym != 0) DEX_HIP(dex::launch_sym_project(y, c->m, sym > 0 ? 1 : -1, c->stream));
+  if (sym != 0) DEX_HIP(dex::launch_sym_project(y, y, c->m, sym > 0 ? 1 : -1, c->stream));
   return 0;
 }
 
@@ -1778,7 +1778,7 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
   const double t_start = now_s();
   if (o.symmetry != 0) {
     // the exchange-symmetric matvec assumes X = sym X^T: project the start block
-    for (int j = 0; j < nev; ++j) DEX_HIP(dex::launch_sym_project(X.cols[j], c->m, o.symmetry, c->stream));
+    for (int j = 0; j < nev; ++j) DEX_HIP(dex::launch_sym_project(X.cols[j], X.cols[j], c->m, o.symmetry, c->stream));
   }
   // NORMALIZE(X) (gplmr.F90:65)
   {
@@ -2213,7 +2213,7 @@ extern "C" int dex_gplmr_eig_device(dex_ctx *c, void *x_dev, double *e, int32_t 
   for (int j = 0; j < nev; ++j) xcols.push_back(static_cast<Dbl2 *>(x_dev) + size_t(j) * c->d);
   for (int j = 0; j < guard; ++j) {
     DEX_HIP(dex::launch_fill_gaussian(guards[j], c->d, 0x67756172ull, uint32_t(j), 0xFFFFFFFFu, c->stream));
-    if (o.symmetry != 0) DEX_HIP(dex::launch_sym_project(guards[j], c->m, o.symmetry, c->stream));
+    if (o.symmetry != 0) DEX_HIP(dex::launch_sym_project(guards[j], guards[j], c->m, o.symmetry, c->stream));
     xcols.push_back(guards[j]);
   }
   const cd sigma(sigma_re, sigma_im);
@@ -2281,12 +2281,13 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
   } else {
     st = 0;
     const size_t bytes = size_t(c->d) * nev * sizeof(Dbl2);
-    if (hipMemcpyAsync(px_dev, x_dev, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+    if (symmetry == 0 && hipMemcpyAsync(px_dev, x_dev, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
       st = fail(DEX_EHIP, "device copy failed");
     // the block operations read one half of an exchange-symmetric vector: any other X
-    // counts as Xs, as in the matvec (no change to an exactly symmetric one)
+    // counts as its symmetric part, as in the matvec (no change to an exactly
+    // symmetric one); PX takes that part in place of a copy (3.1 of 53 ms at NN = 21)
     for (int j = 0; j < nev && symmetry != 0 && !st; ++j)
-      if (dex::launch_sym_project(out.cols[j], c->m, symmetry, c->stream) != hipSuccess)
+      if (dex::launch_sym_project(in.cols[j], out.cols[j], c->m, symmetry, c->stream) != hipSuccess)
         st = fail(DEX_EHIP, "exchange projection failed");
     if (!st) st = S.inner_solve(out, inner_iter, cd(sigma_re, sigma_im));
   }
@@ -2556,7 +2557,7 @@ extern "C" int dex_fill_gaussian_device(dex_ctx *c, void *x_dev, int32_t ncols, 
   for (int j = 0; j < ncols; ++j) {
     Dbl2 *xj = static_cast<Dbl2 *>(x_dev) + size_t(j) * c->d;
     DEX_HIP(dex::launch_fill_gaussian(xj, c->d, seed, uint32_t(j), stream_id, c->stream));
-    if (symmetry != 0) DEX_HIP(dex::launch_sym_project(xj, c->m, symmetry > 0 ? 1 : -1, c->stream));
+    if (symmetry != 0) DEX_HIP(dex::launch_sym_project(xj, xj, c->m, symmetry > 0 ? 1 : -1, c->stream));
   }
   DEX_HIP(hipStreamSynchronize(c->stream));
   return DEX_OK;

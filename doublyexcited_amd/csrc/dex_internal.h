@@ -154,8 +154,8 @@ hipError_t launch_resid(const ColDesc *descs, int nev, const double *sc, const D
 // (g0 + i g1)/sqrt(2) with g from Box-Muller on the counter (i, c, stream, 0).
 hipError_t launch_fill_gaussian(Dbl2 *x, int64_t n, uint64_t seed, uint32_t col, uint32_t stream_id,
                                 hipStream_t s);
-// Exchange projection X <- (X + sign X^T)/2 in the M x M view (in place).
-hipError_t launch_sym_project(Dbl2 *x, int64_t m, int sign, hipStream_t s);
+// Exchange projection Y = (X + sign X^T)/2 in the M x M view (Y may be X).
+hipError_t launch_sym_project(const Dbl2 *x, Dbl2 *y, int64_t m, int sign, hipStream_t s);
 // out(p, q) = sum_b T(p, b) X(q, b) (M x M from two M x K blocks)
 hipError_t launch_lowrank(const Dbl2 *t, const Dbl2 *x, Dbl2 *out, int64_t m, int k, hipStream_t s);
 // W = Y X (conj_x: Y conj(X)) for M x M Y and M x K X

@@ -1810,8 +1810,8 @@ __global__ void k_fill_gaussian(double2 *__restrict__ x, int64_t n, uint64_t see
   x[i] = make_double2(rad * cs * s, rad * sn * s);
 }
 
-// X <- (X + sign X^T)/2 on the M x M matrix, tiles of 32 x 32 above the diagonal.
-__global__ void k_singlet(double2 *__restrict__ x, int64_t m, double sign) {
+// Y = (X + sign X^T)/2 on the M x M matrix, tiles of 32 x 32 above the diagonal (Y may be X).
+__global__ void k_singlet(const double2 *x, double2 *y, int64_t m, double sign) {
   __shared__ double2 ta[32][33], tb[32][33];
   const int64_t bi = blockIdx.x, bj = blockIdx.y;
   if (bi > bj) return;
@@ -1827,11 +1827,11 @@ __global__ void k_singlet(double2 *__restrict__ x, int64_t m, double sign) {
     const int64_t i = bi * 32 + tx, j = bj * 32 + r;
     const double2 a = ta[r][tx], b = tb[tx][r];  // b = x[j + m i]
     const double2 s = make_double2(0.5 * (a.x + sign * b.x), 0.5 * (a.y + sign * b.y));
-    if (i < m && j < m) x[i + m * j] = s;
+    if (i < m && j < m) y[i + m * j] = s;
     const int64_t i2 = bj * 32 + tx, j2 = bi * 32 + r;
     const double2 a2 = tb[r][tx], b2 = ta[tx][r];
     const double2 s2 = make_double2(0.5 * (a2.x + sign * b2.x), 0.5 * (a2.y + sign * b2.y));
-    if (i2 < m && j2 < m) x[i2 + m * j2] = s2;
+    if (i2 < m && j2 < m) y[i2 + m * j2] = s2;
   }
 }
 
@@ -2300,10 +2300,10 @@ hipError_t launch_fill_gaussian(Dbl2 *x, int64_t n, uint64_t seed, uint32_t col,
   return hipGetLastError();
 }
 
-hipError_t launch_sym_project(Dbl2 *x, int64_t m, int sign, hipStream_t s) {
+hipError_t launch_sym_project(const Dbl2 *x, Dbl2 *y, int64_t m, int sign, hipStream_t s) {
   const unsigned nb = unsigned((m + 31) / 32);
-  hipLaunchKernelGGL(k_singlet, dim3(nb, nb), dim3(32, 8), 0, s, reinterpret_cast<double2 *>(x), m,
-                     double(sign));
+  hipLaunchKernelGGL(k_singlet, dim3(nb, nb), dim3(32, 8), 0, s, reinterpret_cast<const double2 *>(x),
+                     reinterpret_cast<double2 *>(y), m, double(sign));
   return hipGetLastError();
 }
 
