@@ -47,6 +47,8 @@ double now_s() {
 constexpr int kMaxDesc = 512;
 constexpr int kMaxSmall = 96 * 64;
 constexpr int kNormCols = 128;  // residual columns to a wait (two sums each in d_dots)
+constexpr size_t kGramOutBytes = 64 * 128 * 16;  // one Gram launch's result
+constexpr size_t kDotsBytes = 64 * 4 * 8;        // column sums: 4 of 64 columns, 2 of kNormCols
 
 }  // namespace
 
@@ -201,10 +203,8 @@ struct dex_ctx {
   void *d_scratch = nullptr;  // this device's copy of `scratch` (dex_matvec_noalloc)
   ColDesc *d_desc = nullptr;
   unsigned char *d_args = nullptr;  // a combine's descriptors, C and beta, packed (one upload)
-  Dbl2 *d_gram_out = nullptr;
   void *d_partial = nullptr;
   size_t partial_bytes = 0;
-  double *d_dots = nullptr;
   int timing = 0;                 // 0 off, 1 every launch, n > 1 a random 1 in n of them
   std::atomic<int> stop{0};       // dex_ctx_stop: solves return at their next iteration boundary
   uint64_t sample_state = 0x9e3779b97f4a7c15ull;
@@ -230,6 +230,13 @@ struct dex_ctx {
   // coefficients): copies from pageable memory would wait for the stream
   char *h_stage = nullptr;
   size_t stage_cap = 0, stage_off = 0;
+  // results of the block reductions, in the same pinned allocation: the reduction
+  // kernels write them there (d_*: the device's addresses) and the host reads them
+  // after its wait.  Copied from device memory they cost a launch and a second wait
+  // each (two iterations of an 8 + 2 column solve, 150 Grams: 93.4 -> 90.0 ms at
+  // NN = 11, 46.3 -> 43.4 at NN = 9).
+  Dbl2 *h_gram = nullptr, *d_gram = nullptr;
+  double *h_dots = nullptr, *d_dots = nullptr;
 };
 
 namespace {
@@ -528,7 +535,7 @@ bool all_complex128(const std::vector<ColDesc> &ds) {
 // exchange-symmetric (antisymmetric) vector: its two halves are each other's mirror
 // images, so Grams and combinations read one (half_blocks grids).
 
-// Runs one Gram launch (kl <= 64, kr <= 128) and copies the kl x kr result
+// Runs one Gram launch (kl <= 64, kr <= 128) and puts the kl x kr result
 // into g (leading dimension ldg) at (i0, j0).  With share > 0 the skipped lower
 // blocks of the Hermitian share x share part are filled by conjugate symmetry.
 int gram_launch_copy(dex_ctx *c, const std::vector<ColDesc> &ds, int kl, int kr, int share,
@@ -540,12 +547,10 @@ int gram_launch_copy(dex_ctx *c, const std::vector<ColDesc> &ds, int kl, int kr,
     const double rows = double(c->d) * (half ? 0.5 : 1.0);
     KTimer kt(c, DEX_K_GRAM, rows * distinct_entry_bytes(ds, ds.size()), 8.0 * rows * (double(kl) * kr - hskip));
     DEX_HIP(dex::launch_gram(c->d_desc, kl, kr, share, c->d, half ? int(c->m) : 0,
-                             reinterpret_cast<Dbl2 *>(c->d_partial), c->d_gram_out, c->stream));
+                             reinterpret_cast<Dbl2 *>(c->d_partial), c->d_gram, c->stream));
   }
-  std::vector<cd> part(size_t(kl) * kr);
-  DEX_HIP(hipMemcpyAsync(part.data(), c->d_gram_out, part.size() * sizeof(Dbl2), hipMemcpyDeviceToHost,
-                         c->stream));
   DEX_HIP(hipStreamSynchronize(c->stream));
+  const cd *part = reinterpret_cast<const cd *>(c->h_gram);
   for (int j = 0; j < kr; ++j)
     for (int i = 0; i < kl; ++i) {
       cd v = part[i + size_t(kl) * j];
@@ -675,9 +680,8 @@ int coldots(dex_ctx *c, const std::vector<ColDesc> &a, const std::vector<ColDesc
     DEX_HIP(dex::launch_coldots(c->d_desc, k, c->d, reinterpret_cast<double *>(c->d_partial), c->d_dots,
                                 c->stream));
   }
-  std::vector<double> h(size_t(k) * 4);
-  DEX_HIP(hipMemcpyAsync(h.data(), c->d_dots, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   DEX_HIP(hipStreamSynchronize(c->stream));
+  const double *h = c->h_dots;
   aa.resize(k);
   ab.resize(k);
   bb.resize(k);
@@ -719,9 +723,8 @@ int residual_cols(dex_ctx *c, const std::vector<Dbl2 *> &x, const std::vector<Db
                               reinterpret_cast<const Dbl2 *>(c->d_args + bd + bs), c->d,
                               reinterpret_cast<double *>(c->d_partial), c->d_dots, c->stream));
   }
-  std::vector<double> h(nev);
-  DEX_HIP(hipMemcpyAsync(h.data(), c->d_dots, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   DEX_HIP(hipStreamSynchronize(c->stream));
+  const double *h = c->h_dots;
   rn.resize(nev);
   for (int j = 0; j < nev; ++j) rn[j] = std::sqrt(h[j]);
   return 0;
@@ -856,15 +859,22 @@ int dex_ctx_create(const dex_params *p, dex_ctx **out) {
     e = hipMemcpy(c->d_vn, c->vn_host.data(), c->vn_host.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = dmalloc(&c->d_desc, kMaxDesc * sizeof(ColDesc));
   if (e == hipSuccess) e = dmalloc(&c->d_args, kMaxDesc * sizeof(ColDesc) + 2 * kMaxSmall * sizeof(Dbl2) + 512);
-  if (e == hipSuccess) e = dmalloc(&c->d_gram_out, 192 * 192 * sizeof(Dbl2));
   c->partial_bytes = std::max(dex::gram_partial_elems(64, 128) * sizeof(Dbl2),
                               dex::coldots_partial_elems(64) * sizeof(double));
   if (e == hipSuccess) e = dmalloc(&c->d_partial, c->partial_bytes);
-  if (e == hipSuccess) e = dmalloc(&c->d_dots, 64 * 4 * sizeof(double));
   for (int i = 0; i < 3 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
   if (e == hipSuccess) {
     c->stage_cap = size_t(4) << 20;
-    e = hipHostMalloc(reinterpret_cast<void **>(&c->h_stage), c->stage_cap, hipHostMallocDefault);
+    e = hipHostMalloc(reinterpret_cast<void **>(&c->h_stage), c->stage_cap + kGramOutBytes + kDotsBytes,
+                      hipHostMallocMapped);
+  }
+  void *mapped = nullptr;
+  if (e == hipSuccess) e = hipHostGetDevicePointer(&mapped, c->h_stage, 0);
+  if (e == hipSuccess) {
+    c->h_gram = reinterpret_cast<Dbl2 *>(c->h_stage + c->stage_cap);
+    c->h_dots = reinterpret_cast<double *>(c->h_stage + c->stage_cap + kGramOutBytes);
+    c->d_gram = reinterpret_cast<Dbl2 *>(static_cast<char *>(mapped) + c->stage_cap);
+    c->d_dots = reinterpret_cast<double *>(static_cast<char *>(mapped) + c->stage_cap + kGramOutBytes);
   }
   // the allocation-free matvec's scratch on this device (the device is current)
   if (e == hipSuccess) e = scratch_address(p->device, &c->d_scratch);
@@ -881,8 +891,7 @@ int dex_ctx_destroy(dex_ctx *c) {
   (void)hipSetDevice(c->p.device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (void *ptr : {(void *)c->d_tinv, (void *)c->d_vn, c->d_u, (void *)c->d_desc,
-                    (void *)c->d_args, (void *)c->d_gram_out, c->d_partial,
-                    (void *)c->d_dots})
+                    (void *)c->d_args, c->d_partial})
     if (ptr) (void)hipFree(ptr);
   for (auto &ev : c->ev)
     if (ev) (void)hipEventDestroy(ev);
@@ -2129,8 +2138,7 @@ int64_t ctx_fixed_bytes(int nn) {
   const int64_t partial = int64_t(std::max(dex::gram_partial_elems(64, 128) * sizeof(Dbl2),
                                            dex::coldots_partial_elems(64) * sizeof(double)));
   return (L * L * L + m) * 8 + int64_t(kMaxDesc) * int64_t(sizeof(ColDesc)) +
-         (int64_t(kMaxDesc) * int64_t(sizeof(ColDesc)) + 2 * kMaxSmall * 16 + 512) + 192 * 192 * 16 + partial +
-         64 * 4 * 8 + vec +
+         (int64_t(kMaxDesc) * int64_t(sizeof(ColDesc)) + 2 * kMaxSmall * 16 + 512) + partial + vec +
          margin_vectors(d) * vec;
 }
 
@@ -2527,9 +2535,8 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
                                           e[2 * j + 1], static_cast<double *>(c->d_partial), c->d_dots + 2 * (j - j0),
                                           {c->d_vn, c->d_tinv, c->coef}, c->stream));
       }
-      double h[2 * kNormCols];
-      DEX_HIP(hipMemcpyAsync(h, c->d_dots, size_t(2 * k) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
       DEX_HIP(hipStreamSynchronize(c->stream));
+      const double *h = c->h_dots;
       for (int j = 0; j < k; ++j) res_out[j0 + j] = std::sqrt(h[2 * j]) / std::sqrt(h[2 * j + 1]);
     }
     return DEX_OK;
