@@ -185,10 +185,10 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtr
     line_apply<NN, R>(xi, [&](int k, R y) {
       const R ki = y + b[c + N2 * k];
       const R vr = R(vn[c + N2 * k] + vq + tinv[t0 - L * L * k] * cf.inv_d3);
-      const R vcr = c1r * vr - shr, vci = c1i * vr - shi;
+      const R vxr = vr * xr[k], vxi = vr * xi[k];
       ZT o;
-      o.x = s2r * kr[k] - s2i * ki + vcr * xr[k] - vci * xi[k];
-      o.y = s2r * ki + s2i * kr[k] + vcr * xi[k] + vci * xr[k];
+      o.x = s2r * kr[k] - s2i * ki + (c1r * vxr - shr * xr[k]) - (c1i * vxi - shi * xi[k]);
+      o.y = s2r * ki + s2i * kr[k] + (c1r * vxi - shr * xi[k]) + (c1i * vxr - shi * xr[k]);
       zq[c + N2 * k] = o;
     });
   }
@@ -396,10 +396,10 @@ __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane
     line_apply<NN, R>(xi, [&](int j, R y) {
       const R ki = y + b[NN * j + i];
       const R vr = R(vn[N2 * k + NN * j + i] + vq + tinv[t0 - L * j] * cf.inv_d3);
-      const R vcr = c1r * vr - shr, vci = c1i * vr - shi;
+      const R vxr = vr * xr[j], vxi = vr * xi[j];
       ZT o;
-      o.x = s2r * kr[j] - s2i * ki + vcr * xr[j] - vci * xi[j];
-      o.y = s2r * ki + s2i * kr[j] + vcr * xi[j] + vci * xr[j];
+      o.x = s2r * kr[j] - s2i * ki + (c1r * vxr - shr * xr[j]) - (c1i * vxi - shi * xi[j]);
+      o.y = s2r * ki + s2i * kr[j] + (c1r * vxi - shr * xi[j]) + (c1i * vxr - shi * xr[j]);
       z[base + NN * j] = o;
     });
   }
