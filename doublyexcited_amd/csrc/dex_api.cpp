@@ -377,6 +377,13 @@ int batch_cols(const dex_ctx *c, int io, int left) {
   return launches > 1 ? (left + launches - 1) / launches : left;
 }
 
+// Whether general columns (consecutive ones) go through the one-launch kernel: small
+// grids, outputs apart from the inputs.
+bool one_launch(const dex_ctx *c, int io, const void *x, const void *y, int ncols) {
+  const size_t bytes = size_t(ncols) * size_t(c->d) * (io == dex::kIoF32 ? 8 : 16);
+  return dex::general_direct(c->nn) && x != y && !chained(x, y, bytes);
+}
+
 // What the passes of H - shift read beside the vectors.
 dex::PotArgs pot_args(const dex_ctx *c, cd shift) {
   dex::PotArgs pot{c->d_vn, c->d_tinv, c->coef};
@@ -398,6 +405,17 @@ int fast_passes(dex_ctx *c, int io, const void *const *x, void *const *y, int nc
   const dex::PotArgs pot = pot_args(c, shift);
   const bool planes = sym == 0 && dex::general_by_planes(c->nn);
   if (pass_events) DEX_HIP(hipEventRecord(c->ev[0], c->stream));
+  if (sym == 0 && one_launch(c, io, x[0], y[0], ncols)) {
+    {
+      KTimer kt(c, DEX_K_PASS1, 2.0 * xb * dd, (24.0 * nn + 14.0) * dd);
+      DEX_HIP(dex::launch_direct(c->nn, io, x[0], y[0], ncols, pot, c->stream));
+    }
+    if (pass_events) {
+      DEX_HIP(hipEventRecord(c->ev[1], c->stream));
+      DEX_HIP(hipEventRecord(c->ev[2], c->stream));
+    }
+    return 0;
+  }
   {
     // reads X, writes Z; three axes (two by planes) of NN real-by-complex MACs an
     // entry and the potential
@@ -1077,6 +1095,8 @@ int dex_matvec_noalloc(dex_ctx *c, const void *in, void *out, int32_t howmany, i
     } else if (symmetry != 0) {
       DEX_HIP(dex::launch_pass1(c->nn, io, true, x, y, k, pot, c->stream));
       DEX_HIP(dex::launch_symfold(c->nn, io, y, k, symmetry, c->stream));
+    } else if (one_launch(c, io, x[0], y[0], k)) {
+      DEX_HIP(dex::launch_direct(c->nn, io, x[0], y[0], k, pot, c->stream));
     } else {
       // Z (fully written by the electron-1 pass before the second pass reads it)
       DEX_HIP(dex::launch_general_first(c->nn, io, x[0], c->d_scratch, k, pot, c->stream));

@@ -100,6 +100,10 @@ bool general_by_planes(int nn);
 hipError_t launch_general_first(int nn, int io, const void *x, void *z, int ncols, const PotArgs &pot, hipStream_t s);
 hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y, int ncols, const MatvecCoef &coef,
                                  hipStream_t s);
+// General vectors of the smallest grids in one launch, on up to kBatchMax consecutive
+// columns; y may overlap no column of x.
+bool general_direct(int nn);
+hipError_t launch_direct(int nn, int io, const void *x, void *y, int ncols, const PotArgs &pot, hipStream_t s);
 // out[0] = ||H x - e x||^2 and out[1] = ||x||^2 of one complex128 column in FP64
 // (general_by_planes grids; z: D entries; partial: 2 doubles a run tile, at most
 // 2 (NN^4 / 8 + 8)).

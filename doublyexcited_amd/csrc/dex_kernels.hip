@@ -532,6 +532,56 @@ __global__ __launch_bounds__(round_up(NN *plane_run<XT>(), 64)) void k_plane2(co
   }
 }
 
+// ---- the smallest grids ----------------------------------------------------------
+// General vectors in one launch: Y = s2 (K1 + K2) X + (c1 Vr - shift) o X, an entry a
+// thread, from the six lines through it.  A vector fits the L2 many times over and a
+// call is all latency: one launch and one wait for loads in place of two launches with
+// an intermediate between.  Threads of a workgroup run along electron 1, so five of
+// the six lines are read in runs along p.  Y must not overlap X: other workgroups read it.
+template <int NN>
+constexpr int direct_threads() {
+  return NN * NN * NN < 256 ? round_up(NN * NN * NN, 64) : 256;
+}
+
+template <int NN, typename R, typename XT>
+__global__ __launch_bounds__(direct_threads<NN>()) void k_direct(ColPtrs xs, ColPtrsW ys,
+                                                                 const double *__restrict__ vn,
+                                                                 const double *__restrict__ tinv, MatvecCoef cf) {
+  constexpr int N2 = NN * NN, N3 = NN * N2, L = 2 * NN + 1, T = direct_threads<NN>();
+  constexpr int TILES = (N3 + T - 1) / T;
+  const int q = int(blockIdx.x) / TILES, p = int(blockIdx.x) % TILES * T + int(threadIdx.x);
+  if (p >= N3) return;
+  const XT *__restrict__ x = static_cast<const XT *>(xs.p[blockIdx.y]);
+  const int pi[3] = {p % NN, p / NN % NN, p / N2}, qi[3] = {q % NN, q / NN % NN, q / N2};
+  constexpr int stride[3] = {1, NN, N2};
+  const XT own = x[p + N3 * q];
+  const R vr = R(vn[p] + vn[q] +
+                 tinv[(qi[0] - pi[0] + NN) + L * ((qi[1] - pi[1] + NN) + L * (qi[2] - pi[2] + NN))] * cf.inv_d3);
+  __shared__ R tau[2 * NN - 1];
+  if (threadIdx.x < 2 * NN - 1) tau[threadIdx.x] = R(tau_rt(int(threadIdx.x) - (NN - 1)));
+  __syncthreads();
+  R kr = R(0), ki = R(0);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    R sr = R(0), si = R(0);
+#pragma unroll
+    for (int l = 0; l < NN; ++l) {
+      const XT u = x[p + stride[a] * (l - pi[a]) + N3 * q], v = x[p + N3 * (q + stride[a] * (l - qi[a]))];
+      const R tp = tau[l - pi[a] + NN - 1], tq = tau[l - qi[a] + NN - 1];
+      sr += tp * R(u.x) + tq * R(v.x);
+      si += tp * R(u.y) + tq * R(v.y);
+    }
+    kr += sr;
+    ki += si;
+  }
+  const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
+  const R vcr = R(cf.c1_re) * vr - R(cf.sh_re), vci = R(cf.c1_im) * vr - R(cf.sh_im);
+  XT o;
+  o.x = s2r * kr - s2i * ki + vcr * R(own.x) - vci * R(own.y);
+  o.y = s2r * ki + s2i * kr + vcr * R(own.y) + vci * R(own.x);
+  static_cast<XT *>(ys.p[blockIdx.y])[p + N3 * q] = o;
+}
+
 // out[e] = sum over nparts of partial[b nelem + e], one workgroup an element.
 __global__ __launch_bounds__(1024) void k_reduce_wide(const double *__restrict__ partial, int nparts, int nelem,
                                                       double *__restrict__ out) {
@@ -678,6 +728,11 @@ constexpr bool fast_fits(int nn, size_t rsize) {
 
 // Largest grid whose general vectors go through the cubes (launch_general_first).
 constexpr int kCubeMaxNN = 11;
+// Largest grid whose general vectors take one launch (k_direct).  Microseconds of a
+// call, two launches and one: one column at NN = 3 23.4 and 20.0, at NN = 5 24.4 and
+// 20.3, 16 columns there 33.3 and 24.3; at NN = 7 one column 27.7 and 23.7, but 16
+// columns 66.6 and 80.0 (each entry reads its six lines, 42 entries, from L2).
+constexpr int kDirectMaxNN = 5;
 
 #define DEX_NN_LIST(X) X(3) X(5) X(7) X(9) X(11) X(13) X(15) X(17) X(19) X(21) X(23) X(25)
 
@@ -756,6 +811,39 @@ hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, h
 // and planes: NN = 11 FP64 68 and 69; 13: 165 and 135; 17: 997 and 745; 21: 3270 and
 // 2850; complex64 at 17: 833 and 455; at 25: 7035 and 4300.
 bool general_by_planes(int nn) { return nn > kCubeMaxNN; }
+
+bool general_direct(int nn) { return nn <= kDirectMaxNN; }
+
+hipError_t launch_direct(int nn, int io, const void *x, void *y, int ncols, const PotArgs &pot, hipStream_t s) {
+  if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
+  ColPtrs xs{};
+  ColPtrsW ys{};
+  const size_t bytes = size_t(nn) * nn * nn * nn * nn * nn * (io == kIoF32 ? 8 : 16);
+  for (int j = 0; j < ncols; ++j) {
+    xs.p[j] = static_cast<const char *>(x) + size_t(j) * bytes;
+    ys.p[j] = static_cast<char *>(y) + size_t(j) * bytes;
+  }
+  switch (nn) {
+#define CASE(N)                                                                                                  \
+  case N:                                                                                                        \
+    if constexpr (N <= kDirectMaxNN) {                                                                           \
+      constexpr int T = direct_threads<N>();                                                                     \
+      const dim3 g(N * N * N * ((N * N * N + T - 1) / T), unsigned(ncols)), b(T);                                \
+      if (io == kIoF64)                                                                                          \
+        hipLaunchKernelGGL((k_direct<N, double, double2>), g, b, 0, s, xs, ys, pot.vn, pot.tinv, pot.cf);        \
+      else if (io == kIoF32)                                                                                     \
+        hipLaunchKernelGGL((k_direct<N, float, float2>), g, b, 0, s, xs, ys, pot.vn, pot.tinv, pot.cf);          \
+      else                                                                                                       \
+        hipLaunchKernelGGL((k_direct<N, float, double2>), g, b, 0, s, xs, ys, pot.vn, pot.tinv, pot.cf);         \
+      return hipGetLastError();                                                                                  \
+    }                                                                                                            \
+    return hipErrorInvalidValue;
+    DEX_NN_LIST(CASE)
+#undef CASE
+    default:
+      return hipErrorInvalidValue;
+  }
+}
 
 hipError_t launch_general_first(int nn, int io, const void *x, void *z, int ncols, const PotArgs &pot, hipStream_t s) {
   if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
