@@ -137,6 +137,13 @@ __device__ __forceinline__ void plane_axes(const R (&x)[NN], R *__restrict__ a, 
   __syncthreads();
 }
 
+// a b, not fused into the addition that follows.
+template <typename R>
+__device__ __forceinline__ R rounded_product(R a, R b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
 // Electron-1 pass on the cube of electron-2 index q = blockIdx.x (contiguous) of
 // column blockIdx.y: Z = s2 tau3D X + w (c1 Vr - shift) o X.  w = 1/2 for
 // exchange-(anti)symmetric vectors (Y = Z + sign Z^T follows, k_symfold), 1 for
@@ -149,7 +156,12 @@ __device__ __forceinline__ void plane_axes(const R (&x)[NN], R *__restrict__ a, 
 // (a wave's memory operations complete in order).  The loop also let the compiler
 // keep vn in registers, which cost the second workgroup: FP32 at NN = 19 ran 277 us
 // a column looped and 175 us not, at NN = 21 487 and 354.
-template <int NN, typename R, typename XT, typename ZT>
+//
+// SHIFT: H - shift, each product of the potential term less that of the shift.  A
+// variant of its own: with a zero shift the plain matvec took 1-2% more (4 columns at
+// NN = 19 in complex64 1366 for 1346 us, one at NN = 25 6.96 for 6.85 ms).  Without SHIFT
+// the same products are rounded, so that a zero shift and none give the same bits.
+template <int NN, typename R, typename XT, typename ZT, bool SHIFT>
 __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtrsW zs, const double *__restrict__ vn,
                                                               const double *__restrict__ tinv, MatvecCoef cf,
                                                               double w) {
@@ -187,8 +199,13 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtr
       const R vr = R(vn[c + N2 * k] + vq + tinv[t0 - L * L * k] * cf.inv_d3);
       const R vxr = vr * xr[k], vxi = vr * xi[k];
       ZT o;
-      o.x = s2r * kr[k] - s2i * ki + (c1r * vxr - shr * xr[k]) - (c1i * vxi - shi * xi[k]);
-      o.y = s2r * ki + s2i * kr[k] + (c1r * vxi - shr * xi[k]) + (c1i * vxr - shi * xr[k]);
+      if constexpr (SHIFT) {
+        o.x = s2r * kr[k] - s2i * ki + (c1r * vxr - shr * xr[k]) - (c1i * vxi - shi * xi[k]);
+        o.y = s2r * ki + s2i * kr[k] + (c1r * vxi - shr * xi[k]) + (c1i * vxr - shi * xr[k]);
+      } else {
+        o.x = s2r * kr[k] - s2i * ki + rounded_product(c1r, vxr) - rounded_product(c1i, vxi);
+        o.y = s2r * ki + s2i * kr[k] + rounded_product(c1r, vxi) + rounded_product(c1i, vxr);
+      }
       zq[c + N2 * k] = o;
     });
   }
@@ -334,7 +351,7 @@ __global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, i
 // of the first axis in registers (contracted there), the second axis goes through
 // the LDS buffers a (entries) and b (its sums), one real component at a time.
 // 32 + 48 + 48 bytes an entry over the three passes, 4.6 TB/s of them at NN = 25 in
-// FP64 (6.8 ms a vector; six passes of one axis and the potential's took 16.8), with
+// FP64 (6.9 ms a vector; six passes of one axis and the potential's took 16.8), with
 // 8 waves a CU in flight (two workgroups: 80 KB of LDS, 205-240 registers).
 template <typename XT>
 constexpr int plane_run() {
@@ -348,7 +365,7 @@ constexpr int plane1_planes() {
 // Axes i1 and j1 and the potential: Z = s2 (tau x 1 + 1 x tau) X + (c1 Vr - shift) o X.
 // blockIdx: electron-2 index q, group of kp = plane1_planes() planes k1.  Thread (i, g) keeps the
 // j line of plane g.
-template <int NN, typename R, typename XT, typename ZT>
+template <int NN, typename R, typename XT, typename ZT, bool SHIFT>
 __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane1(
     const XT *__restrict__ x, ZT *__restrict__ z, const double *__restrict__ vn, const double *__restrict__ tinv,
     MatvecCoef cf) {
@@ -398,8 +415,13 @@ __global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane
       const R vr = R(vn[N2 * k + NN * j + i] + vq + tinv[t0 - L * j] * cf.inv_d3);
       const R vxr = vr * xr[j], vxi = vr * xi[j];
       ZT o;
-      o.x = s2r * kr[j] - s2i * ki + (c1r * vxr - shr * xr[j]) - (c1i * vxi - shi * xi[j]);
-      o.y = s2r * ki + s2i * kr[j] + (c1r * vxi - shr * xi[j]) + (c1i * vxr - shi * xr[j]);
+      if constexpr (SHIFT) {
+        o.x = s2r * kr[j] - s2i * ki + (c1r * vxr - shr * xr[j]) - (c1i * vxi - shi * xi[j]);
+        o.y = s2r * ki + s2i * kr[j] + (c1r * vxi - shr * xi[j]) + (c1i * vxr - shi * xr[j]);
+      } else {
+        o.x = s2r * kr[j] - s2i * ki + rounded_product(c1r, vxr) - rounded_product(c1i, vxi);
+        o.y = s2r * ki + s2i * kr[j] + rounded_product(c1r, vxi) + rounded_product(c1i, vxr);
+      }
       z[base + NN * j] = o;
     });
   }
@@ -615,6 +637,8 @@ bool set_lds(const void *kernel, size_t lds, std::atomic<bool> &done) {
   return true;
 }
 
+bool shifted(const MatvecCoef &cf) { return cf.sh_re != 0.0 || cf.sh_im != 0.0; }
+
 // LDS bytes of the passes' two cubes of reals.
 template <int NN, typename R>
 constexpr size_t cube_lds() {
@@ -623,8 +647,9 @@ constexpr size_t cube_lds() {
 
 template <int NN, typename R, typename XT, typename ZT>
 bool pass1_setup() {
-  static std::atomic<bool> attr{false};
-  return set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT>), cube_lds<NN, R>(), attr);
+  static std::atomic<bool> plain{false}, shifted{false};
+  return set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, false>), cube_lds<NN, R>(), plain) &&
+         set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, true>), cube_lds<NN, R>(), shifted);
 }
 
 template <int NN, typename R, typename XT, typename YT>
@@ -636,8 +661,13 @@ bool pass2_setup() {
 template <int NN, typename R, typename XT, typename ZT>
 hipError_t pass1_nn(const ColPtrs &xs, const ColPtrsW &zs, int ncols, const PotArgs &pot, double w, hipStream_t s) {
   if (!pass1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
-  hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT>), dim3(NN * NN * NN, unsigned(ncols)), dim3(cube_threads<NN>()),
-                     (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv, pot.cf, w);
+  const dim3 g(NN * NN * NN, unsigned(ncols)), b(cube_threads<NN>());
+  if (shifted(pot.cf))
+    hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, true>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv, pot.cf,
+                       w);
+  else
+    hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, false>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv,
+                       pot.cf, w);
   return hipGetLastError();
 }
 
@@ -662,8 +692,9 @@ constexpr size_t plane2_lds() {
 
 template <int NN, typename R, typename XT, typename ZT>
 bool plane1_setup() {
-  static std::atomic<bool> attr{false};
-  return set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT>), plane1_lds<NN, R>(), attr);
+  static std::atomic<bool> plain{false}, shifted{false};
+  return set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, false>), plane1_lds<NN, R>(), plain) &&
+         set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, true>), plane1_lds<NN, R>(), shifted);
 }
 
 template <int NN, typename R, typename XT, typename ZT, typename YT>
@@ -681,9 +712,15 @@ template <int NN, typename R, typename XT, typename ZT>
 hipError_t plane1_nn(const void *x, void *z, const PotArgs &pot, hipStream_t s) {
   if (!plane1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
   constexpr int G = plane1_planes<NN>();
-  hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT>), dim3(NN * NN * NN, (NN + G - 1) / G), dim3(round_up(NN * G, 64)),
-                     (plane1_lds<NN, R>()), s, static_cast<const XT *>(x), static_cast<ZT *>(z), pot.vn, pot.tinv,
-                     pot.cf);
+  const dim3 g(NN * NN * NN, (NN + G - 1) / G), b(round_up(NN * G, 64));
+  const XT *xx = static_cast<const XT *>(x);
+  ZT *zz = static_cast<ZT *>(z);
+  if (shifted(pot.cf))
+    hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, true>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
+                       pot.cf);
+  else
+    hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, false>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
+                       pot.cf);
   return hipGetLastError();
 }
 
