@@ -120,8 +120,9 @@ int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howma
  * the process ends, so grids with the LDS kernels are limited to NN <= 11 in an
  * FP64 context and NN <= 13 in an FP32 one (larger: DEX_ESIZE), in either
  * symmetry; FP64 grids without them (NN >= 23) keep U in Y.
- * General columns go one at a time, exchange-symmetric ones in batches as above;
- * no kernel timing is recorded.  Calls that overlap on one GPU share the array and
+ * Columns go in the batches of dex_matvec_sym_device (outputs that overlap other
+ * columns' inputs one at a time); at NN <= 5 outputs apart from the inputs need no U.
+ * No kernel timing is recorded.  Calls that overlap on one GPU share the array and
  * race: order them on one stream or serialise them.  U needs no clearing (each
  * column's first pass writes all of it). */
 int dex_matvec_noalloc(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
@@ -346,9 +347,9 @@ int dex_get_kernel_timing(const dex_ctx *ctx, double *pass1_ms, double *pass2_ms
  * the host from the launch shapes) accumulate until dex_reset_kernel_stats.  No reference
  * counterpart (the reference times with MPI_WTIME only, gplmr.F90:64-380). */
 enum {
-  DEX_K_PASS1 = 0,   /* electron-1 three-axis kinetic pass */
-  DEX_K_PASS2 = 1,   /* electron-2 pass with the potential (general vectors) */
-  DEX_K_SYMADD = 2,  /* exchange transpose-add pass with the potential */
+  DEX_K_PASS1 = 0,   /* first pass: kinetic axes of electron 1, potential (NN <= 5: all of H) */
+  DEX_K_PASS2 = 1,   /* the remaining kinetic passes (general vectors) */
+  DEX_K_SYMADD = 2,  /* exchange transpose-add pass */
   DEX_K_GRAM = 3,    /* block Gram (with its partial-sum reduction) */
   DEX_K_COMBINE = 4, /* block linear combination */
   DEX_K_COLDOTS = 5, /* per-column dots and norms, and the residual step (scaled X, AX and W) */
