@@ -1,0 +1,37 @@
+"""Rules of the kernel source that no run on a device shows reliably."""
+import re
+from pathlib import Path
+
+SOURCE = Path(__file__).resolve().parents[1] / "doublyexcited_amd" / "csrc" / "dex_kernels.hip"
+
+
+def _kernels():
+    """(name, parameters, body) of every __global__ function."""
+    text = re.sub(r"//[^\n]*", "", SOURCE.read_text())
+
+    def closing(at, pair):  # the index behind the bracket that closes the one at `at`
+        depth = 0
+        for i in range(at, len(text)):
+            depth += (text[i] == pair[0]) - (text[i] == pair[1])
+            if depth == 0:
+                return i + 1
+        raise AssertionError("unbalanced brackets")
+
+    for g in re.finditer(r"__global__", text):
+        head = re.compile(r"\b(k_\w+)\s*\(").search(text, g.end())
+        end = closing(head.end() - 1, "()")
+        body = text.index("{", end)
+        yield head.group(1), text[head.end():end - 1], text[body:closing(body, "{}")]
+
+
+def test_a_thread_leaves_a_kernel_only_behind_its_barriers():
+    """A return before a __syncthreads() takes the whole workgroup: its condition is of
+    blockIdx alone (a tile pair beyond the matrix, the lower triangle of tiles)."""
+    uniform = ("!sym_tile(m, nblk, ta, tb)", "bi > bj")
+    seen = 0
+    for name, _, body in _kernels():
+        before = body[:body.rfind("__syncthreads()")] if "__syncthreads()" in body else ""
+        for r in re.finditer(r"if \((.*)\)\s*return;", before):
+            seen += 1
+            assert r.group(1) in uniform, (name, r.group(0))
+    assert seen >= 3  # k_symfold, k_combine_sym, k_singlet
