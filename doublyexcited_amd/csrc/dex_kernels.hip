@@ -224,13 +224,12 @@ __device__ __forceinline__ int64_t xcd_group_map(int64_t b, int64_t m) {
 
 // Electron-2 pass for general vectors: Y = Z + s2 tau3D X on the stride-M cube
 // of each electron-1 index p of column blockIdx.y (columns M^2 entries apart; Z from
-// k_pass1 with w = 1; Y may
-// be X's or Z's storage: a thread reads each entry of Z before it writes that of Y,
-// and the workgroup's entries of X before any).
+// k_pass1 with w = 1).  Y may be X's or Z's storage (so none is __restrict__): a thread
+// reads each entry of Z before it writes that of Y, and the workgroup's entries of X
+// before any.
 template <int NN, typename R, typename XT, typename YT>
-__global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *__restrict__ x,
-                                                              const typename Cplx<R>::type *__restrict__ z,
-                                                              YT *__restrict__ y, MatvecCoef cf) {
+__global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *x, const typename Cplx<R>::type *z, YT *y,
+                                                              MatvecCoef cf) {
   using C = typename Cplx<R>::type;
   constexpr int N2 = NN * NN;
   constexpr int N3 = NN * N2;
@@ -255,12 +254,14 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *__restri
   plane_axes<NN, R>(xi, a, b, c);
   if (on) {
     const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
+    C zv[NN];  // ahead of the stores, behind which each load would wait in turn
+#pragma unroll
+    for (int k = 0; k < NN; ++k) zv[k] = z[p + M * (c + N2 * k)];
     line_apply<NN, R>(xi, [&](int k, R t) {
       const R ki = t + b[c + N2 * k];
-      const C zv = z[p + M * (c + N2 * k)];
       YT o;
-      o.x = zv.x + (s2r * kr[k] - s2i * ki);
-      o.y = zv.y + (s2r * ki + s2i * kr[k]);
+      o.x = zv[k].x + (s2r * kr[k] - s2i * ki);
+      o.y = zv[k].y + (s2r * ki + s2i * kr[k]);
       y[p + M * (c + N2 * k)] = o;
     });
   }

@@ -35,3 +35,15 @@ def test_a_thread_leaves_a_kernel_only_behind_its_barriers():
             seen += 1
             assert r.group(1) in uniform, (name, r.group(0))
     assert seen >= 3  # k_symfold, k_combine_sym, k_singlet
+
+
+def test_arrays_that_may_be_one_are_not_declared_apart():
+    """Kernels whose callers pass one array as input and output declare neither
+    __restrict__: the general second passes (Y over X or Z) and the projection (Y over X)."""
+    shared = {"k_pass2": ("x", "z", "y"), "k_plane2": ("x", "z", "y"), "k_singlet": ("x", "y")}
+    got = {name: params for name, params, _ in _kernels() if name in shared}
+    assert set(got) == set(shared)
+    for name, arrays in shared.items():
+        for a in arrays:
+            assert re.search(rf"\*\s*{a}\b", got[name]), (name, a)
+            assert not re.search(rf"__restrict__\s+{a}\b", got[name]), (name, a)
