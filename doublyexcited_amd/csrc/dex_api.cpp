@@ -2303,22 +2303,24 @@ extern "C" int dex_precblock_device(dex_ctx *c, const void *x_dev, void *px_dev,
     in.cols.push_back(const_cast<Dbl2 *>(static_cast<const Dbl2 *>(x_dev)) + size_t(j) * c->d);
     out.cols.push_back(static_cast<Dbl2 *>(px_dev) + size_t(j) * c->d);
   }
-  int st;
-  if (inner_iter == 1) {
-    st = S.matblock(in, out);
-  } else {
-    st = 0;
-    const size_t bytes = size_t(c->d) * nev * sizeof(Dbl2);
-    if (symmetry == 0 && hipMemcpyAsync(px_dev, x_dev, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
-      st = fail(DEX_EHIP, "device copy failed");
-    // the block operations read one half of an exchange-symmetric vector: any other X
-    // counts as its symmetric part, as in the matvec (no change to an exactly
-    // symmetric one); PX takes that part in place of a copy (3.1 of 53 ms at NN = 21)
-    for (int j = 0; j < nev && symmetry != 0 && !st; ++j)
+  int st = 0;
+  // PX takes X: with symmetry its (anti)symmetric part, which is what any other X counts
+  // as: the block operations read one half of a vector, and the symmetric passes give
+  // H X only for X = symmetry X^T.  No change to an exactly symmetric X; writing PX here
+  // saves a copy (3.1 of 53 ms at NN = 21, order 4 on 4 columns).
+  if (symmetry != 0) {
+    for (int j = 0; j < nev && !st; ++j)
       if (dex::launch_sym_project(in.cols[j], out.cols[j], c->m, symmetry, c->stream) != hipSuccess)
         st = fail(DEX_EHIP, "exchange projection failed");
-    if (!st) st = S.inner_solve(out, inner_iter, cd(sigma_re, sigma_im));
+  } else if (inner_iter > 1) {
+    const size_t bytes = size_t(c->d) * nev * sizeof(Dbl2);
+    if (hipMemcpyAsync(px_dev, x_dev, bytes, hipMemcpyDeviceToDevice, c->stream) != hipSuccess)
+      st = fail(DEX_EHIP, "device copy failed");
   }
+  // order 1: H X, with symmetry in place (the symmetric passes allow it)
+  if (!st)
+    st = inner_iter == 1 ? S.matblock(symmetry != 0 ? out : in, out)
+                         : S.inner_solve(out, inner_iter, cd(sigma_re, sigma_im));
   if (hipStreamSynchronize(c->stream) != hipSuccess && !st) st = fail(DEX_EHIP, "stream synchronise failed");
   return st;
 }

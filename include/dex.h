@@ -104,10 +104,11 @@ int dex_matvec_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
 /* HAMMULT for exchange-(anti)symmetric vectors, X(P,Q) = symmetry * X(Q,P)
  * (symmetry = +1 singlet, -1 triplet; 0 is dex_matvec_device).  Electron 2's
  * kinetic term is then the transpose of electron 1's, so the second pass is a
- * coalesced transpose-add in Y's own storage; the result is Y = H Xs with
- * Xs = (X + symmetry X^T)/2, exactly (anti)symmetric.  This is how the reference's start
- * vectors enter (HELIUM_ORBITAL with SIGN = +-1, hammod.F90:1059-1063); HAMMULT
- * itself has no such mode.  Needs the LDS kernels for the grid (dex_info.fast_path).
+ * coalesced transpose-add in Y's own storage; Y = H X, exactly (anti)symmetric.  X must be
+ * (anti)symmetric: nothing projects it, and for any other X, Y is neither H X nor H of its
+ * (anti)symmetric part.  This is how the reference's start vectors enter (HELIUM_ORBITAL
+ * with SIGN = +-1, hammod.F90:1059-1063); HAMMULT itself has no such mode.  Needs the LDS
+ * kernels for the grid (dex_info.fast_path).
  * With howmany >= 2 (and kernel timing off) the columns go through the passes in
  * even batches of up to 16 per launch on small grids, 4 on large ones. */
 int dex_matvec_sym_device(dex_ctx *ctx, const void *in, void *out, int32_t howmany,
@@ -249,8 +250,8 @@ int dex_residuals_device(dex_ctx *ctx, const void *x_dev, const double *e, int32
  * ||(H - sigma) PX - X|| (PRECBLOCK_BASIC -> basicblocklansolve,
  * gplmr.F90:674-770, harmonic_ritz_small.F90:258-324), every column
  * multiplied.  inner_iter = 0 is an error, as in the reference (:487-489).
- * symmetry: 0, or +-1 for exchange-(anti)symmetric X (any other X counts as
- * Xs = (X + symmetry X^T)/2). */
+ * symmetry: 0, or +-1 for exchange-(anti)symmetric X (in every order any other X counts
+ * as Xs = (X + symmetry X^T)/2). */
 int dex_precblock_device(dex_ctx *ctx, const void *x_dev, void *px_dev, int32_t m, int32_t mb,
                          int32_t nev, double sigma_re, double sigma_im, int32_t inner_iter,
                          int32_t symmetry);

@@ -71,3 +71,24 @@ def test_single_precision_basis_by_halves(dex, sym, cols):
             e.append(g.gplmr_eig_device(x, -0.7 - 0.002j, cols, maxit=2, tol=1e-7, symmetry=symmetry, inner_iter=8,
                                         inner_fp32=True).e)
         assert abs(e[0] - e[1]).max() <= 1e-5
+
+
+@pytest.mark.parametrize("n,cols,sym", [(2, 1, 1), (2, 17, -1), (5, 3, 1), (6, 2, -1)])
+def test_order_one_of_other_vectors_is_that_of_their_symmetric_part(dex, n, cols, sym):
+    """Order 1 is H X: for X of no symmetry H of its (anti)symmetric part, by the general
+    passes here.  Bound: the same products in another summation order, 1e-13 of max|y|."""
+    print(f"case: order 1 of other vectors n={n} cols={cols} sym={sym}", flush=True)
+    with dex.HeliumGrid(n, 0.5, 0.3) as g:
+        gen = torch.Generator(device="cuda").manual_seed(70 + n)
+        x = torch.randn(cols, g.m, g.m, dtype=torch.complex128, device="cuda", generator=gen)
+        xs = (0.5 * (x + sym * x.transpose(1, 2))).contiguous().view(-1)
+        x = x.view(-1)
+        kept, y, ref = x.clone(), torch.full_like(x, float("nan")), torch.empty_like(x)
+        g.precblock_device(x, y, cols, -0.7 - 0.002j, 1, symmetry=sym)
+        assert torch.equal(x, kept)
+        # general passes one column at a time, outputs over the inputs: two launches at every grid
+        ref.copy_(xs)
+        for j in range(cols):
+            v = ref[j * g.d:(j + 1) * g.d]
+            g.matvec_device(v, v, 1)
+        assert (y - ref).abs().max().item() <= 1e-13 * ref.abs().max().item()
