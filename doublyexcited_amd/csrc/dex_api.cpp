@@ -487,14 +487,14 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
   return 0;
 }
 
-// H - shift on complex64 device vectors in FP32 arithmetic (x, y hold D complex64).
-int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym, bool pass_events = false, cd shift = 0.0) {
+// H on complex64 device vectors in FP32 arithmetic (x, y hold D complex64).
+int apply_h32(dex_ctx *c, const Dbl2 *x, Dbl2 *y, int sym, bool pass_events = false) {
   if (!c->fast32) return fail(DEX_EUNSUPPORTED, "no FP32 matvec for this grid");
   if (sym == 0)
     if (int st = ensure_u(c)) return st;
   const void *xp = x;
   void *yp = y;
-  return fast_passes(c, dex::kIoF32, &xp, &yp, 1, sym, c->d_u, pass_events && c->timing, shift);
+  return fast_passes(c, dex::kIoF32, &xp, &yp, 1, sym, c->d_u, pass_events && c->timing);
 }
 
 // ---- block helpers on one context ------------------------------------------
@@ -1245,7 +1245,7 @@ struct Solver {
   std::vector<Dbl2 *> pool32;  // free complex64 work vectors (tagged pointers)
 
   // H - shift on every column of `in` into `out`.  complex128 columns get the FP64
-  // matvec, complex64 columns (both sides) the FP32 one.
+  // matvec, complex64 columns (both sides) the FP32 one, which takes no shift.
   int matblock(const Block &in, const Block &out, cd shift = 0.0) {
     const double t0 = now_s();
     if (out.size() < in.size()) return fail(DEX_EINVAL, "matblock: output block too small");
@@ -1253,6 +1253,7 @@ struct Solver {
     for (int j = 0; j < in.size(); ++j)
       if (is32(in.cols[j]) != is32(in.cols[0]) || is32(out.cols[j]) != is32(in.cols[j])) same = false;
     const bool lo = in.size() > 0 && is32(in.cols[0]);
+    if (lo && shift != 0.0) return fail(DEX_EINVAL, "matblock: a shift on complex64 columns");
     if (same && sym != 0 && in.size() >= 2 && (lo ? c->fast32 : c->fast64)) {
       // exchange-symmetric columns: a batch per pair of launches
       std::vector<const void *> xi;
@@ -1270,7 +1271,7 @@ struct Solver {
     for (int j = 0; j < in.size(); ++j) {
       if (is32(in.cols[j]) != is32(out.cols[j])) return fail(DEX_EINVAL, "matblock: mixed storage formats");
       if (is32(in.cols[j])) {
-        if (int st = apply_h32(c, untag(in.cols[j]), untag(out.cols[j]), sym, false, shift)) return st;
+        if (int st = apply_h32(c, untag(in.cols[j]), untag(out.cols[j]), sym)) return st;
       } else if (int st = apply_h(c, in.cols[j], out.cols[j], false, sym, false, shift)) {
         return st;
       }
@@ -1527,7 +1528,7 @@ struct Solver {
   // 0.5 is the criterion of Daniel, Gragg, Kaufman and Stewart (Math. Comp. 30
   // (1976) 772-795); the subtraction loses about eps / keep of relative
   // accuracy in R, so a smaller keep_min trades orthogonality for a pass.  q
-  // must be orthonormal.  The input is `wd` (plain descriptors),
+  // must be orthonormal.  The input is `wd` (descriptors: plain columns or a - sigma b),
   // the result goes to `w` (which may be the storage wd reads).  On success
   // `cq` and `r` satisfy w_in = q cq + w_out r; `ok` is false when the
   // projected block is numerically rank deficient (then w holds the projected,
@@ -1679,14 +1680,18 @@ struct Solver {
       Block hq;
       hq.fmt = bf;
       if (int st = grow(hq, kb)) return st;
-      // the matvec applies the shift: formed by the Grams and combinations as
-      // H Q_j - sigma Q_j, Q_j went through each of them a second time
-      if (int st = matblock(qj, hq, sigma)) return st;
+      // In FP64 the matvec applies the shift: formed by the Grams and combinations as
+      // H Q_j - sigma Q_j, Q_j went through each of them a second time.  A complex64 basis
+      // keeps that form: they form the difference in FP64, where the FP32 matvec would
+      // round sigma and store the difference in complex64.
+      if (int st = matblock(qj, hq, bf ? cd(0.0) : sigma)) return st;
+      std::vector<ColDesc> wd;
+      for (int i = 0; i < kb; ++i) wd.push_back(bf ? shifted(hq.cols[i], qj.cols[i], sigma) : plain(hq.cols[i]));
       std::vector<cd> cj, rj;
       const bool last = j == m - 1;
       // a preconditioner's basis: one pass unless the projection cancels
       // more than 99.9% of a column (R keeps ~1e-13 relative accuracy)
-      if (int st = cgs_cholqr(qall, descs_of(hq), hq, cj, rj, ok, !last, 1e-3)) return st;
+      if (int st = cgs_cholqr(qall, wd, hq, cj, rj, ok, !last, 1e-3)) return st;
       if (!ok) rj.assign(size_t(kb) * kb, 0.0);  // (H - sigma) Q_j lies in span(Q): the space is exhausted
       hc.push_back(cj);
       hr.push_back(rj);

@@ -39,8 +39,7 @@ struct Dbl2 {
 };
 
 // One column of a tall block as seen by the block kernels: the value at row r
-// is a[r] - sig * b[r] (b may be null; the combinations take a alone).  Used to form
-// A Q - sigma Q on the fly.
+// is a[r] - sig * b[r] (b may be null), formed in FP64.  Used for A Q - sigma Q on the fly.
 // In the Gram kernel, bslot >= 0 also stores the raw b[r] in that extra
 // column slot (so Q is read once when both B and Q are operands), and a
 // column with a == nullptr is one whose values another column supplies.
@@ -56,7 +55,7 @@ struct MatvecCoef {
   double s2_re, s2_im;   // e^{-2 i theta} / delta^2 multiplying the kinetic sum
   double c1_re, c1_im;   // e^{-i theta} multiplying the real potential
   double inv_d3;         // 1 / delta^3 (electron-electron term)
-  double sh_re = 0.0, sh_im = 0.0;  // the two-electron passes apply H - (sh_re + i sh_im)
+  double sh_re = 0.0, sh_im = 0.0;  // the two-electron passes apply H - (sh_re + i sh_im) (FP64 forms only)
 };
 
 // Sets every kernel's function attributes and caches the occupancy figures the

@@ -639,6 +639,8 @@ bool set_lds(const void *kernel, size_t lds, std::atomic<bool> &done) {
   return true;
 }
 
+// A shift is applied in FP64 only: a complex64 basis takes it in the block kernels
+// (a - sig b of the descriptors), which form it in FP64.
 bool shifted(const MatvecCoef &cf) { return cf.sh_re != 0.0 || cf.sh_im != 0.0; }
 
 // LDS bytes of the passes' two cubes of reals.
@@ -650,8 +652,10 @@ constexpr size_t cube_lds() {
 template <int NN, typename R, typename XT, typename ZT>
 bool pass1_setup() {
   static std::atomic<bool> plain{false}, shifted{false};
-  return set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, false>), cube_lds<NN, R>(), plain) &&
-         set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, true>), cube_lds<NN, R>(), shifted);
+  if constexpr (sizeof(R) == 8) {
+    if (!set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, true>), cube_lds<NN, R>(), shifted)) return false;
+  }
+  return set_lds(reinterpret_cast<const void *>(&k_pass1<NN, R, XT, ZT, false>), cube_lds<NN, R>(), plain);
 }
 
 template <int NN, typename R, typename XT, typename YT>
@@ -664,12 +668,16 @@ template <int NN, typename R, typename XT, typename ZT>
 hipError_t pass1_nn(const ColPtrs &xs, const ColPtrsW &zs, int ncols, const PotArgs &pot, double w, hipStream_t s) {
   if (!pass1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
   const dim3 g(NN * NN * NN, unsigned(ncols)), b(cube_threads<NN>());
-  if (shifted(pot.cf))
-    hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, true>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv, pot.cf,
-                       w);
-  else
-    hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, false>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv,
-                       pot.cf, w);
+  if (shifted(pot.cf)) {
+    if constexpr (sizeof(R) == 8) {
+      hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, true>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv,
+                         pot.cf, w);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL((k_pass1<NN, R, XT, ZT, false>), g, b, (cube_lds<NN, R>()), s, xs, zs, pot.vn, pot.tinv, pot.cf,
+                     w);
   return hipGetLastError();
 }
 
@@ -695,8 +703,10 @@ constexpr size_t plane2_lds() {
 template <int NN, typename R, typename XT, typename ZT>
 bool plane1_setup() {
   static std::atomic<bool> plain{false}, shifted{false};
-  return set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, false>), plane1_lds<NN, R>(), plain) &&
-         set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, true>), plane1_lds<NN, R>(), shifted);
+  if constexpr (sizeof(R) == 8) {
+    if (!set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, true>), plane1_lds<NN, R>(), shifted)) return false;
+  }
+  return set_lds(reinterpret_cast<const void *>(&k_plane1<NN, R, XT, ZT, false>), plane1_lds<NN, R>(), plain);
 }
 
 template <int NN, typename R, typename XT, typename ZT, typename YT>
@@ -717,12 +727,16 @@ hipError_t plane1_nn(const void *x, void *z, const PotArgs &pot, hipStream_t s) 
   const dim3 g(NN * NN * NN, (NN + G - 1) / G), b(round_up(NN * G, 64));
   const XT *xx = static_cast<const XT *>(x);
   ZT *zz = static_cast<ZT *>(z);
-  if (shifted(pot.cf))
-    hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, true>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
-                       pot.cf);
-  else
-    hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, false>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
-                       pot.cf);
+  if (shifted(pot.cf)) {
+    if constexpr (sizeof(R) == 8) {
+      hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, true>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
+                         pot.cf);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL((k_plane1<NN, R, XT, ZT, false>), g, b, (plane1_lds<NN, R>()), s, xx, zz, pot.vn, pot.tinv,
+                     pot.cf);
   return hipGetLastError();
 }
 
@@ -854,7 +868,7 @@ bool general_by_planes(int nn) { return nn > kCubeMaxNN; }
 bool general_direct(int nn) { return nn <= kDirectMaxNN; }
 
 hipError_t launch_direct(int nn, int io, const void *x, void *y, int ncols, const PotArgs &pot, hipStream_t s) {
-  if (ncols < 1 || ncols > kBatchMax) return hipErrorInvalidValue;
+  if (ncols < 1 || ncols > kBatchMax || (io != kIoF64 && shifted(pot.cf))) return hipErrorInvalidValue;
   ColPtrs xs{};
   ColPtrsW ys{};
   const size_t bytes = size_t(nn) * nn * nn * nn * nn * nn * (io == kIoF32 ? 8 : 16);
@@ -1024,6 +1038,18 @@ __device__ __forceinline__ double2 col_value(const ColDesc &c, int64_t r) {
   o.x = va.x - (c.sig_re * vb.x - c.sig_im * vb.y);
   o.y = va.y - (c.sig_re * vb.y + c.sig_im * vb.x);
   return o;
+}
+
+// Rows r, r + 1 of a descriptor's column, as ld_col2 reads them.
+__device__ __forceinline__ void col_values2(const ColDesc &c, int64_t r, bool two, double2 &v0, double2 &v1) {
+  ld_col2(c.a, c.fmt, r, two, v0, v1);
+  if (c.b == nullptr) return;
+  double2 b0, b1;
+  ld_col2(c.b, c.fmt, r, two, b0, b1);
+  v0.x -= c.sig_re * b0.x - c.sig_im * b0.y;
+  v0.y -= c.sig_re * b0.y + c.sig_im * b0.x;
+  v1.x -= c.sig_re * b1.x - c.sig_im * b1.y;
+  v1.y -= c.sig_re * b1.y + c.sig_im * b1.x;
 }
 
 // The row tiles a workgroup of the Gram kernels takes, in order.
@@ -1503,24 +1529,30 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
   }
   // element p of this thread: row pair e % HALF of input column e / HALF
   const void *pa[PMAX];
+  const void *pb[PMAX];
   int pf[PMAX];
 #pragma unroll
   for (int p = 0; p < PMAX; ++p) {
     const int e = tid + kCombThreads * p;
     pa[p] = nullptr;
+    pb[p] = nullptr;
     pf[p] = 0;
     if (e < HALF * nin) {
       const ColDesc &dc = descs[e / HALF];
       pa[p] = dc.a;
+      pb[p] = dc.b;
       pf[p] = dc.fmt;
     }
   }
-  double2 va[PMAX][2];
+  double2 va[PMAX][2], vb[PMAX][2];
   auto fetch = [&](int64_t rb) {
 #pragma unroll
     for (int p = 0; p < PMAX; ++p) {
       const int64_t r = rb + 2 * ((tid + kCombThreads * p) % HALF);
-      if (pa[p] != nullptr && r < d) ld_col2(pa[p], pf[p], r, r + 1 < d, va[p][0], va[p][1]);
+      if (pa[p] != nullptr && r < d) {
+        ld_col2(pa[p], pf[p], r, r + 1 < d, va[p][0], va[p][1]);
+        if (pb[p] != nullptr) ld_col2(pb[p], pf[p], r, r + 1 < d, vb[p][0], vb[p][1]);
+      }
     }
   };
   const int64_t ntile = (d + kCombRows - 1) / kCombRows;
@@ -1536,7 +1568,14 @@ __global__ __launch_bounds__(kCombThreads) void k_combine(const ColDesc *__restr
       const int r = 2 * (e % HALF), c = e / HALF;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (r + h < nr) tin[c * kCombRows + r + h] = va[p][h];
+        if (r + h >= nr) continue;
+        double2 v = va[p][h];
+        if (pb[p] != nullptr) {
+          const ColDesc &dc = descs[c];
+          v.x -= dc.sig_re * vb[p][h].x - dc.sig_im * vb[p][h].y;
+          v.y -= dc.sig_re * vb[p][h].y + dc.sig_im * vb[p][h].x;
+        }
+        tin[c * kCombRows + r + h] = v;
       }
     }
     __syncthreads();
@@ -1677,9 +1716,9 @@ __global__ __launch_bounds__(256) void k_combine_w(const ColDesc *__restrict__ d
         for (int k = 0; k < RPL; ++k) v[k] = make_double2(0.0, 0.0);
         if (ok0) {
           if constexpr (RPL == 2) {
-            ld_col2(dc.a, dc.fmt, r0, ok1, v[0], v[RPL - 1]);
+            col_values2(dc, r0, ok1, v[0], v[RPL - 1]);
           } else {
-            v[0] = ld_col(dc.a, dc.fmt, r0);
+            v[0] = col_value(dc, r0);
           }
         }
         add_products<JN, RPL>(v, cm + size_t(JN) * i, ax, ay);
@@ -1766,7 +1805,7 @@ __global__ __launch_bounds__(512) void k_combine_sym(const ColDesc *__restrict__
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         v[k] = make_double2(0.0, 0.0);
-        if (ok[k]) v[k] = ld_col(dc.a, dc.fmt, at[k]);
+        if (ok[k]) v[k] = col_value(dc, at[k]);
       }
       add_products<JN, 2>(v, cm + size_t(JN) * i, ax, ay);
     }
