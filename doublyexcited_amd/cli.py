@@ -164,7 +164,7 @@ def run(cfg: dict, out=sys.stdout, workdir: str | Path = ".") -> dict:
     import torch
 
     from .eigvecs import read_eigenvectors, write_eigenvectors
-    from .hamiltonian import HeliumGrid
+    from .hamiltonian import HeliumGrid, with_room
     from .orbitals import heplus_orbitals
 
     if cfg["NUCLEI"] != 1 or not cfg["NUC_ON_GRID"]:
@@ -188,11 +188,11 @@ def run(cfg: dict, out=sys.stdout, workdir: str | Path = ".") -> dict:
                     tfactor=int(cfg["TFACTOR"])) as g:
         if cfg["READVECS"]:
             vecs = read_eigenvectors(bindir / str(cfg["INVECFILE"]), m=g.m, num=nev)
-            x = torch.from_numpy(vecs.reshape(-1).copy()).to("cuda")
+            x = with_room(g.device, lambda: torch.from_numpy(vecs.reshape(-1).copy()).to("cuda"))
             ex = np.zeros(nev, dtype=np.complex128)
             for j in range(nev):
                 xj = x[j * g.d:(j + 1) * g.d]
-                y = torch.empty_like(xj)
+                y = with_room(g.device, lambda: torch.empty_like(x[:g.d]))
                 g.matvec_device(xj, y, 1, symmetry=sym)
                 ex[j] = complex(torch.vdot(xj, y).item() / torch.vdot(xj, xj).item())
         else:

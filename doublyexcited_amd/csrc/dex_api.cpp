@@ -98,7 +98,8 @@ hipError_t scratch_address(int device, void **ptr) {
 // most an eighth of the device's memory stays listed (the blocks idle longest go
 // first), all of it is freed when the last context on the device is destroyed,
 // and when an allocation of this library fails the list is freed and the
-// allocation tried again.
+// allocation tried again.  Other allocators of the process cannot reach it: they ask
+// for it with dex_trim_idle, as the request server does to stay under its cap.
 namespace {
 struct IdleBlocks {
   std::mutex mu;
@@ -112,13 +113,23 @@ void free_blocks(const std::vector<std::pair<void *, size_t>> &blocks) {
   for (const auto &b : blocks) (void)hipFree(b.first);
 }
 
-void drop_idle(int device) {
+// Takes the blocks idle longest off the list until at most `keep` bytes stay (with its
+// lock held); the caller frees them.
+std::vector<std::pair<void *, size_t>> unlist(IdleBlocks &l, size_t keep) {
+  size_t n = 0;
+  while (l.bytes > keep) l.bytes -= l.idle[n++].second;
+  const auto end = l.idle.begin() + std::ptrdiff_t(n);
+  std::vector<std::pair<void *, size_t>> out(l.idle.begin(), end);
+  l.idle.erase(l.idle.begin(), end);
+  return out;
+}
+
+void drop_idle(int device, size_t keep = 0) {
   std::vector<std::pair<void *, size_t>> out;
   {
     IdleBlocks &l = g_idle[device];
     std::lock_guard<std::mutex> lk(l.mu);
-    out.swap(l.idle);
-    l.bytes = 0;
+    out = unlist(l, keep);
   }
   free_blocks(out);
 }
@@ -157,10 +168,7 @@ void block_give(int device, void *ptr, size_t bytes) {
     std::lock_guard<std::mutex> lk(l.mu);
     l.idle.emplace_back(ptr, bytes);
     l.bytes += bytes;
-    size_t n = 0;
-    while (l.bytes > l.cap) l.bytes -= l.idle[n++].second;
-    out.assign(l.idle.begin(), l.idle.begin() + std::ptrdiff_t(n));
-    l.idle.erase(l.idle.begin(), l.idle.begin() + std::ptrdiff_t(n));
+    out = unlist(l, l.cap);
   }
   free_blocks(out);
 }
@@ -2145,9 +2153,10 @@ int gplmr_run(dex_ctx *c, const std::vector<Dbl2 *> &xcols, int nconv, cd *e_out
 
 }  // namespace
 
-// Small grids: a margin of up to 16 vectors in the count below (512 MiB at
-// most), for work vectors of other sizes that stay listed while contexts live.
-// Admission decisions depend on it.
+// Small grids: a margin of up to 16 vectors in the count below (512 MiB at most), for
+// what a context allocates beside the counted vectors: the general matvec's intermediates
+// of several columns (64 MiB at most, general_cols) and the rounding of each vector's
+// allocation.  Admission decisions depend on it.
 int64_t margin_vectors(int64_t d) {
   const int64_t b = (int64_t(512) << 20) / (d * 16);
   return b >= 2 ? std::min<int64_t>(b, dex::kBatchMax) : 0;
@@ -2193,6 +2202,19 @@ extern "C" int64_t dex_gplmr_footprint(const dex_ctx *c, int32_t nev, int32_t ns
                                        const dex_solve_opts *opts) {
   if (!c) return -1;
   return solve_footprint(c->nn, c->p.precision, nev, ns, inner_iter, opts);
+}
+
+extern "C" int64_t dex_idle_bytes(int32_t device) {
+  if (device < 0 || device >= kMaxDevices) return -1;
+  IdleBlocks &l = g_idle[device];
+  std::lock_guard<std::mutex> lk(l.mu);
+  return int64_t(l.bytes);
+}
+
+extern "C" int dex_trim_idle(int32_t device, int64_t keep_bytes) {
+  if (device < 0 || device >= kMaxDevices || keep_bytes < 0) return fail(DEX_EINVAL, "dex_trim_idle: bad argument");
+  drop_idle(device, size_t(keep_bytes));
+  return DEX_OK;
 }
 
 extern "C" int64_t dex_solve_footprint(const dex_params *p, int32_t nev, int32_t ns, int32_t inner_iter,

@@ -62,6 +62,31 @@ def _check_dev(t, ncols: int, d: int, device: int, single: bool = False, name: s
         raise DexError(_lib.DEX_ESIZE, f"{name} holds {t.numel()} entries, the call needs {ncols} x {d}")
 
 
+def idle_bytes(device: int = 0) -> int:
+    """Bytes of work vectors the library keeps on a GPU between calls
+    (dex_idle_bytes): at most an eighth of its memory, none once every
+    ``HeliumGrid`` there is closed."""
+    return int(_lib.load().dex_idle_bytes(device))
+
+
+def trim_idle(device: int = 0, keep_bytes: int = 0) -> None:
+    """Gives idle work vectors back to the device until at most ``keep_bytes``
+    stay, for allocations of other owners (dex_trim_idle)."""
+    check(_lib.load().dex_trim_idle(device, int(keep_bytes)))
+
+
+def with_room(device: int, make):
+    """``make()``, a torch allocation; once more without the idle work vectors
+    where it runs out of memory."""
+    import torch
+
+    try:
+        return make()
+    except torch.OutOfMemoryError:
+        trim_idle(device)
+        return make()
+
+
 @dataclasses.dataclass
 class SolveResult:
     e: np.ndarray
@@ -307,7 +332,8 @@ class HeliumGrid:
             raise DexError(_lib.DEX_ESIZE, "orbitals must be an M x numorbs array")
         k = orb.shape[1]
         orb = np.ascontiguousarray(orb.reshape(-1, order="F"))  # column-major, flat
-        psi = torch.empty(self.d * numout, dtype=torch.complex128, device=f"cuda:{self.device}")
+        psi = with_room(self.device, lambda: torch.empty(self.d * numout, dtype=torch.complex128,
+                                                         device=f"cuda:{self.device}"))
         e0 = np.zeros(numout, dtype=np.complex128)
         ex = np.zeros(numout, dtype=np.complex128)
         check(self._lib.dex_diagsubspace_device(self._ctx, orb.view(np.float64).ctypes.data_as(_dp), k,

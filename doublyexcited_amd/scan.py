@@ -41,13 +41,13 @@ def theta_scan(points, sigma: complex, nev: int, tol: float, ns: int = 1, inner_
     import torch
 
     from .eigvecs import sixd_fix, write_eigenvectors
-    from .hamiltonian import HeliumGrid
+    from .hamiltonian import HeliumGrid, with_room
 
     out: list[ScanPoint] = []
     prev, prev_n = None, None
     for i, (n, delta, theta) in enumerate(points):
         with HeliumGrid(n, delta, theta, precision=precision, device=device) as g:
-            x = torch.empty(g.d * nev, dtype=torch.complex128, device=f"cuda:{device}")
+            x = with_room(device, lambda: torch.empty(g.d * nev, dtype=torch.complex128, device=f"cuda:{device}"))
             use_warm = warm and prev is not None
             if use_warm and prev_n == n:
                 x.copy_(prev)

@@ -3,8 +3,9 @@
 Requests (grid N, spacing, scaling angle theta, complex shift sigma, block
 size, tolerance, precision) arrive over time.  The scheduler admits a request
 as soon as (a) a worker slot is free and (b) its device footprint fits, together
-with every solve already on the GPU, under the HBM cap.  Each admitted solve owns
-a context (its own HIP stream and buffers), so solves overlap on the device.
+with every solve already on the GPU, under the HBM cap; work vectors that the library
+keeps from finished solves are given back as far as the cap needs it.  Each admitted
+solve owns a context (its own HIP stream and buffers), so solves overlap on the device.
 Results carry arrival->completion latency.  A request that fails, whether it is
 rejected at admission or errors in the solver, yields an error result; it never
 stops the service.
@@ -204,6 +205,17 @@ class Server:
             for g in self._active.values():
                 g.stop()
 
+    def _make_room(self) -> None:
+        """Before an admitted solve allocates: the idle work vectors of finished
+        solves and every reservation together stay under the cap.  (They stay so
+        until the next admission: what a solve returns to the list, its
+        reservation covered until then.)"""
+        from .hamiltonian import trim_idle
+
+        with self._cv:
+            keep = self.cap - self._in_use
+        trim_idle(self.device, max(0, int(keep)))
+
     def _execute(self, req: Request):
         """The request's solve on the device: (solve result, FP64 residuals of
         the returned pairs, sampled kernel statistics, kernel totals).  The
@@ -211,10 +223,12 @@ class Server:
         import torch
 
         import doublyexcited_amd as dex
+        from .hamiltonian import with_room
 
         torch.cuda.set_device(self.device)
         with dex.HeliumGrid(req.n, req.delta, req.theta, precision=req.precision, device=self.device) as g:
-            x = torch.empty(g.d * req.nev, dtype=torch.complex128, device=f"cuda:{self.device}")
+            x = with_room(self.device, lambda: torch.empty(g.d * req.nev, dtype=torch.complex128,
+                                                           device=f"cuda:{self.device}"))
             g.fill_gaussian_device(x, req.nev, seed=req.seed, symmetry=1)
             if self.timing:
                 g.set_kernel_timing(self.timing)
@@ -237,6 +251,7 @@ class Server:
     def _solve(self, req: Request, t_admit: float, t0: float) -> Result:
         """Runs one request; t_admit and the returned times are relative to t0."""
         try:
+            self._make_room()
             r, res, stats, totals = self._execute(req)
             done = time.time() - t0
             conv = int(np.sum(res <= req.tol))

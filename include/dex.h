@@ -292,14 +292,26 @@ int dex_heplus_lanczos_device(dex_ctx *ctx, int32_t blocksize, int32_t kdim, int
  * opts: inner_block, guard and inner_fp32; NULL for the defaults) holds on this
  * context: the caller's block X, the solver's work vectors (complex64 search
  * blocks in an FP32 context) and the context's own fixed buffers (tables,
- * block-kernel scratch, matvec intermediates).  No reference counterpart (the
- * reference allocates its work arrays inside GPLMR_EIG, gplmr.F90:31-36). */
+ * block-kernel scratch, matvec intermediates).  Idle work vectors (dex_idle_bytes) are
+ * not counted.  No reference counterpart (the reference allocates its work arrays inside
+ * GPLMR_EIG, gplmr.F90:31-36). */
 int64_t dex_gplmr_footprint(const dex_ctx *ctx, int32_t nev, int32_t ns, int32_t inner_iter,
                             const dex_solve_opts *opts);
 /* The same figure from the parameters alone (p->n and p->precision), before
  * any context exists and without a device: a request server's admission test. */
 int64_t dex_solve_footprint(const dex_params *p, int32_t nev, int32_t ns, int32_t inner_iter,
                             const dex_solve_opts *opts);
+
+/* Idle work vectors.  A solve, inner solve, residual check or host-pointer call returns
+ * its work vectors to a list of its device, from which later calls of any context take
+ * vectors of the same size.  The list holds at most an eighth of the device's memory; it
+ * is freed when the device's last context is destroyed and when an allocation of the
+ * library fails.  Other allocators of the process cannot use what is listed:
+ * dex_idle_bytes says how much that is (-1: bad ordinal), and dex_trim_idle frees the
+ * vectors idle longest until at most keep_bytes stay.  Both from any thread, and
+ * neither changes the thread's current device.  No reference counterpart. */
+int64_t dex_idle_bytes(int32_t device);
+int dex_trim_idle(int32_t device, int64_t keep_bytes);
 
 /* Eigenvector files in the reference's format, READWRITE_EIGENVECTORS
  * (utils.F90:82-181): a Fortran unformatted sequential file (gfortran record

@@ -88,3 +88,56 @@ def test_inner_solve_uses_its_exchange_symmetry(dex):
             assert (totals["symadd"][0] > 0) == (sym != 0) and (totals["pass2"][0] > 0) == (sym == 0)
             got[sym] = y
         assert (got[0] - got[1]).abs().max().item() <= 1e-9 * got[0].abs().max().item()
+
+
+def test_idle_work_vectors_are_given_back_on_request(dex):
+    print("case: trim idle", flush=True)
+    with dex.HeliumGrid(4, 0.5, 0.3) as g:
+        x = _block(g, 4, 1)
+        y, z = torch.empty_like(x), torch.empty_like(x)
+        g.precblock_device(x, y, 4, -0.7 - 0.002j, 6, symmetry=1)
+        vec, held = 16 * g.d, dex.idle_bytes()
+        assert held >= 28 * vec and held % vec == 0
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        dex.trim_idle(keep_bytes=held - 3 * vec + 1)  # whole vectors: one byte less than three takes three
+        assert dex.idle_bytes() == held - 3 * vec
+        dex.trim_idle()
+        assert dex.idle_bytes() == 0 and torch.cuda.mem_get_info()[0] - free >= held
+        g.precblock_device(x, z, 4, -0.7 - 0.002j, 6, symmetry=1)
+        assert torch.equal(y, z) and dex.idle_bytes() == held
+
+
+def test_server_keeps_idle_work_vectors_under_its_cap(dex):
+    """Requests one after the other while another context stays open: each leaves its work
+    vectors listed, in sizes (three grids, two formats) that the next cannot use.  The cap
+    holds the largest request; the device's use beyond the start stays under it, where all
+    that the requests leave would not."""
+    from doublyexcited_amd.serve import Request, Server
+
+    print("case: server cap with idle work vectors", flush=True)
+    reqs = [Request(arrival=0.0, rid=i, n=n, delta=0.5, theta=0.3, sigma=-0.78 - 0.002j, nev=8, tol=1e-9, maxit=2,
+                    seed=i, inner_iter=4, guard=2, precision=p)
+            for i, (n, p) in enumerate(((6, "fp64"), (6, "mixed"), (5, "fp64"), (5, "mixed"), (4, "fp64")))]
+    need = [r.need() for r in reqs]
+    used = []  # bytes after each request
+
+    class Watched(Server):
+        def _execute(self, req):
+            out = super()._execute(req)
+            torch.cuda.empty_cache()
+            torch.cuda.synchronize()
+            used.append(base - torch.cuda.mem_get_info()[0])
+            return out
+
+    with dex.HeliumGrid(1, 0.5, 0.3):
+        dex.trim_idle()
+        torch.cuda.empty_cache()
+        torch.cuda.synchronize()
+        base = torch.cuda.mem_get_info()[0]
+        cap = max(need)
+        out = Watched(hbm_cap_bytes=cap, slots=1).run(reqs, realtime=False)
+        assert all(r.ok for r in out), [r.error for r in out]
+        print("case: used", used, need, flush=True)
+        assert used[0] > 0.5 * need[0] and max(used) <= cap, (used, need)
+        dex.trim_idle()

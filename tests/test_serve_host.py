@@ -154,3 +154,61 @@ def test_plans_fit_the_cap_and_widen_where_memory_allows():
             assert plans["mixed"]["ns"] >= plans["fp64"]["ns"] or plans["mixed"]["guard"] > plans["fp64"]["guard"]
     p21 = plan_solve(10, 16, "fp64", cap)
     assert p21 == dict(ns=1, inner_iter=4, inner_block=4, guard=0)
+
+
+def test_idle_work_vectors_leave_room_for_the_reservations(monkeypatch):
+    """Before each admitted solve allocates, the server has the library give back its idle
+    work vectors beyond what the cap leaves beside every reservation."""
+    from types import SimpleNamespace
+
+    from doublyexcited_amd import hamiltonian
+
+    trims = []
+    monkeypatch.setattr(hamiltonian, "trim_idle", lambda device=0, keep_bytes=0: trims.append((device, keep_bytes)))
+
+    class FakeServer(Server):
+        def _execute(self, req):
+            return (SimpleNamespace(converged=True, iterations=1, e=np.zeros(req.nev, complex), matvecs=1,
+                                    fp64_restarts_used=0), np.zeros(req.nev), None, None)
+
+    reqs = [Request(arrival=0.0, rid=i, n=n, delta=0.5, theta=0.3, sigma=-0.78 + 0j, nev=4, tol=1e-7)
+            for i, n in enumerate((6, 5, 7))]
+    cap = max(r.need() for r in reqs) + 5e9
+    out = FakeServer(hbm_cap_bytes=cap, slots=1, device=3).run(reqs, realtime=False)
+    assert all(r.ok for r in out)
+    assert trims == [(3, int(cap - r.need())) for r in reqs]
+
+
+def test_idle_memory_calls_without_a_device():
+    import pytest
+
+    import doublyexcited_amd as dex
+
+    assert dex.idle_bytes(0) == 0 and dex.idle_bytes(-1) == -1
+    dex.trim_idle(0, 0)
+    for device, keep in ((-1, 0), (0, -1), (1 << 20, 0)):
+        with pytest.raises(dex.DexError):
+            dex.trim_idle(device, keep)
+
+
+def test_a_torch_allocation_out_of_memory_is_tried_without_the_idle_vectors(monkeypatch):
+    import pytest
+    import torch
+
+    from doublyexcited_amd import hamiltonian
+
+    trims = []
+    monkeypatch.setattr(hamiltonian, "trim_idle", lambda device=0, keep_bytes=0: trims.append((device, keep_bytes)))
+
+    def make():
+        if not trims:
+            raise torch.OutOfMemoryError("full")
+        return "memory"
+
+    assert hamiltonian.with_room(2, make) == "memory" and trims == [(2, 0)]
+
+    def never():
+        raise torch.OutOfMemoryError("full")
+
+    with pytest.raises(torch.OutOfMemoryError):
+        hamiltonian.with_room(2, never)
