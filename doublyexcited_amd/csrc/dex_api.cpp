@@ -206,6 +206,7 @@ struct dex_ctx {
   dex::MatvecCoef coef{};
   hipStream_t stream = nullptr;
   bool fast64 = false, fast32 = false;
+  bool axes = false;  // FP64 by launch_axes
   void *d_u = nullptr;  // the general matvec's intermediates (ensure_u)
   size_t u_bytes = 0;
   void *d_scratch = nullptr;  // this device's copy of `scratch` (dex_matvec_noalloc)
@@ -462,8 +463,12 @@ int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, i
 }
 
 // H - shift on one complex128 column in FP64 with the intermediate in Y's own storage
-// (grids without an FP64 cube; x and y must differ).
+// (grids without an FP64 cube, and cross-check contexts; x and y must differ).
 int generic_passes(dex_ctx *c, const void *x, void *y, cd shift = 0.0) {
+  if (c->axes) {
+    DEX_HIP(dex::launch_axes(c->nn, static_cast<const Dbl2 *>(x), static_cast<Dbl2 *>(y), pot_args(c, shift), c->stream));
+    return 0;
+  }
   DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, pot_args(c, shift), c->stream));
   DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, 1, c->coef, c->stream));
   return 0;
@@ -854,10 +859,13 @@ int dex_ctx_create(const dex_params *p, dex_ctx **out) {
   c->coef.inv_d3 = 1.0 / (p->delta * p->delta * p->delta);
   c->fast64 = dex::fast_matvec_supported(nn, false);
   c->fast32 = dex::fast_matvec_supported(nn, true);
-  // DEX_MATVEC=generic takes the grids without an FP64 cube's route even where the LDS
-  // two-pass kernels exist (used to cross-check the two implementations).
+  // DEX_MATVEC=generic: FP64 by the kernels of launch_axes at every grid, to cross-check
+  // the others.
   if (const char *mv = std::getenv("DEX_MATVEC"))
-    if (std::strcmp(mv, "generic") == 0) c->fast64 = false;
+    if (std::strcmp(mv, "generic") == 0) {
+      c->axes = true;
+      c->fast64 = false;
+    }
   // (the device ordinal was accepted by hipSetDevice; the scratch address below bounds it)
   if (p->device < 0 || p->device >= kMaxDevices) {
     delete c;
@@ -2573,7 +2581,7 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
   DEX_HIP(blocks.take(&v, size_t(c->d) * sizeof(Dbl2)));
   Dbl2 *ax = static_cast<Dbl2 *>(v);
   int st = DEX_OK;
-  if (dex::general_by_planes(c->nn)) {
+  if (dex::general_by_planes(c->nn) && !c->axes) {
     // the sums come from the matvec's last pass, 128 columns to a wait
     const double dd = double(c->d);
     for (int j0 = 0; j0 < nev; j0 += kNormCols) {

@@ -103,6 +103,9 @@ hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y
 // columns; y may overlap no column of x.
 bool general_direct(int nn);
 hipError_t launch_direct(int nn, int io, const void *x, void *y, int ncols, const PotArgs &pot, hipStream_t s);
+// General vectors in FP64 by kernels apart from the passes above (cross-check; y must not
+// overlap x).
+hipError_t launch_axes(int nn, const Dbl2 *x, Dbl2 *y, const PotArgs &pot, hipStream_t s);
 // out[0] = ||H x - e x||^2 and out[1] = ||x||^2 of one complex128 column in FP64
 // (general_by_planes grids; z: D entries; partial: 2 doubles a run tile, at most
 // 2 (NN^4 / 8 + 8)).

@@ -606,6 +606,63 @@ __global__ __launch_bounds__(direct_threads<NN>()) void k_direct(ColPtrs xs, Col
   if (e1 < N3) static_cast<XT *>(ys.p[blockIdx.y])[p + N3 * q] = o;
 }
 
+// ---- cross-check ---------------------------------------------------------------
+// General vectors in FP64 by seven launches that share nothing with the passes above
+// (no LDS, no even-odd lines, no fused axes): one launch an axis, a thread a line of
+// stride `stride`, and the potential's.  Contexts made under DEX_MATVEC=generic take
+// them, so that the two programs can be compared at any grid; no other context does
+// (NN = 25: 16.8 ms a vector where the planes take 6.9).
+template <int NN>
+__global__ __launch_bounds__(256) void k_axis(const double2 *__restrict__ x, double2 *__restrict__ y, int64_t stride,
+                                              int64_t nlines, int accumulate) {
+  const int64_t line = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (line >= nlines) return;
+  const int64_t off = line % stride + line / stride * stride * NN;
+  double2 v[NN];
+#pragma unroll
+  for (int l = 0; l < NN; ++l) v[l] = x[off + stride * l];
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    double2 o = accumulate ? y[off + stride * i] : make_double2(0.0, 0.0);
+    double ar = 0.0, ai = 0.0;
+#pragma unroll
+    for (int l = 0; l < NN; ++l) {
+      ar += tau_rt(l - i) * v[l].x;
+      ai += tau_rt(l - i) * v[l].y;
+    }
+    o.x += ar;
+    o.y += ai;
+    y[off + stride * i] = o;
+  }
+}
+
+// Y = s2 Y + (c1 Vr - shift) o X
+__global__ __launch_bounds__(256) void k_potential(const double2 *__restrict__ x, double2 *__restrict__ y,
+                                                   const double *__restrict__ vn, const double *__restrict__ tinv,
+                                                   int nn, int64_t m, MatvecCoef cf) {
+  const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (idx >= m * m) return;
+  const int p = int(idx % m), q = int(idx / m), L = 2 * nn + 1;
+  const int ti = (q % nn - p % nn + nn) +
+                 L * ((q / nn % nn - p / nn % nn + nn) + L * (q / (nn * nn) - p / (nn * nn) + nn));
+  const double vr = vn[p] + vn[q] + tinv[ti] * cf.inv_d3;
+  const double fr = vr * cf.c1_re - cf.sh_re, fi = vr * cf.c1_im - cf.sh_im;
+  const double2 xv = x[idx], k = y[idx];
+  y[idx] = make_double2(cf.s2_re * k.x - cf.s2_im * k.y + (fr * xv.x - fi * xv.y),
+                        cf.s2_re * k.y + cf.s2_im * k.x + (fr * xv.y + fi * xv.x));
+}
+
+template <int NN>
+hipError_t axes_nn(const double2 *x, double2 *y, const PotArgs &pot, hipStream_t s) {
+  const int64_t m = int64_t(NN) * NN * NN, lines = m * m / NN;
+  int64_t stride = 1;
+  for (int axis = 0; axis < 6; ++axis, stride *= NN)
+    hipLaunchKernelGGL(k_axis<NN>, dim3(unsigned((lines + 255) / 256)), dim3(256), 0, s, x, y, stride, lines, axis);
+  hipLaunchKernelGGL(k_potential, dim3(unsigned((m * m + 255) / 256)), dim3(256), 0, s, x, y, pot.vn, pot.tinv, NN, m,
+                     pot.cf);
+  return hipGetLastError();
+}
+
 // out[e] = sum over nparts of partial[b nelem + e], one workgroup an element.
 __global__ __launch_bounds__(1024) void k_reduce_wide(const double *__restrict__ partial, int nparts, int nelem,
                                                       double *__restrict__ out) {
@@ -942,6 +999,18 @@ hipError_t launch_general_second(int nn, int io, const void *x, void *z, void *y
       if (io == kIoF32) return pass2_nn<N, float, float2, float2>(x, z, y, ncols, coef, s);        \
       return pass2_nn<N, float, double2, double2>(x, z, y, ncols, coef, s);                        \
     }
+    DEX_NN_LIST(CASE)
+#undef CASE
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_axes(int nn, const Dbl2 *x, Dbl2 *y, const PotArgs &pot, hipStream_t s) {
+  switch (nn) {
+#define CASE(N) \
+  case N:       \
+    return axes_nn<N>(reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y), pot, s);
     DEX_NN_LIST(CASE)
 #undef CASE
     default:
