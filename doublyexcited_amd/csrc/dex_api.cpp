@@ -462,14 +462,27 @@ int apply_h_batch(dex_ctx *c, const void *const *x, void *const *y, int ncols, i
   return 0;
 }
 
+// The general matvec's first pass and the rest by planes, in FP64: bytes and flops an entry
+// (norms: the last pass writes nothing).
+constexpr double kPlaneFirstBytes = 32.0;
+constexpr double plane_rest_bytes(bool norms) { return norms ? 80.0 : 96.0; }
+
 // H - shift on one complex128 column in FP64 with the intermediate in Y's own storage
 // (grids without an FP64 cube, and cross-check contexts; x and y must differ).
 int generic_passes(dex_ctx *c, const void *x, void *y, cd shift = 0.0) {
+  const double dd = double(c->d), nn = double(c->nn);
+  const dex::PotArgs pot = pot_args(c, shift);
   if (c->axes) {
-    DEX_HIP(dex::launch_axes(c->nn, static_cast<const Dbl2 *>(x), static_cast<Dbl2 *>(y), pot_args(c, shift), c->stream));
+    // six axes, all but the first adding to Y, and the potential
+    KTimer kt(c, DEX_K_GENERIC, (32.0 + 5 * 48.0 + 48.0) * dd, (24.0 * nn + 14.0) * dd);
+    DEX_HIP(dex::launch_axes(c->nn, static_cast<const Dbl2 *>(x), static_cast<Dbl2 *>(y), pot, c->stream));
     return 0;
   }
-  DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, pot_args(c, shift), c->stream));
+  {
+    KTimer kt(c, DEX_K_PASS1, kPlaneFirstBytes * dd, (8.0 * nn + 16.0) * dd);
+    DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, x, y, 1, pot, c->stream));
+  }
+  KTimer kt(c, DEX_K_PASS2, plane_rest_bytes(false) * dd, (16.0 * nn + 8.0) * dd);
   DEX_HIP(dex::launch_general_second(c->nn, dex::kIoF64, x, y, y, 1, c->coef, c->stream));
   return 0;
 }
@@ -487,7 +500,6 @@ int apply_h(dex_ctx *c, const Dbl2 *x, Dbl2 *y, bool single, int sym = 0, bool p
     return fast_passes(c, single ? dex::kIoMixed : dex::kIoF64, &xp, &yp, 1, sym, c->d_u,
                        pass_events && c->timing, shift);
   }
-  KTimer kt(c, DEX_K_GENERIC, 32.0 * double(c->d), (24.0 * c->nn + 14.0) * double(c->d));
   if (int st = generic_passes(c, x, y, shift)) return st;
   // The general operator carries the rounding-level exchange-odd (even) part of
   // an exchange-even (odd) x into y, where the transpose-add kernels, which the
@@ -2587,10 +2599,14 @@ extern "C" int dex_residuals_device(dex_ctx *c, const void *x_dev, const double 
     for (int j0 = 0; j0 < nev; j0 += kNormCols) {
       const int k = std::min(nev - j0, kNormCols);
       for (int j = j0; j < j0 + k; ++j) {
-        KTimer kt(c, DEX_K_GENERIC, 112.0 * dd, (24.0 * c->nn + 24.0) * dd);
-        DEX_HIP(dex::launch_general_norms(c->nn, static_cast<const Dbl2 *>(x_dev) + size_t(j) * c->d, ax, e[2 * j],
-                                          e[2 * j + 1], static_cast<double *>(c->d_partial), c->d_dots + 2 * (j - j0),
-                                          {c->d_vn, c->d_tinv, c->coef}, c->stream));
+        const Dbl2 *xj = static_cast<const Dbl2 *>(x_dev) + size_t(j) * c->d;
+        {
+          KTimer kt(c, DEX_K_PASS1, kPlaneFirstBytes * dd, (8.0 * c->nn + 16.0) * dd);
+          DEX_HIP(dex::launch_general_first(c->nn, dex::kIoF64, xj, ax, 1, pot_args(c, 0.0), c->stream));
+        }
+        KTimer kt(c, DEX_K_PASS2, plane_rest_bytes(true) * dd, (16.0 * c->nn + 18.0) * dd);
+        DEX_HIP(dex::launch_general_norms(c->nn, xj, ax, e[2 * j], e[2 * j + 1], static_cast<double *>(c->d_partial),
+                                          c->d_dots + 2 * (j - j0), c->coef, c->stream));
       }
       DEX_HIP(hipStreamSynchronize(c->stream));
       const double *h = c->h_dots;

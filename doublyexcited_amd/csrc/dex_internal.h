@@ -106,11 +106,11 @@ hipError_t launch_direct(int nn, int io, const void *x, void *y, int ncols, cons
 // General vectors in FP64 by kernels apart from the passes above (cross-check; y must not
 // overlap x).
 hipError_t launch_axes(int nn, const Dbl2 *x, Dbl2 *y, const PotArgs &pot, hipStream_t s);
-// out[0] = ||H x - e x||^2 and out[1] = ||x||^2 of one complex128 column in FP64
-// (general_by_planes grids; z: D entries; partial: 2 doubles a run tile, at most
-// 2 (NN^4 / 8 + 8)).
+// launch_general_second's sums in its place: out[0] = ||H x - e x||^2 and out[1] = ||x||^2 of
+// one complex128 column in FP64 (general_by_planes grids; z from launch_general_first;
+// partial: 2 doubles a run tile, at most 2 (NN^4 / 8 + 8)).
 hipError_t launch_general_norms(int nn, const Dbl2 *x, Dbl2 *z, double e_re, double e_im, double *partial,
-                                double *out, const PotArgs &pot, hipStream_t s);
+                                double *out, const MatvecCoef &coef, hipStream_t s);
 // Second pass for X = sign X^T, in place on ncols columns: Y <- Y + sign Y^T.
 hipError_t launch_symfold(int nn, int io, void *const *y, int ncols, int sign, hipStream_t s);
 // G(kl x kr, column-major) = L^H R summed over d rows, kl <= 64, kr <= 128.

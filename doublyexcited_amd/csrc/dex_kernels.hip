@@ -1019,15 +1019,12 @@ hipError_t launch_axes(int nn, const Dbl2 *x, Dbl2 *y, const PotArgs &pot, hipSt
 }
 
 hipError_t launch_general_norms(int nn, const Dbl2 *x, Dbl2 *z, double e_re, double e_im, double *partial,
-                                double *out, const PotArgs &pot, hipStream_t s) {
-  if (!general_by_planes(nn)) return hipErrorInvalidValue;
-  const hipError_t e = launch_general_first(nn, kIoF64, x, z, 1, pot, s);
-  if (e != hipSuccess) return e;
+                                double *out, const MatvecCoef &coef, hipStream_t s) {
   switch (nn) {
 #define CASE(N)                                                                                                  \
   case N:                                                                                                        \
     if constexpr (N > kCubeMaxNN)                                                                                \
-      return plane2_nn<N, double, double2, double2, double2>(x, z, nullptr, pot.cf, s, partial, e_re, e_im, out); \
+      return plane2_nn<N, double, double2, double2, double2>(x, z, nullptr, coef, s, partial, e_re, e_im, out);   \
     return hipErrorInvalidValue;
     DEX_NN_LIST(CASE)
 #undef CASE

@@ -23,37 +23,50 @@ def short(name: str) -> str:
     return n
 
 
-# kernel -> the library's kernel class (the classes of its launch statistics):
-# (class, whether a dispatch of it counts as one launch of the class).  A Gram
-# launch is the MFMA partial kernel plus its partial-sum reduction, a residual
-# step is its kernel plus a reduction, both counted once.
-CLASSES = (
-    ("k_gram_mfma", "gram", True), ("k_gram_pk", "gram", True), ("k_reduce_partials", "gram", False),
-    ("k_combine", "combine", True),
-    ("k_pass1", "pass1", True), ("k_symadd", "symadd", True), ("k_pass2", "pass2", True),
-    ("k_coldots", "coldots", True), ("k_resid", "coldots", True), ("k_reduce_real", "coldots", False),
-)
+# kernel -> (the library's kernel class, launches of the class that one dispatch of the
+# kernel is).  A Gram is its partial kernel and the partial-sum reduction, a residual
+# step its kernel and a reduction, the planes' remaining passes two dispatches (the last
+# followed by a reduction where it forms residual norms), a general matvec of a
+# cross-check context six axes and the potential.
+CLASSES = {
+    "k_pass1": ("pass1", 1.0), "k_plane1": ("pass1", 1.0), "k_direct": ("pass1", 1.0),
+    "k_pass2": ("pass2", 1.0), "k_plane2": ("pass2", 0.5), "k_reduce_wide": ("pass2", 0.0),
+    "k_symfold": ("symadd", 1.0),
+    "k_gram_mfma": ("gram", 1.0), "k_gram_pk": ("gram", 1.0), "k_reduce_partials": ("gram", 0.0),
+    "k_combine": ("combine", 1.0), "k_combine_w": ("combine", 1.0), "k_combine_sym": ("combine", 1.0),
+    "k_coldots": ("coldots", 1.0), "k_resid": ("coldots", 1.0), "k_reduce_real": ("coldots", 0.0),
+    "k_axis": ("generic", 0.0), "k_potential": ("generic", 1.0),
+}
+# kernels outside the classes: start vectors, projections, conversions, the one-electron
+# Lanczos and the orbital subspace
+UNCLASSED = ("k_fill_gaussian", "k_singlet", "k_to_single", "k_to_double", "k_h1", "k_small_dots",
+             "k_small_lincomb", "k_lowrank", "k_ywx")
+
+
+def base(name: str) -> str:
+    """A kernel's own name: no return type, namespaces, template or parameter list."""
+    n = name.replace("(anonymous namespace)::", "")
+    return n.split("<")[0].split("(")[0].replace("void ", "").strip().split("::")[-1]
 
 
 def kernel_class(name: str):
-    n = short(name)
-    for prefix, cls, counts in CLASSES:
-        if n.split("<")[0].split()[-1] == prefix or n.split("<")[0].split()[-1].startswith(prefix + "_"):
-            return cls, counts
-    return None, False
+    """(class, launches of it that a dispatch is); (None, 0.0) outside the classes."""
+    return CLASSES.get(base(name), (None, 0.0))
 
 
 def class_table(rows) -> list[str]:
     tot = {}
     for r in rows:
-        cls, counts = kernel_class(r["Name"])
+        cls, share = kernel_class(r["Name"])
         if cls is None:
-            continue
-        t, n = tot.get(cls, (0.0, 0))
-        tot[cls] = (t + float(r["TotalDurationNs"]), n + (int(r["Calls"]) if counts else 0))
+            if not base(r["Name"]).startswith("k_"):
+                continue  # another library's
+            cls, share = "(no class)", 1.0
+        t, n = tot.get(cls, (0.0, 0.0))
+        tot[cls] = (t + float(r["TotalDurationNs"]), n + share * int(r["Calls"]))
     out = ["| class | launches | total ms | avg us per launch |", "|---|---:|---:|---:|"]
     for cls, (t, n) in sorted(tot.items(), key=lambda kv: -kv[1][0]):
-        out.append(f"| {cls} | {n} | {t / 1e6:.1f} | {t / n / 1e3 if n else 0.0:.1f} |")
+        out.append(f"| {cls} | {n:g} | {t / 1e6:.1f} | {t / n / 1e3 if n else 0.0:.1f} |")
     return out
 
 
@@ -77,7 +90,7 @@ def summarize(path: str, title: str = "", command: str = "") -> str:
                    f"{100.0 * t / tot:.2f} |")
     out.append("")
     out.append("Per kernel class (the library's launch-statistics classes; a Gram launch includes its "
-               "partial-sum reduction):\n")
+               "partial-sum reduction, a plane matvec's remaining passes are one launch):\n")
     out.extend(class_table(rows))
     return "\n".join(out) + "\n"
 

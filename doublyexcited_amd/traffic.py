@@ -11,8 +11,9 @@ calibration kernel (an elementwise multiply that reads and writes 1 GiB) and
 then the profiled solve, whose per-class algorithmic bytes and launch counts it
 writes to ``STATS_JSON``.  The calibration dispatch scales each counter to
 bytes (FETCH_SIZE reports half of the bytes read on this part); per kernel
-class the scaled traffic per dispatch is divided by the algorithmic bytes per
-launch.  Prints a Markdown table and writes ``{"traffic_over_algorithmic":
+class the scaled traffic per launch is divided by the algorithmic bytes per
+launch.  A class with launches but no kernel of its own in the passes is an
+error.  Prints a Markdown table and writes ``{"traffic_over_algorithmic":
 {class: ratio}}`` to ``OUT_JSON`` when given.
 """
 from __future__ import annotations
@@ -22,26 +23,9 @@ import json
 import sys
 from pathlib import Path
 
-# kernel-name prefixes of the library's classes (dex_get_kernel_stats order)
-CLASSES = {
-    "pass1": ("k_pass1",),
-    "pass2": ("k_pass2",),
-    "symadd": ("k_symadd",),
-    "gram": ("k_gram_mfma", "k_gram_pk", "k_reduce_partials"),
-    "combine": ("k_combine",),
-    "coldots": ("k_coldots", "k_resid", "k_reduce_real"),
-    "generic": ("k_axis", "k_potential"),
-}
-# partial-sum reductions that finish a launch of their class (not launches themselves)
-HELPERS = ("k_reduce_partials", "k_reduce_real")
+from .profsummary import base, kernel_class
+
 CAL_BYTES = 1 << 30  # the calibration kernel reads and writes 1 GiB
-
-
-def _base(name: str) -> str:
-    """The kernel's own name: no return type, namespaces, template or
-    parameter list."""
-    n = name.replace("(anonymous namespace)::", "")
-    return n.split("<")[0].split("(")[0].replace("void ", "").strip().split("::")[-1]
 
 
 def _rows(d: Path, counter: str):
@@ -65,14 +49,6 @@ def _per_dispatch(rows):
     return acc
 
 
-def _cls(name: str):
-    base = _base(name)
-    for c, prefixes in CLASSES.items():
-        if any(base.startswith(p) for p in prefixes):
-            return c
-    return None
-
-
 def analyse(fetch_dir, write_dir, stats_json):
     fetch = _per_dispatch(_rows(fetch_dir, "FETCH_SIZE"))
     write = _per_dispatch(_rows(write_dir, "WRITE_SIZE"))
@@ -88,21 +64,21 @@ def analyse(fetch_dir, write_dir, stats_json):
     totals = stats.get("totals", stats)
     table = []
     ratios = {}
-    for c in CLASSES:
-        fv = [v for (n, _), v in fetch.items() if _cls(n) == c and not _base(n).startswith(HELPERS)]
-        wv = [v for (n, _), v in write.items() if _cls(n) == c and not _base(n).startswith(HELPERS)]
-        if not fv or c not in totals:
-            continue
-        launches, alg_bytes = totals[c][0], totals[c][1]
+    for c, (launches, alg_bytes, *_) in totals.items():
         if launches <= 0:
             continue
-        # the class's small helper kernels (partial-sum reductions) add their own traffic
-        fh = [v for (n, _), v in fetch.items() if _cls(n) == c]
-        wh = [v for (n, _), v in write.items() if _cls(n) == c]
-        traffic = (sum(fh) * f_scale + sum(wh) * w_scale) * 1024.0 / len(fv)
+        # the class's kernels, the helpers that finish a launch (partial-sum reductions) among them
+        fv = [(n, v) for (n, _), v in fetch.items() if kernel_class(n)[0] == c]
+        wv = [(n, v) for (n, _), v in write.items() if kernel_class(n)[0] == c]
+        nf, nw = (sum(kernel_class(n)[1] for n, _ in x) for x in (fv, wv))
+        if nf <= 0 or nw <= 0:
+            raise SystemExit(f"class {c}: {launches} launches in {stats_json}, but none of its kernels in the "
+                             f"counter passes (kernels seen: {sorted({base(n) for n, _ in fetch})})")
+        f, w = sum(v for _, v in fv) / nf, sum(v for _, v in wv) / nw
+        traffic = (f * f_scale + w * w_scale) * 1024.0
         alg = alg_bytes / launches
         ratios[c] = traffic / alg
-        table.append((c, len(fv), sum(fv) / len(fv), sum(wv) / len(wv), traffic / 1e9, alg / 1e9, traffic / alg))
+        table.append((c, nf, f, w, traffic / 1e9, alg / 1e9, traffic / alg))
     return cf, cw, f_scale, w_scale, table, ratios
 
 
@@ -114,11 +90,11 @@ def main(argv=None) -> int:
     cf, cw, fs, ws, table, ratios = analyse(argv[0], argv[1], argv[2])
     print(f"Calibration (1 GiB read + 1 GiB written): FETCH_SIZE {cf:.1f} KiB, WRITE_SIZE {cw:.1f} KiB; "
           f"scale FETCH x {fs:.4f}, WRITE x {ws:.4f}\n")
-    print("| class | dispatches | FETCH_SIZE KiB/dispatch | WRITE_SIZE KiB/dispatch | scaled traffic GB/launch "
+    print("| class | launches | FETCH_SIZE KiB/launch | WRITE_SIZE KiB/launch | scaled traffic GB/launch "
           "| algorithmic GB/launch | traffic / algorithmic |")
     print("|---|---:|---:|---:|---:|---:|---:|")
     for c, n, f, w, t, a, r in table:
-        print(f"| {c} | {n} | {f:.1f} | {w:.1f} | {t:.4f} | {a:.4f} | {r:.3f} |")
+        print(f"| {c} | {n:g} | {f:.1f} | {w:.1f} | {t:.4f} | {a:.4f} | {r:.3f} |")
     if len(argv) > 3:
         Path(argv[3]).write_text(json.dumps({"source": argv[2], "traffic_over_algorithmic": ratios}, indent=1))
     return 0

@@ -366,7 +366,7 @@ enum {
   DEX_K_GRAM = 3,    /* block Gram (with its partial-sum reduction) */
   DEX_K_COMBINE = 4, /* block linear combination */
   DEX_K_COLDOTS = 5, /* per-column dots and norms, and the residual step (scaled X, AX and W) */
-  DEX_K_GENERIC = 6, /* generic-grid matvec */
+  DEX_K_GENERIC = 6, /* general matvec of a context made under DEX_MATVEC=generic */
   DEX_KCLASSES = 7
 };
 int dex_get_kernel_stats(dex_ctx *ctx, int32_t kclass, double *total_ms, int64_t *launches,

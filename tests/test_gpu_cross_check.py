@@ -63,3 +63,23 @@ def test_shifted_solve_on_the_other_kernels(dex, monkeypatch):
             out.append(y)
     assert (out[0] - out[1]).abs().max().item() <= 1e-10 * out[1].abs().max().item()
     assert not torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n", [6, 11])
+def test_launches_are_booked_by_the_kernels_that_run(dex, monkeypatch, n):
+    """The planes' passes under pass1 and pass2, with the intermediate in Y (NN=23) and for
+    residual norms too: 32 bytes an entry, then 96, or 80 where the last pass writes sums; a
+    cross-check context's launches, 320 bytes an entry, under generic."""
+    print(f"case: booked launches N={n}", flush=True)
+    monkeypatch.delenv("DEX_MATVEC", raising=False)
+    x = torch.randn((2 * n + 1) ** 6, dtype=torch.complex128, device="cuda")
+    for env in (None, "generic"):
+        if env:
+            monkeypatch.setenv("DEX_MATVEC", env)
+        with dex.HeliumGrid(n, 0.45, 0.3) as g:
+            for call, rest in ((lambda: g.matvec_device(x, torch.empty_like(x), 1), 96),
+                               (lambda: g.residuals_device(x, np.array([-0.7 + 0j])), 80)):
+                g.reset_kernel_stats()
+                call()
+                t = {k: (v[0], v[1] / g.d) for k, v in g.kernel_totals().items() if v[0] and k != "coldots"}
+                assert t == ({"generic": (1, 320)} if env else {"pass1": (1, 32), "pass2": (1, rest)})

@@ -47,3 +47,17 @@ def test_arrays_that_may_be_one_are_not_declared_apart():
         for a in arrays:
             assert re.search(rf"\*\s*{a}\b", got[name]), (name, a)
             assert not re.search(rf"__restrict__\s+{a}\b", got[name]), (name, a)
+
+
+def test_every_kernel_has_its_class_in_the_profile_tools():
+    """A kernel without a class drops out of the class table and the traffic ratios; a class
+    entry without a kernel is stale."""
+    from doublyexcited_amd import _lib, profsummary
+
+    names = {name for name, _, _ in _kernels()}
+    assert set(profsummary.CLASSES) | set(profsummary.UNCLASSED) == names
+    assert not set(profsummary.CLASSES) & set(profsummary.UNCLASSED)
+    assert {c for c, _ in profsummary.CLASSES.values()} == set(_lib.KERNEL_CLASSES)
+    for name, (cls, share) in profsummary.CLASSES.items():
+        full = f"void dex::(anonymous namespace)::{name}<21, double, HIP_vector_type<double, 2u>, false>(dex::Arg, int)"
+        assert profsummary.kernel_class(full) == (cls, share)

@@ -2,6 +2,9 @@
 calibration scaling and per-class traffic / algorithmic ratios."""
 import json
 
+import pytest
+
+from doublyexcited_amd.profsummary import class_table
 from doublyexcited_amd.traffic import analyse
 
 HDR = "Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value\n"
@@ -53,3 +56,47 @@ def test_ratios_from_calibrated_counters(tmp_path):
     assert abs(ratios["gram"] - (1e9 + 1e6) / 0.9e9) < 1e-9
     assert abs(ratios["coldots"] - 1.0) < 1e-9
     assert {row[0]: row[1] for row in table} == {"combine": 2, "gram": 1, "coldots": 2}
+
+
+NS = "void dex::(anonymous namespace)::"
+MUL = "void at::native::vectorized_elementwise_kernel<4, at::native::AUnaryFunctor<c10::complex<double> > >(int)"
+
+
+def _passes(tmp_path, kernels, totals):
+    """Counter passes of one dispatch per (kernel, GB read, GB written)."""
+    gib_kib = (1 << 30) / 1024.0
+    rows = [(i + 2, NS + k + "(int)", r, w) for i, (k, r, w) in enumerate(kernels)]
+    _write(tmp_path / "f", "FETCH_SIZE", [(1, MUL, gib_kib / 2)] + [(i, k, r * 1e9 / 2048) for i, k, r, _ in rows])
+    _write(tmp_path / "w", "WRITE_SIZE", [(1, MUL, gib_kib)] + [(i, k, w * 1e9 / 1024) for i, k, _, w in rows])
+    stats = tmp_path / "stats.json"
+    stats.write_text(json.dumps({"totals": totals}))
+    return analyse(tmp_path / "f", tmp_path / "w", stats)
+
+
+def test_matvec_passes_fall_into_their_classes(tmp_path):
+    """The transpose-add, the planes (two dispatches of the remaining passes a launch, with a
+    reduction for norms) and a cross-check context's seven launches."""
+    kernels = [("k_pass1<21, double, HIP_vector_type<double, 2u>, false>", 1.0, 1.0),
+               ("k_symfold<HIP_vector_type<double, 2u> >", 1.0, 1.0),
+               ("k_plane1<25, double>", 1.0, 1.0), ("k_plane2<25, double, false>", 2.0, 1.0),
+               ("k_plane2<25, double, true>", 2.0, 0.0), ("k_reduce_wide", 0.5, 0.0)]
+    kernels += [("k_axis<5>", 1.0, 1.0)] * 6 + [("k_potential", 2.0, 1.0)]
+    *_, table, ratios = _passes(tmp_path, kernels, {
+        "pass1": [2, 4e9, 0], "symadd": [1, 2e9, 0], "pass2": [1, 5.5e9, 0], "generic": [1, 15e9, 0],
+        "combine": [0, 0.0, 0]})
+    assert {row[0]: row[1] for row in table} == {"pass1": 2, "symadd": 1, "pass2": 1, "generic": 1}
+    assert all(abs(r - 1.0) < 1e-9 for r in ratios.values()) and len(ratios) == 4
+
+
+def test_a_class_without_its_kernels_is_an_error(tmp_path):
+    with pytest.raises(SystemExit, match="symadd.*k_renamed"):
+        _passes(tmp_path, [("k_renamed", 1.0, 1.0)], {"symadd": [3, 6e9, 0]})
+
+
+def test_class_table_counts_launches_and_names_what_has_no_class():
+    rows = [{"Name": NS + k + "(int)", "Calls": str(n), "TotalDurationNs": str(t)} for k, n, t in (
+        ("k_symfold<float>", 4, 4e6), ("k_plane1<13, double>", 3, 3e6), ("k_plane2<13, double, false>", 6, 12e6),
+        ("k_singlet", 2, 1e6))]
+    rows.append({"Name": MUL, "Calls": "9", "TotalDurationNs": "9e6"})
+    assert class_table(rows)[2:] == ["| pass2 | 3 | 12.0 | 4000.0 |", "| symadd | 4 | 4.0 | 1000.0 |",
+                                     "| pass1 | 3 | 3.0 | 1000.0 |", "| (no class) | 2 | 1.0 | 500.0 |"]
