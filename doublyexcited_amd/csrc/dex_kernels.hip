@@ -137,7 +137,12 @@ __device__ __forceinline__ void plane_axes(const R (&x)[NN], R *__restrict__ a, 
   __syncthreads();
 }
 
-// a b, not fused into the addition that follows.
+// a b, rounded by itself: of the two products of a potential term the compiler would fuse
+// one into the addition, which one depending on the code around it.  Neither form is the
+// more accurate.  Rounded, so that results do not move with that choice: their last bits
+// decide where a solve ends whose last pair has a rival at nearly the same distance from
+// sigma (NN = 11, theta 0.31: levels at 0.806 and 0.823; of four starts, two end warm and
+// cold solves apart).
 template <typename R>
 __device__ __forceinline__ R rounded_product(R a, R b) {
 #pragma clang fp contract(off)
@@ -157,10 +162,9 @@ __device__ __forceinline__ R rounded_product(R a, R b) {
 // keep vn in registers, which cost the second workgroup: FP32 at NN = 19 ran 277 us
 // a column looped and 175 us not, at NN = 21 487 and 354.
 //
-// SHIFT: H - shift, each product of the potential term less that of the shift.  A
-// variant of its own: with a zero shift the plain matvec took 1-2% more (4 columns at
-// NN = 19 in complex64 1366 for 1346 us, one at NN = 25 6.96 for 6.85 ms).  Without SHIFT
-// the same products are rounded, so that a zero shift and none give the same bits.
+// SHIFT: H - shift (FP64 forms), each product of the potential term less that of the
+// shift.  A variant of its own: with a zero shift the plain matvec took 1-2% more (one
+// column at NN = 25 6.96 for 6.85 ms).
 template <int NN, typename R, typename XT, typename ZT, bool SHIFT>
 __global__ __launch_bounds__(cube_threads<NN>()) void k_pass1(ColPtrs xs, ColPtrsW zs, const double *__restrict__ vn,
                                                               const double *__restrict__ tinv, MatvecCoef cf,

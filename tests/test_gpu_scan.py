@@ -73,3 +73,25 @@ def test_scan_at_the_scan_configuration_grids(dex):
     for w, c in ((warm[1], cold[0]), (warm[2], cold[1])):
         assert match(w.e, c.e) < 1e-8 and match(c.e, w.e) < 1e-8
     assert warm[1].iterations < cold[0].iterations
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 3])
+def test_scan_levels_do_not_depend_on_the_start(dex, seed):
+    """At NN=11, theta 0.31, levels lie at |E - sigma| of 0.806 and 0.823: which of them ends a
+    solve's 8 pairs is up to the last bits of its start and its arithmetic.  Warm and cold
+    points from any start converge 8 pairs, each within 1e-8 au of a level of a wider solve,
+    and hold every level clear of that near tie."""
+    from doublyexcited_amd.scan import theta_scan
+
+    kw = dict(sigma=-0.78 - 0.002j, tol=1e-8, ns=3, inner_iter=8, guard=2, maxit=400)
+    print(f"case: scan levels, start {seed}", flush=True)
+    levels = theta_scan([(5, 0.5, 0.31)], nev=12, warm=False, seed=17, **kw)[0]
+    assert levels.converged_pairs == 12
+    near = levels.e[np.abs(levels.e - kw["sigma"]) < 0.80]
+    assert len(near) >= 6
+    warm = theta_scan([(5, 0.5, 0.30), (5, 0.5, 0.31)], nev=8, warm=True, seed=seed, **kw)[1]
+    cold = theta_scan([(5, 0.5, 0.31)], nev=8, warm=False, seed=50 + seed, **kw)[0]
+    for p in (warm, cold):
+        print(f"  warm {p.warm}: {np.sort(np.abs(p.e - kw['sigma']))}", flush=True)
+        assert p.converged_pairs == 8
+        assert match(p.e, levels.e) < 1e-8 and match(near, p.e) < 1e-8
