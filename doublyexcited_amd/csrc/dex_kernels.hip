@@ -588,25 +588,30 @@ __global__ __launch_bounds__(direct_threads<NN>()) void k_direct(ColPtrs xs, Col
   __shared__ R tau[2 * NN - 1];
   if (threadIdx.x < 2 * NN - 1) tau[threadIdx.x] = R(tau_rt(int(threadIdx.x) - (NN - 1)));
   __syncthreads();
-  R kr = R(0), ki = R(0);
+  // each line's sum by itself, then the lines pairwise: fewer roundings on the way than in
+  // one running sum
+  R kr[3], ki[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    R sr = R(0), si = R(0);
+    R pr = R(0), pim = R(0), qr = R(0), qim = R(0);
 #pragma unroll
     for (int l = 0; l < NN; ++l) {
       const XT u = x[p + stride[a] * (l - pi[a]) + N3 * q], v = x[p + N3 * (q + stride[a] * (l - qi[a]))];
       const R tp = tau[l - pi[a] + NN - 1], tq = tau[l - qi[a] + NN - 1];
-      sr += tp * R(u.x) + tq * R(v.x);
-      si += tp * R(u.y) + tq * R(v.y);
+      pr += tp * R(u.x);
+      pim += tp * R(u.y);
+      qr += tq * R(v.x);
+      qim += tq * R(v.y);
     }
-    kr += sr;
-    ki += si;
+    kr[a] = pr + qr;
+    ki[a] = pim + qim;
   }
+  const R sr = (kr[0] + kr[1]) + kr[2], si = (ki[0] + ki[1]) + ki[2];
   const R s2r = R(cf.s2_re), s2i = R(cf.s2_im);
   const R vcr = R(cf.c1_re) * vr - R(cf.sh_re), vci = R(cf.c1_im) * vr - R(cf.sh_im);
   XT o;
-  o.x = s2r * kr - s2i * ki + vcr * R(own.x) - vci * R(own.y);
-  o.y = s2r * ki + s2i * kr + vcr * R(own.y) + vci * R(own.x);
+  o.x = s2r * sr - s2i * si + vcr * R(own.x) - vci * R(own.y);
+  o.y = s2r * si + s2i * sr + vcr * R(own.y) + vci * R(own.x);
   if (e1 < N3) static_cast<XT *>(ys.p[blockIdx.y])[p + N3 * q] = o;
 }
 
