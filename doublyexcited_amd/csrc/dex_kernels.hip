@@ -681,10 +681,11 @@ __global__ __launch_bounds__(1024) void k_reduce_wide(const double *__restrict__
   for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    s = 0.0;
-    for (int w = 0; w < 16; ++w) s += red[w];
-    out[blockIdx.x] = s;
+  // pairwise to the end: the last additions carry most of the rounding error
+  if (threadIdx.x < 64) {
+    s = threadIdx.x < 16 ? red[threadIdx.x] : 0.0;
+    for (int off = 8; off > 0; off >>= 1) s += __shfl_down(s, off);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
   }
 }
 
