@@ -362,19 +362,16 @@ template <typename XT>
 constexpr int plane_run() {
   return int(128 / sizeof(XT));  // entries of a 128-byte run
 }
-template <int NN>
-constexpr int plane1_planes() {
-  return NN >= 9 ? 8 : 16;  // i1 x j1 planes of a workgroup
-}
+constexpr int kPlane1Planes = 8;  // i1 x j1 planes of a workgroup
 
 // Axes i1 and j1 and the potential: Z = s2 (tau x 1 + 1 x tau) X + (c1 Vr - shift) o X.
-// blockIdx: electron-2 index q, group of kp = plane1_planes() planes k1.  Thread (i, g) keeps the
+// blockIdx: electron-2 index q, group of kPlane1Planes planes k1.  Thread (i, g) keeps the
 // j line of plane g.
 template <int NN, typename R, typename XT, typename ZT, bool SHIFT>
-__global__ __launch_bounds__(round_up(NN *plane1_planes<NN>(), 64)) void k_plane1(
+__global__ __launch_bounds__(round_up(NN *kPlane1Planes, 64)) void k_plane1(
     const XT *__restrict__ x, ZT *__restrict__ z, const double *__restrict__ vn, const double *__restrict__ tinv,
     MatvecCoef cf) {
-  constexpr int N2 = NN * NN, N3 = NN * N2, L = 2 * NN + 1, G = plane1_planes<NN>();
+  constexpr int N2 = NN * NN, N3 = NN * N2, L = 2 * NN + 1, G = kPlane1Planes;
   extern __shared__ __align__(16) unsigned char smem[];
   const int i = threadIdx.x % NN, g = threadIdx.x / NN, k = int(blockIdx.y) * G + g;
   const bool on = g < G && k < NN;
@@ -760,7 +757,7 @@ hipError_t pass2_nn(const void *x, const void *z, void *y, int ncols, const Matv
 
 template <int NN, typename R>
 constexpr size_t plane1_lds() {
-  return size_t(2) * plane1_planes<NN>() * NN * NN * sizeof(R);
+  return size_t(2) * kPlane1Planes * NN * NN * sizeof(R);
 }
 template <int NN, typename R, typename XT>
 constexpr size_t plane2_lds() {
@@ -790,7 +787,7 @@ bool plane2_setup() {
 template <int NN, typename R, typename XT, typename ZT>
 hipError_t plane1_nn(const void *x, void *z, const PotArgs &pot, hipStream_t s) {
   if (!plane1_setup<NN, R, XT, ZT>()) return hipErrorInvalidDeviceFunction;
-  constexpr int G = plane1_planes<NN>();
+  constexpr int G = kPlane1Planes;
   const dim3 g(NN * NN * NN, (NN + G - 1) / G), b(round_up(NN * G, 64));
   const XT *xx = static_cast<const XT *>(x);
   ZT *zz = static_cast<ZT *>(z);
