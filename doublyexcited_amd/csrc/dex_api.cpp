@@ -89,11 +89,11 @@ hipError_t scratch_address(int device, void **ptr) {
 // A solve, an inner solve or a residual check takes its work vectors (one
 // allocation a vector: 54 for an order-8 inner solve of 6 columns) from this
 // per-device list and returns them to it with its stream idle.  Allocating and
-// freeing them on each call cost far more than the work, since the driver clears
-// what it hands out: with the list an order-8 inner solve of 6 columns at NN = 13
-// (4 GB of vectors) takes 20.7 ms instead of 120, one of order 4 on 4 columns at
-// NN = 21 (27 GB) 108 ms instead of 316 to 1350, two eigensolver iterations of
-// 10 columns at NN = 11 149 ms instead of 206.
+// freeing them on each call costs up to far more than the work, since the driver
+// clears what it hands out and how long that takes scatters: with the list an order-8
+// inner solve of 6 columns at NN = 13 (4 GB of vectors) takes 9.4 ms, 22 to 24 with
+// the list freed after each call; one of order 4 on 4 columns at NN = 21 (27 GB) 50
+// for 53 to 3400, two eigensolver iterations of 10 columns at NN = 11 88 for 143 to 840.
 // Any thread and context may take a listed block: nothing is queued on it.  At
 // most an eighth of the device's memory stays listed (the blocks idle longest go
 // first), all of it is freed when the last context on the device is destroyed,

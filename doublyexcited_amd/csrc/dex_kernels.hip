@@ -283,8 +283,8 @@ __global__ __launch_bounds__(cube_threads<NN>()) void k_pass2(const XT *x, const
 // M is odd, so a tile's 512-byte runs start at any multiple of 16 bytes and share
 // their first and last 128-byte lines with the next tiles along p.  Tiles go to
 // the XCDs (consecutive workgroups: round robin) in blocks of 4 x 4, so that most
-// shared lines meet in one L2.  Bound by HBM (32 bytes an entry): 4.7 TB/s at NN = 21
-// in FP64, 5.4 TB/s on complex64.  The form before, which read X and U = tau3D X
+// shared lines meet in one L2.  Bound by HBM (32 bytes an entry, 16 in complex64): 4.8
+// TB/s at NN = 21 in FP64, 4.65 on complex64.  The form before, which read X and U = tau3D X
 // and rebuilt the potential here, moved 48 bytes an entry (1.0 ms a vector at
 // NN = 21 where this takes 0.58).
 constexpr int kSymT = 32;
@@ -355,8 +355,9 @@ __global__ __launch_bounds__(256) void k_symfold(ColPtrsW ys, int m, int nblk, i
 // A workgroup holds NN x NN lines of kPlaneRun entries: each thread keeps one line
 // of the first axis in registers (contracted there), the second axis goes through
 // the LDS buffers a (entries) and b (its sums), one real component at a time.
-// 32 + 48 + 48 bytes an entry over the three passes, 4.6 TB/s of them at NN = 25 in
-// FP64 (6.9 ms a vector; six passes of one axis and the potential's took 16.8), with
+// 32 + 48 + 48 bytes an entry over the three passes, 4.5 TB/s of them at NN = 25 in
+// FP64 (k_plane1 4.0, k_plane2 4.7; 6.9 ms a vector where six passes of one axis and the
+// potential's take 16.8), with
 // 8 waves a CU in flight (two workgroups: 80 KB of LDS, 205-240 registers).
 template <typename XT>
 constexpr int plane_run() {
